@@ -89,6 +89,48 @@ __global__ __launch_bounds__(256) void k_logsum(int64_t n, const double* __restr
     }
 }
 
+// ---------------------------------------------------------------- rows
+// Eight consecutive features of a node's row as FP32: one 16-byte load (BF16)
+// or two (FP32), so a row is 8 lanes wide and a wave moves eight rows at once.
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+
+__device__ inline void load8(const Bf16* __restrict__ p, float (&v)[8]) {
+    const u32x4_t u = *reinterpret_cast<const u32x4_t*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[2 * e] = __uint_as_float(u[e] << 16);
+        v[2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+    }
+}
+__device__ inline void load8(const float* __restrict__ p, float (&v)[8]) {
+    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(p), b = *reinterpret_cast<const f32x4_t*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+}
+__device__ inline void store8(Bf16* __restrict__ p, const float (&v)[8]) {
+    u32x4_t u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        Bf16 lo, hi;
+        stv(lo, v[2 * e]);
+        stv(hi, v[2 * e + 1]);
+        u[e] = (uint32_t)lo.v | ((uint32_t)hi.v << 16);
+    }
+    *reinterpret_cast<u32x4_t*>(p) = u;
+}
+__device__ inline void store8(float* __restrict__ p, const float (&v)[8]) {
+    *reinterpret_cast<f32x4_t*>(p) = f32x4_t{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f32x4_t*>(p + 4) = f32x4_t{v[4], v[5], v[6], v[7]};
+}
+// four consecutive features
+__device__ inline f32x4_t load4(const Bf16* __restrict__ p) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    return f32x4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                   __uint_as_float(u.y & 0xffff0000u)};
+}
+__device__ inline f32x4_t load4(const float* __restrict__ p) { return *reinterpret_cast<const f32x4_t*>(p); }
+
 // ------------------------------------------------------------ dense layers
 template <typename AT, typename IT>
 __global__ __launch_bounds__(256) void k_dense(int64_t N, const IT* __restrict__ in1, int k1,
@@ -120,6 +162,31 @@ __global__ __launch_bounds__(256) void k_dense(int64_t N, const IT* __restrict__
     }
 }
 
+// The input layers (K = 4 row or 2 column features): a thread per 8 outputs of
+// a node, the terms in the order of k_dense.  Bound by the write of the N x 64
+// activations; k_dense, which stages four nodes at a time behind two barriers,
+// took 89 us where this takes 23 us (mean of the two layers, m + n =
+// 1.07 million nodes, BF16).
+template <typename AT, int K>
+__global__ __launch_bounds__(256) void k_dense_in(int64_t N, const float* __restrict__ in, const float* __restrict__ W,
+                                                  const float* __restrict__ b, AT* __restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
+    const int64_t node = t >> 3;
+    const int o = 8 * (int)(t & 7);
+    if (node >= N) return;
+    float x[K], v[8];
+#pragma unroll
+    for (int k = 0; k < K; ++k) x[k] = in[node * K + k];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float acc = b[o + e];
+#pragma unroll
+        for (int k = 0; k < K; ++k) acc = __builtin_fmaf(x[k], W[k * kNnH + o + e], acc);
+        v[e] = fmaxf(acc, 0.0f);
+    }
+    store8(out + node * kNnH + o, v);
+}
+
 // The BF16 layers with K = k1 + k2 a multiple of 32 (the message layers and
 // the head) run on V_MFMA_F32_16X16X32_BF16 with FP32 accumulation: a
 // workgroup takes 64 nodes, each wave 16 of them across the 64 outputs (four
@@ -131,8 +198,6 @@ __global__ __launch_bounds__(256) void k_dense(int64_t N, const IT* __restrict__
 // elements against bank conflicts) as BF16, which is exact: the BF16 mode's
 // weights are BF16-rounded.
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
 __device__ inline uint16_t bf16_bits(float x) {
     Bf16 h;
@@ -196,19 +261,39 @@ __global__ void k_mfma_bf16_probe(const float* __restrict__ a, const float* __re
     for (int r = 0; r < 4; ++r) out[4 * l + r] = d[r];
 }
 
-// out[node] = sum_{p in adj(node)} val[p] src[idx[p]] / max(deg, 1)
+// out[node] = sum_{p in adj(node)} val[p] src[idx[p]] / max(deg, 1), p ascending.
+// Bound by the gathered rows (128 or 256 bytes each).  Eight lanes per node,
+// eight features each, so a wave gathers eight rows per load and four of a
+// node's rows are in flight (indices past the end repeat the last one; their
+// terms are dropped): 54 us per layer where a wave per node with one row in
+// flight took 251 us (mean of four, 2.23 million nonzeros, 1.07 million nodes, BF16).
 template <typename AT>
 __global__ __launch_bounds__(256) void k_mean(int32_t N, const int64_t* __restrict__ ptr,
                                               const int32_t* __restrict__ idx, const double* __restrict__ val,
                                               const AT* __restrict__ src, AT* __restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    const int32_t node = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
+    const int64_t node = t >> 3;
+    const int f = 8 * (int)(t & 7);
     if (node >= N) return;
     const int64_t b = ptr[node], e = ptr[node + 1];
-    float acc = 0.0f;
-    for (int64_t p = b; p < e; ++p) acc += (float)val[p] * ldv(src[(int64_t)idx[p] * kNnH + lane]);
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t p = b; p < e; p += 4) {
+        float w[4], x[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = p + u < e ? p + u : e - 1;
+            w[u] = (float)val[q];
+            load8(src + (int64_t)idx[q] * kNnH + f, x[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[k] = p + u < e ? __builtin_fmaf(w[u], x[u][k], acc[k]) : acc[k];
+    }
     const float deg = (float)(e - b > 1 ? e - b : 1);
-    stv(out[(int64_t)node * kNnH + lane], acc / deg);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k] = acc[k] / deg;
+    store8(out + node * kNnH + f, acc);
 }
 
 template <typename AT>
@@ -267,125 +352,291 @@ __global__ void k_out_bwd(int32_t m, const AT* __restrict__ z, const float* __re
     dpre[t] = ldv(z[t]) > 0.0f ? dyv[i] * wo[o] : 0.0f;
 }
 
-// partial[blk][o] = sum_i dyv_i z[i][o] (o < 64), partial[blk][64] = sum_i dyv_i
+// Weight gradients.  Every block leaves one partial of the whole gradient of
+// its layer, nn_wgrad_blocks(N) of them, and k_reduce_blocks adds them up in
+// block order; the waves of a block add into LDS one after the other.
+
+// the 4 (wave) x 4 (lane group) partial sums of four consecutive outputs per
+// lane, added over the lane groups by a fixed butterfly
+__device__ inline f32x4_t sum_groups(f32x4_t v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] += __shfl_xor(v[e], 16);
+        v[e] += __shfl_xor(v[e], 32);
+    }
+    return v;
+}
+
+// partial[blk][o] = sum_i dyv_i z[i][o] (o < 64), partial[blk][64] = sum_i dyv_i:
+// 16 lanes per node, four outputs each; bound by reading z
 template <typename AT>
 __global__ __launch_bounds__(256) void k_out_w(int32_t m, const AT* __restrict__ z, const float* __restrict__ dyv,
                                                float* __restrict__ partial) {
-    const int t = threadIdx.x;
-    const int64_t b0 = (int64_t)blockIdx.x * kNnChunk, b1 = std::min<int64_t>(b0 + kNnChunk, m);
-    float acc = 0.0f;
-    if (t < kNnH) {
-        for (int64_t i = b0; i < b1; ++i) acc += dyv[i] * ldv(z[i * kNnH + t]);
-    } else if (t == kNnH) {
-        for (int64_t i = b0; i < b1; ++i) acc += dyv[i];
+    __shared__ float red[4][kNnH + 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane & 15, lk = lane >> 4;
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f}, bs = acc;
+    for (int64_t i0 = ((int64_t)blockIdx.x * 4 + wave) * 4; i0 < m; i0 += (int64_t)gridDim.x * 16) {
+        const int64_t i = i0 + lk < m ? i0 + lk : m - 1;
+        const float d = i0 + lk < m ? dyv[i] : 0.0f;
+        const f32x4_t v = load4(z + i * kNnH + 4 * lc);
+        acc += d * v;
+        bs[0] += d;
     }
-    if (t <= kNnH) partial[(int64_t)blockIdx.x * (kNnH + 1) + t] = acc;
-}
-
-template <typename AT>
-__global__ void k_relu_bwd(int64_t N, const AT* __restrict__ h, const float* __restrict__ dh, float* __restrict__ dpre) {
-    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
-    if (t >= N * kNnH) return;
-    dpre[t] = ldv(h[t]) > 0.0f ? dh[t] : 0.0f;
-}
-
-// din[node][k] = sum_o dpre[node][o] W[k][o], k < k1 -> din1 (+= if acc1), else din2
-__global__ __launch_bounds__(256) void k_dense_bwd_in(int64_t N, const float* __restrict__ dpre,
-                                                      const float* __restrict__ W, int k1, int k2,
-                                                      float* __restrict__ din1, float* __restrict__ din2, int acc1) {
-    __shared__ float Ws[2 * kNnH * kNnH];
-    const int K = k1 + k2;
-    for (int t = threadIdx.x; t < K * kNnH; t += kB) Ws[t] = W[t];
+    acc = sum_groups(acc);
+    bs = sum_groups(bs);
+    if (lk == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave][4 * lc + e] = acc[e];
+        if (lc == 0) red[wave][kNnH] = bs[0];
+    }
     __syncthreads();
-    const int64_t total = N * K;
-    for (int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x; t < total; t += (int64_t)gridDim.x * kB) {
-        const int64_t node = t / K;
-        const int k = (int)(t - node * K);
-        const float* dp = dpre + node * kNnH;
-        float acc = 0.0f;
-        for (int o = 0; o < kNnH; ++o) acc += dp[o] * Ws[k * kNnH + o];
-        if (k < k1) {
-            float* d = din1 + node * k1 + k;
-            *d = acc1 ? *d + acc : acc;
-        } else {
-            din2[node * k2 + (k - k1)] = acc;
+    const int t = threadIdx.x;
+    if (t <= kNnH) partial[(int64_t)blockIdx.x * (kNnH + 1) + t] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+}
+
+// The gradient entering a layer's products: dh masked by the layer's ReLU
+// output h (h null: dh as it is).  Masking here saves a pass that would read
+// dh and h and write the masked rows for two readers.
+template <typename AT>
+__device__ inline f32x4_t masked4(const float* __restrict__ dh, const AT* __restrict__ h, int64_t at) {
+    f32x4_t d = load4(dh + at);
+    if (h) {
+        const f32x4_t a = load4(h + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[e] = a[e] > 0.0f ? d[e] : 0.0f;
+    }
+    return d;
+}
+
+// din[node][k] = sum_o dpre[node][o] W[k][o]; k < 64 -> din1 (+= if acc1), the
+// others -> din2.  V_MFMA_F32_16X16X4_F32 with FP32 accumulation: a wave takes
+// 16 nodes; A holds 16 rows of W (features), B the nodes, and inner slot 4 s + g
+// (step s, lane group g) stands for o = 16 g + s, so a lane's 16 values of a
+// node are 64 contiguous bytes and its 16 x kTiles weights stay in registers.
+// D[feature][node] leaves four consecutive features of a node in a lane.
+// Bound by reading dpre and writing din; a thread per output with the weights
+// in LDS took 543 us where this takes 49 us (mean of five layers,
+// m = 98,799, n = 262,080).
+template <typename AT, int kTiles>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_dense_bwd_in(int64_t N, const float* __restrict__ dh, const AT* __restrict__ h, const float* __restrict__ W,
+                    float* __restrict__ din1, float* __restrict__ din2, int acc1) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane & 15, lk = lane >> 4;
+    float wv[kTiles][16];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4_t v = load4(W + (16 * t + lc) * kNnH + 16 * lk + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wv[t][4 * q + e] = v[e];
+        }
+    for (int64_t n0 = ((int64_t)blockIdx.x * 4 + wave) * 16; n0 < N; n0 += (int64_t)gridDim.x * 64) {
+        const int64_t node = n0 + lc;
+        const int64_t at = (node < N ? node : N - 1) * kNnH + 16 * lk;
+        f32x4_t d[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = masked4(dh, h, at + 4 * q);
+        f32x4_t acc[kTiles];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[t][s], d[s >> 2][s & 3], acc[t], 0, 0, 0);
+        if (node < N) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) {
+                float* p = (t < 4 ? din1 : din2) + node * kNnH + 16 * (t & 3) + 4 * lk;
+                f32x4_t v = acc[t];
+                if (t < 4 && acc1) v += *reinterpret_cast<const f32x4_t*>(p);
+                *reinterpret_cast<f32x4_t*>(p) = v;
+            }
         }
     }
 }
 
 // partial[blk][k][o] = sum over the block's nodes of x_k dpre_o, x = [in1 in2 1]
-template <typename AT, typename IT>
-__global__ __launch_bounds__(256) void k_dense_bwd_w(int64_t N, const IT* __restrict__ in1, int k1,
-                                                     const AT* __restrict__ in2, int k2,
-                                                     const float* __restrict__ dpre, float* __restrict__ partial) {
-    constexpr int kStage = 8;
-    constexpr int kMaxU = (2 * kNnH + 1) * kNnH / kB + 1;   // 33
-    __shared__ float xs[kStage][2 * kNnH + 1];
-    __shared__ float ds[kStage][kNnH];
-    const int K = k1 + k2, KP = K + 1;
-    const int npair = KP * kNnH;
-    const int t = threadIdx.x;
-    float acc[kMaxU];
+// with 64 features per input (kTiles = 4 or 8 tiles of 16).
+// V_MFMA_F32_16X16X4_F32 with the nodes as the inner dimension: lane group g
+// carries node 4 q + g of a wave's four, a lane four consecutive features of
+// each input and four consecutive outputs, so rows are read as whole lines
+// straight into operand registers (tile t's row i stands for feature 4 i + t,
+// its column j of output tile u for output 4 j + u).  kDeep groups of four
+// nodes are loaded ahead of the products.  Bound by the matrix cores in FP32;
+// the form it replaces (products on the vector units, operands from LDS one
+// element at a time) took 1,668 us where this takes 41 us (mean of five
+// layers, m = 98,799, n = 262,080).
+template <typename AT, int kTiles>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_dense_bwd_w(int64_t N, const AT* __restrict__ in1, const AT* __restrict__ in2, const float* __restrict__ dh,
+                   const AT* __restrict__ h, float* __restrict__ partial) {
+    constexpr int kDeep = 2, kIn = kTiles / 4;
+    constexpr int K = kTiles * 16;
+    __shared__ __attribute__((aligned(16))) float Wg[(K + 1) * kNnH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane & 15, lk = lane >> 4;
+    f32x4_t acc[kTiles][4], bs = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int u = 0; u < kMaxU; ++u) acc[u] = 0.0f;
-    const int64_t b0 = (int64_t)blockIdx.x * kNnChunk, b1 = std::min<int64_t>(b0 + kNnChunk, N);
-    for (int64_t base = b0; base < b1; base += kStage) {
-        for (int s = t; s < kStage * KP; s += kB) {
-            const int q = s / KP, k = s - q * KP;
-            const int64_t node = base + q;
-            float v = 0.0f;
-            if (node < b1) {
-                if (k < k1) v = ldv(in1[node * k1 + k]);
-                else if (k < K) v = ldv(in2[node * k2 + (k - k1)]);
-                else v = 1.0f;
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[t][u] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4_t x[kDeep][kIn], d[kDeep];
+    const int64_t step = (int64_t)gridDim.x * 4 * 4 * kDeep;
+    auto load = [&](int64_t base) {
+#pragma unroll
+        for (int q = 0; q < kDeep; ++q) {
+            const int64_t node = base + 4 * q + lk;
+            const int64_t at = (node < N ? node : N - 1) * kNnH + 4 * lc;
+            x[q][0] = load4(in1 + at);
+            if constexpr (kIn == 2) x[q][1] = load4(in2 + at);
+            d[q] = masked4(dh, h, at);
+            if (node >= N) {   // contributes zeros
+                d[q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < kIn; ++k) x[q][k] = d[q];
             }
-            xs[q][k] = v;
         }
-        for (int s = t; s < kStage * kNnH; s += kB) {
-            const int q = s / kNnH, o = s - q * kNnH;
-            const int64_t node = base + q;
-            ds[q][o] = node < b1 ? dpre[node * kNnH + o] : 0.0f;
-        }
-        __syncthreads();
-        for (int q = 0; q < kStage; ++q) {
+    };
+    int64_t base = ((int64_t)blockIdx.x * 4 + wave) * 4 * kDeep;
+    if (base < N) load(base);
+    for (; base < N; base += step) {
+        f32x4_t xc[kDeep][kIn], dc[kDeep];
 #pragma unroll
-            for (int u = 0; u < kMaxU; ++u) {
-                const int p = t + kB * u;
-                if (p < npair) acc[u] += xs[q][p >> 6] * ds[q][p & 63];
+        for (int q = 0; q < kDeep; ++q) {
+#pragma unroll
+            for (int k = 0; k < kIn; ++k) xc[q][k] = x[q][k];
+            dc[q] = d[q];
+        }
+        if (base + step < N) load(base + step);
+#pragma unroll
+        for (int q = 0; q < kDeep; ++q) {
+            bs += dc[q];
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xc[q][t >> 2][t & 3], dc[q][u], acc[t][u], 0, 0, 0);
+        }
+    }
+    bs = sum_groups(bs);
+    // D's row i = 4 lk + r of tile t is feature 4 i + t, its column lc of u is
+    // output 4 lc + u: four outputs of a feature are 16 bytes
+    for (int w = 0; w < 4; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    f32x4_t* p = reinterpret_cast<f32x4_t*>(
+                        &Wg[(64 * (t >> 2) + 16 * lk + 4 * r + (t & 3)) * kNnH + 4 * lc]);
+                    const f32x4_t v = {acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]};
+                    *p = w ? *p + v : v;
+                }
+            if (lk == 0) {
+                f32x4_t* p = reinterpret_cast<f32x4_t*>(&Wg[K * kNnH + 4 * lc]);
+                *p = w ? *p + bs : bs;
             }
         }
         __syncthreads();
     }
-#pragma unroll
-    for (int u = 0; u < kMaxU; ++u) {
-        const int p = t + kB * u;
-        if (p < npair) partial[(int64_t)blockIdx.x * npair + p] = acc[u];
-    }
+    float* out = partial + (int64_t)blockIdx.x * (K + 1) * kNnH;
+    for (int t = threadIdx.x; t < (K + 1) * kNnH; t += kB) out[t] = Wg[t];
 }
 
-__global__ void k_reduce_blocks(int npar, int nblk, const float* __restrict__ partial, float* __restrict__ out) {
-    const int p = blockIdx.x * kB + threadIdx.x;
-    if (p >= npar) return;
+// the same for the input layers (K = 4 row or 2 column features): 16 lanes per
+// node, four outputs each, on the vector units; bound by reading dh and h
+// (28 us per layer, 501 us before)
+template <typename AT, int K>
+__global__ __launch_bounds__(256) void k_dense_bwd_w_in(int64_t N, const float* __restrict__ in,
+                                                        const float* __restrict__ dh, const AT* __restrict__ h,
+                                                        float* __restrict__ partial) {
+    __shared__ float red[4][(K + 1) * kNnH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane & 15, lk = lane >> 4;
+    f32x4_t acc[K + 1];
+#pragma unroll
+    for (int k = 0; k <= K; ++k) acc[k] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+    for (int64_t n0 = ((int64_t)blockIdx.x * 4 + wave) * 4; n0 < N; n0 += (int64_t)gridDim.x * 16) {
+        const int64_t node = n0 + lk < N ? n0 + lk : N - 1;
+        f32x4_t d = masked4(dh, h, node * kNnH + 4 * lc);
+        float x[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) x[k] = in[node * K + k];
+        if (n0 + lk >= N) d = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < K; ++k) acc[k] += x[k] * d;
+        acc[K] += d;
+    }
+#pragma unroll
+    for (int k = 0; k <= K; ++k) {
+        acc[k] = sum_groups(acc[k]);
+        if (lk == 0)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[wave][k * kNnH + 4 * lc + e] = acc[k][e];
+    }
+    __syncthreads();
+    float* out = partial + (int64_t)blockIdx.x * (K + 1) * kNnH;
+    for (int t = threadIdx.x; t < (K + 1) * kNnH; t += kB) out[t] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+}
+
+// out[p] = sum over the blocks of partial[blk][p]: 64 parameters per
+// workgroup, 16 waves over the blocks (one chain per thread over all of them
+// took 39 us where this takes 5 us)
+__global__ __launch_bounds__(1024) void k_reduce_blocks(int npar, int nblk, const float* __restrict__ partial,
+                                                        float* __restrict__ out) {
+    __shared__ float red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    const int pc = p < npar ? p : npar - 1;
     float s = 0.0f;
-    for (int b = 0; b < nblk; ++b) s += partial[(int64_t)b * npar + p];
+#pragma unroll 4
+    for (int b = wave; b < nblk; b += 16) s += partial[(int64_t)b * npar + pc];
+    red[wave][lane] = s;
+    __syncthreads();
+    if (wave != 0 || p >= npar) return;
+    s = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) s += red[w][lane];
     out[p] = s;
 }
 
-// din[src][f] += sum_{p in adjT(src)} valT[p] dout[idxT[p]][f] / deg(idxT[p])
+// din[src][f] (+)= sum_{p in adjT(src)} valT[p] / deg(idxT[p]) dout[idxT[p]][f],
+// laid out as k_mean (38 us per layer, 106 us with a wave per node)
+template <bool kAdd>
 __global__ __launch_bounds__(256) void k_mean_bwd(int32_t Nsrc, const int64_t* __restrict__ ptrT,
                                                   const int32_t* __restrict__ idxT, const double* __restrict__ valT,
                                                   const int64_t* __restrict__ ptrF, const float* __restrict__ dout,
                                                   float* __restrict__ din) {
-    const int lane = threadIdx.x & 63;
-    const int32_t node = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
+    const int64_t node = t >> 3;
+    const int f = 8 * (int)(t & 7);
     if (node >= Nsrc) return;
-    float acc = 0.0f;
-    for (int64_t p = ptrT[node]; p < ptrT[node + 1]; ++p) {
-        const int32_t j = idxT[p];
-        const int64_t deg = ptrF[j + 1] - ptrF[j];
-        acc += (float)valT[p] * dout[(int64_t)j * kNnH + lane] / (float)(deg > 1 ? deg : 1);
+    const int64_t b = ptrT[node], e = ptrT[node + 1];
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t p = b; p < e; p += 4) {
+        float w[4], x[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = p + u < e ? p + u : e - 1;
+            const int32_t j = idxT[q];
+            const int64_t deg = ptrF[j + 1] - ptrF[j];
+            w[u] = (float)valT[q] / (float)(deg > 1 ? deg : 1);
+            load8(dout + (int64_t)j * kNnH + f, x[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[k] = p + u < e ? acc[k] + w[u] * x[u][k] : acc[k];
     }
-    din[(int64_t)node * kNnH + lane] += acc;
+    float* o = din + node * kNnH + f;
+    if (kAdd) {
+        float old[8];
+        load8(o, old);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] += old[k];
+    }
+    store8(o, acc);
 }
 
 __global__ void k_adam(int npar, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ mo,
@@ -430,7 +681,15 @@ void nn_dense(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const flo
             return;
         }
     }
-    help::launch_kernel(k_dense<AT, IT>, grid_cap((N + 3) / 4, 2048), kB, 0, st, N, in1, k1, in2, k2, W, b, out);
+    if constexpr (std::is_same<IT, float>::value) {
+        if (k2 == 0 && (k1 == kNnFR || k1 == kNnFC)) {   // the input layers
+            if (k1 == kNnFR) help::launch_kernel(k_dense_in<AT, kNnFR>, grid_for(8 * N), kB, 0, st, N, in1, W, b, out);
+            else help::launch_kernel(k_dense_in<AT, kNnFC>, grid_for(8 * N), kB, 0, st, N, in1, W, b, out);
+            return;
+        }
+    }
+    if constexpr (std::is_same<AT, IT>::value)
+        help::launch_kernel(k_dense<AT, IT>, grid_cap((N + 3) / 4, 2048), kB, 0, st, N, in1, k1, in2, k2, W, b, out);
 }
 
 void nn_mfma_bf16_probe(const float* a, const float* b, float* out, hipStream_t st) {
@@ -440,7 +699,7 @@ void nn_mfma_bf16_probe(const float* a, const float* b, float* out, hipStream_t 
 template <typename AT>
 void nn_mean(int32_t N, const int64_t* ptr, const int32_t* idx, const double* val, const AT* src, AT* out,
              hipStream_t st) {
-    if (N > 0) help::launch_kernel(k_mean<AT>, (N + 3) / 4, kB, 0, st, N, ptr, idx, val, src, out);
+    if (N > 0) help::launch_kernel(k_mean<AT>, grid_for(8 * (int64_t)N), kB, 0, st, N, ptr, idx, val, src, out);
 }
 
 template <typename AT>
@@ -464,38 +723,49 @@ void nn_out_bwd(int32_t m, const AT* z, const float* dyv, const float* wo, float
     if (m > 0) help::launch_kernel(k_out_bwd<AT>, grid_for((int64_t)m * kNnH), kB, 0, st, m, z, dyv, wo, dpre);
 }
 
+// one block per 64 nodes (each of its waves then has 16), at most two per CU
+int nn_wgrad_blocks(int64_t N) { return grid_cap((N + 63) / 64, kNnMaxBlocks); }
+
 template <typename AT>
 void nn_out_w(int32_t m, const AT* z, const float* dyv, float* partial, hipStream_t st) {
-    if (m > 0) help::launch_kernel(k_out_w<AT>, (m + kNnChunk - 1) / kNnChunk, kB, 0, st, m, z, dyv, partial);
+    if (m > 0) help::launch_kernel(k_out_w<AT>, nn_wgrad_blocks(m), kB, 0, st, m, z, dyv, partial);
 }
 
 template <typename AT>
-void nn_relu_bwd(int64_t N, const AT* h, const float* dh, float* dpre, hipStream_t st) {
-    if (N > 0) help::launch_kernel(k_relu_bwd<AT>, grid_for(N * kNnH), kB, 0, st, N, h, dh, dpre);
-}
-
-void nn_dense_bwd_in(int64_t N, const float* dpre, const float* W, int k1, int k2, float* din1, float* din2,
+void nn_dense_bwd_in(int64_t N, const float* dh, const AT* h, const float* W, float* din1, float* din2,
                      bool accumulate1, hipStream_t st) {
-    if (N > 0)
-        help::launch_kernel(k_dense_bwd_in, grid_cap((N * (k1 + k2) + kB - 1) / kB, 4096), kB, 0, st, N, dpre, W, k1, k2, din1, din2,
-                                                                                    accumulate1 ? 1 : 0);
+    if (N <= 0) return;
+    const int nb = grid_cap((N + 63) / 64, kNnMaxBlocks);
+    if (din2) help::launch_kernel(k_dense_bwd_in<AT, 8>, nb, kB, 0, st, N, dh, h, W, din1, din2, accumulate1 ? 1 : 0);
+    else help::launch_kernel(k_dense_bwd_in<AT, 4>, nb, kB, 0, st, N, dh, h, W, din1, din2, accumulate1 ? 1 : 0);
 }
 
-template <typename AT, typename IT>
-void nn_dense_bwd_w(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const float* dpre, float* partial,
+template <typename AT>
+void nn_dense_bwd_w(int64_t N, const AT* in1, const AT* in2, const float* dh, const AT* h, float* partial,
                     hipStream_t st) {
-    if (N > 0)
-        help::launch_kernel(k_dense_bwd_w<AT, IT>, (int)((N + kNnChunk - 1) / kNnChunk), kB, 0, st, N, in1, k1, in2, k2, dpre,
-                                                                                   partial);
+    if (N <= 0) return;
+    if (in2) help::launch_kernel(k_dense_bwd_w<AT, 8>, nn_wgrad_blocks(N), kB, 0, st, N, in1, in2, dh, h, partial);
+    else help::launch_kernel(k_dense_bwd_w<AT, 4>, nn_wgrad_blocks(N), kB, 0, st, N, in1, in2, dh, h, partial);
+}
+
+template <typename AT>
+void nn_dense_bwd_w_in(int64_t N, const float* in, int k, const float* dh, const AT* h, float* partial,
+                       hipStream_t st) {
+    if (N <= 0) return;
+    if (k == kNnFR) help::launch_kernel(k_dense_bwd_w_in<AT, kNnFR>, nn_wgrad_blocks(N), kB, 0, st, N, in, dh, h, partial);
+    else help::launch_kernel(k_dense_bwd_w_in<AT, kNnFC>, nn_wgrad_blocks(N), kB, 0, st, N, in, dh, h, partial);
 }
 
 void nn_reduce_blocks(int npar, int nblk, const float* partial, float* out, hipStream_t st) {
-    help::launch_kernel(k_reduce_blocks, grid_for(npar), kB, 0, st, npar, nblk, partial, out);
+    help::launch_kernel(k_reduce_blocks, (npar + 63) / 64, 1024, 0, st, npar, nblk, partial, out);
 }
 
 void nn_mean_bwd(int32_t Nsrc, const int64_t* ptrT, const int32_t* idxT, const double* valT, const int64_t* ptrF,
-                 const float* dout, float* din, hipStream_t st) {
-    if (Nsrc > 0) help::launch_kernel(k_mean_bwd, (Nsrc + 3) / 4, kB, 0, st, Nsrc, ptrT, idxT, valT, ptrF, dout, din);
+                 const float* dout, float* din, bool accumulate, hipStream_t st) {
+    if (Nsrc <= 0) return;
+    const int nb = grid_for(8 * (int64_t)Nsrc);
+    if (accumulate) help::launch_kernel(k_mean_bwd<true>, nb, kB, 0, st, Nsrc, ptrT, idxT, valT, ptrF, dout, din);
+    else help::launch_kernel(k_mean_bwd<false>, nb, kB, 0, st, Nsrc, ptrT, idxT, valT, ptrF, dout, din);
 }
 
 void nn_adam(int npar, float* p, const float* g, float* mo, float* ve, float lr, float b1, float b2, float eps,
@@ -516,14 +786,14 @@ void nn_check_finite(int32_t m, const double* x, int32_t* flag, hipStream_t st) 
                                 double*, hipStream_t);                                                           \
     template void nn_out_bwd<AT>(int32_t, const AT*, const float*, const float*, float*, hipStream_t);            \
     template void nn_out_w<AT>(int32_t, const AT*, const float*, float*, hipStream_t);                           \
-    template void nn_relu_bwd<AT>(int64_t, const AT*, const float*, float*, hipStream_t);                        \
-    template void nn_dense_bwd_w<AT, AT>(int64_t, const AT*, int, const AT*, int, const float*, float*, hipStream_t);
+    template void nn_dense_bwd_in<AT>(int64_t, const float*, const AT*, const float*, float*, float*, bool,       \
+                                      hipStream_t);                                                              \
+    template void nn_dense_bwd_w<AT>(int64_t, const AT*, const AT*, const float*, const AT*, float*, hipStream_t); \
+    template void nn_dense_bwd_w_in<AT>(int64_t, const float*, int, const float*, const AT*, float*, hipStream_t);
 NN_INST(float)
 NN_INST(Bf16)
 template void nn_dense<Bf16, float>(int64_t, const float*, int, const Bf16*, int, const float*, const float*, Bf16*,
                                     hipStream_t);
-template void nn_dense_bwd_w<Bf16, float>(int64_t, const float*, int, const Bf16*, int, const float*, float*,
-                                          hipStream_t);
 #undef NN_INST
 
 }  // namespace help

@@ -29,7 +29,7 @@ namespace help {
 constexpr int kNnH = 64;       // hidden width
 constexpr int kNnFR = 4;       // row input features
 constexpr int kNnFC = 2;       // column input features
-constexpr int kNnChunk = 1024; // nodes per block of the weight-gradient partials
+constexpr int kNnMaxBlocks = 512; // most partials of a layer's weight gradient: two workgroups per CU
 
 // offsets of the parameter blocks in the flat FP32 parameter vector
 struct NnLayout {
@@ -67,22 +67,28 @@ void nn_output_grad(int32_t m, const float* y, const double* dy, const double* g
                     float* dyv, hipStream_t st);
 template <typename AT>
 void nn_out_bwd(int32_t m, const AT* z, const float* dyv, const float* wo, float* dpre, hipStream_t st);
-// partial[blk][0..63] = sum dyv_i z_i, partial[blk][64] = sum dyv_i (blocks of kNnChunk rows)
+// blocks (and so partials) of the weight-gradient kernels below for N nodes
+int nn_wgrad_blocks(int64_t N);
+// partial[blk][0..63] = sum dyv_i z_i, partial[blk][64] = sum dyv_i
 template <typename AT>
 void nn_out_w(int32_t m, const AT* z, const float* dyv, float* partial, hipStream_t st);
+// dIn = dpre W^T with dpre = dh masked by the ReLU output h (h null: dh); 64
+// inputs into din1, 64 more into din2 unless it is null; accumulate adds into din1
 template <typename AT>
-void nn_relu_bwd(int64_t N, const AT* h, const float* dh, float* dpre, hipStream_t st);
-// dIn = dpre W^T (columns split into the two inputs); accumulate adds into dIn
-void nn_dense_bwd_in(int64_t N, const float* dpre, const float* W, int k1, int k2, float* din1, float* din2,
+void nn_dense_bwd_in(int64_t N, const float* dh, const AT* h, const float* W, float* din1, float* din2,
                      bool accumulate1, hipStream_t st);
-// partial (per block of kNnChunk nodes) of [in1 in2 1]^T dpre, (k1+k2+1) x 64
-template <typename AT, typename IT>
-void nn_dense_bwd_w(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const float* dpre, float* partial,
+// partial of [in1 in2 1]^T dpre ((64 or 128) + 1 rows of 64), in2 may be null
+template <typename AT>
+void nn_dense_bwd_w(int64_t N, const AT* in1, const AT* in2, const float* dh, const AT* h, float* partial,
                     hipStream_t st);
+// the same for an input layer of k = kNnFR or kNnFC features
+template <typename AT>
+void nn_dense_bwd_w_in(int64_t N, const float* in, int k, const float* dh, const AT* h, float* partial,
+                       hipStream_t st);
 void nn_reduce_blocks(int npar, int nblk, const float* partial, float* out, hipStream_t st);
-// din[src] += sum over the transposed adjacency of val * dout[dst] / deg(dst)
+// din[src] (+)= sum over the transposed adjacency of val * dout[dst] / deg(dst)
 void nn_mean_bwd(int32_t Nsrc, const int64_t* ptrT, const int32_t* idxT, const double* valT,
-                 const int64_t* ptrF, const float* dout, float* din, hipStream_t st);
+                 const int64_t* ptrF, const float* dout, float* din, bool accumulate, hipStream_t st);
 void nn_adam(int npar, float* p, const float* g, float* mo, float* ve, float lr, float b1, float b2, float eps,
              int t, int bf16, float* pw, hipStream_t st);
 void nn_check_finite(int32_t m, const double* x, int32_t* flag, hipStream_t st);

@@ -62,8 +62,7 @@ void ensure_workspace(help_mpnn* net, int32_t m, int32_t n) {
     net->R1.alloc(M * kNnH); net->R2.alloc(M * kNnH);
     net->C1.alloc(N * kNnH); net->C2.alloc(N * kNnH);
     net->P.alloc(MN * kNnH); net->Q.alloc(MN * kNnH);
-    const int64_t nblk = (MN + help::kNnChunk - 1) / help::kNnChunk;
-    net->partial.alloc(nblk * (2 * kNnH + 1) * kNnH);
+    net->partial.alloc((size_t)help::kNnMaxBlocks * (2 * kNnH + 1) * kNnH);
     const size_t esz = net->bf16 ? sizeof(Bf16) : sizeof(float);
     net->act.alloc((size_t)kNnH * esz * (6 * M + 5 * N));
 }
@@ -132,13 +131,21 @@ void forward(help_mpnn* net, help_gpu* h, const double* d, const double* r, doub
     HIPCHK(hipGetLastError());
 }
 
-// weight gradient of one dense layer into grad[off .. off + (k1+k2+1)*64)
-template <typename AT, typename IT>
-void dense_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const IT* in1, int k1, const AT* in2, int k2,
-                 const float* dpre, int off) {
-    const int nblk = (int)((N + help::kNnChunk - 1) / help::kNnChunk);
-    help::nn_dense_bwd_w<AT, IT>(N, in1, k1, in2, k2, dpre, net->partial.p, st);
-    help::nn_reduce_blocks((k1 + k2 + 1) * kNnH, nblk, net->partial.p, net->grad.p + off, st);
+// weight gradient of one dense layer ([in1 in2 1]^T of the masked dh) into
+// grad[off .. off + (k+1)*64); in2 may be null
+template <typename AT>
+void dense_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const AT* in1, const AT* in2, const float* dh, const AT* h,
+                 int off) {
+    help::nn_dense_bwd_w<AT>(N, in1, in2, dh, h, net->partial.p, st);
+    help::nn_reduce_blocks(((in2 ? 2 : 1) * kNnH + 1) * kNnH, help::nn_wgrad_blocks(N), net->partial.p,
+                           net->grad.p + off, st);
+}
+// the same for an input layer of k features
+template <typename AT>
+void input_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const float* in, int k, const float* dh, const AT* h,
+                 int off) {
+    help::nn_dense_bwd_w_in<AT>(N, in, k, dh, h, net->partial.p, st);
+    help::nn_reduce_blocks((k + 1) * kNnH, help::nn_wgrad_blocks(N), net->partial.p, net->grad.p + off, st);
 }
 
 template <typename AT>
@@ -163,37 +170,30 @@ void backward(help_mpnn* net, help_gpu* h, const double* dy) {
     float *R1 = net->R1.p, *R2 = net->R2.p, *C1 = net->C1.p, *C2 = net->C2.p, *P = net->P.p, *Q = net->Q.p;
     // head
     help::nn_out_w<AT>(m, a.z, net->dyv.p, net->partial.p, st);
-    help::nn_reduce_blocks(kNnH + 1, (m + help::kNnChunk - 1) / help::kNnChunk, net->partial.p,
-                           net->grad.p + NnLayout::wo, st);
+    help::nn_reduce_blocks(kNnH + 1, help::nn_wgrad_blocks(m), net->partial.p, net->grad.p + NnLayout::wo, st);
     help::nn_out_bwd<AT>(m, a.z, net->dyv.p, W + NnLayout::wo, P, st);
-    dense_wgrad<AT, AT>(net, st, m, a.hr2, kNnH, (const AT*)nullptr, 0, P, NnLayout::Wh);
-    help::nn_dense_bwd_in(m, P, W + NnLayout::Wh, kNnH, 0, R1, nullptr, false, st);            // d hr2
+    const AT* none = nullptr;
+    dense_wgrad<AT>(net, st, m, a.hr2, none, P, none, NnLayout::Wh);
+    help::nn_dense_bwd_in<AT>(m, P, none, W + NnLayout::Wh, R1, nullptr, false, st);             // d hr2
     // L4: hr2 = relu([hr1 ar4] W4 + b4), ar4 = mean(hc2)
-    help::nn_relu_bwd<AT>(m, a.hr2, R1, P, st);
-    dense_wgrad<AT, AT>(net, st, m, a.hr1, kNnH, a.ar4, kNnH, P, NnLayout::W(4));
-    help::nn_dense_bwd_in(m, P, W + NnLayout::W(4), kNnH, kNnH, R2, Q, false, st);               // d hr1, d ar4
-    HIPCHK(hipMemsetAsync(C1, 0, sizeof(float) * (size_t)n * kNnH, st));
-    help::nn_mean_bwd(n, cp, ri, cv, rp, Q, C1, st);                                            // d hc2
+    dense_wgrad<AT>(net, st, m, a.hr1, a.ar4, R1, a.hr2, NnLayout::W(4));
+    help::nn_dense_bwd_in<AT>(m, R1, a.hr2, W + NnLayout::W(4), R2, Q, false, st);               // d hr1, d ar4
+    help::nn_mean_bwd(n, cp, ri, cv, rp, Q, C1, false, st);                                     // d hc2
     // L3: hc2 = relu([hc1 ac3] W3 + b3), ac3 = meanT(hr1)
-    help::nn_relu_bwd<AT>(n, a.hc2, C1, P, st);
-    dense_wgrad<AT, AT>(net, st, n, a.hc1, kNnH, a.ac3, kNnH, P, NnLayout::W(3));
-    help::nn_dense_bwd_in(n, P, W + NnLayout::W(3), kNnH, kNnH, C2, Q, false, st);               // d hc1, d ac3
-    help::nn_mean_bwd(m, rp, ci, rv, cp, Q, R2, st);                                            // d hr1 +=
+    dense_wgrad<AT>(net, st, n, a.hc1, a.ac3, C1, a.hc2, NnLayout::W(3));
+    help::nn_dense_bwd_in<AT>(n, C1, a.hc2, W + NnLayout::W(3), C2, Q, false, st);               // d hc1, d ac3
+    help::nn_mean_bwd(m, rp, ci, rv, cp, Q, R2, true, st);                                      // d hr1 +=
     // L2: hr1 = relu([hr0 ar2] W2 + b2), ar2 = mean(hc1)
-    help::nn_relu_bwd<AT>(m, a.hr1, R2, P, st);
-    dense_wgrad<AT, AT>(net, st, m, a.hr0, kNnH, a.ar2, kNnH, P, NnLayout::W(2));
-    help::nn_dense_bwd_in(m, P, W + NnLayout::W(2), kNnH, kNnH, R1, Q, false, st);               // d hr0, d ar2
-    help::nn_mean_bwd(n, cp, ri, cv, rp, Q, C2, st);                                            // d hc1 +=
+    dense_wgrad<AT>(net, st, m, a.hr0, a.ar2, R2, a.hr1, NnLayout::W(2));
+    help::nn_dense_bwd_in<AT>(m, R2, a.hr1, W + NnLayout::W(2), R1, Q, false, st);               // d hr0, d ar2
+    help::nn_mean_bwd(n, cp, ri, cv, rp, Q, C2, true, st);                                      // d hc1 +=
     // L1: hc1 = relu([hc0 ac1] W1 + b1), ac1 = meanT(hr0)
-    help::nn_relu_bwd<AT>(n, a.hc1, C2, P, st);
-    dense_wgrad<AT, AT>(net, st, n, a.hc0, kNnH, a.ac1, kNnH, P, NnLayout::W(1));
-    help::nn_dense_bwd_in(n, P, W + NnLayout::W(1), kNnH, kNnH, C1, Q, false, st);               // d hc0, d ac1
-    help::nn_mean_bwd(m, rp, ci, rv, cp, Q, R1, st);                                            // d hr0 +=
+    dense_wgrad<AT>(net, st, n, a.hc0, a.ac1, C2, a.hc1, NnLayout::W(1));
+    help::nn_dense_bwd_in<AT>(n, C2, a.hc1, W + NnLayout::W(1), C1, Q, false, st);               // d hc0, d ac1
+    help::nn_mean_bwd(m, rp, ci, rv, cp, Q, R1, true, st);                                      // d hr0 +=
     // input layers
-    help::nn_relu_bwd<AT>(m, a.hr0, R1, P, st);
-    dense_wgrad<AT, float>(net, st, m, net->xr.p, help::kNnFR, (const AT*)nullptr, 0, P, NnLayout::Wr0);
-    help::nn_relu_bwd<AT>(n, a.hc0, C1, P, st);
-    dense_wgrad<AT, float>(net, st, n, net->xc.p, help::kNnFC, (const AT*)nullptr, 0, P, NnLayout::Wc0);
+    input_wgrad<AT>(net, st, m, net->xr.p, help::kNnFR, R1, a.hr0, NnLayout::Wr0);
+    input_wgrad<AT>(net, st, n, net->xc.p, help::kNnFC, C1, a.hc0, NnLayout::Wc0);
     HIPCHK(hipGetLastError());
     net->have_grad = true;
 }

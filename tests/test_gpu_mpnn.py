@@ -67,6 +67,32 @@ def test_gradients_fp32_match_autograd():
     be.destruct()
 
 
+@pytest.mark.parametrize("name,maker", [
+    ("fewer nodes than a tile", lambda: instances.mcf(side=2, commodities=1, pairs=1, seed=51)),
+    ("ragged tiles", lambda: instances.mcf(side=9, commodities=5, pairs=3, seed=52)),
+    ("more columns than one pass of the blocks", lambda: instances.random_lp(40, 33000, 2, seed=53))])
+def test_gradients_fp32_node_counts(name, maker):
+    """The backward kernels take 16 nodes per wave, 64 per block and at most
+    512 blocks: node counts below a tile, with remainders, and beyond one pass
+    of the blocks, against the oracle within the bars of
+    test_gradients_fp32_match_autograd."""
+    import mpnn_oracle as MO
+    inst = maker()
+    rng = np.random.default_rng(6)
+    d = np.exp(rng.uniform(-2, 2, inst.n) * np.log(10.0))
+    r, dy = rng.standard_normal(inst.m), rng.standard_normal(inst.m) * 1e-2
+    be = graph_handle(inst)
+    net = Mpnn(bf16=False, seed=7)
+    loss, g = net.loss_grad(be, d, r, dy, want_grad=True)
+    lo, go, _ = MO.loss_and_grad(net.params(), inst.to_scipy(), d, r, dy)
+    rel_g = np.linalg.norm(g - go) / np.linalg.norm(go)
+    _flush(f"mpnn fp32, {name}: m={inst.m} n={inst.n} loss {loss:.8f} vs {lo:.8f}; grad rel err {rel_g:.2e}")
+    assert abs(loss - lo) <= 1e-5 * abs(lo)
+    assert rel_g <= 1e-4
+    net.close()
+    be.destruct()
+
+
 def test_gradients_bf16_close_to_autograd():
     import mpnn_oracle as MO
     inst, d, r, dy = _case(seed=1)
