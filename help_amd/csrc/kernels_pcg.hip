@@ -3,15 +3,15 @@
 // * Row-split CSR products: A has rows of wildly different lengths (Zipf row
 //   popularity gives rows with millions of nonzeros), so rows up to
 //   kLightRow nonzeros take a thread, rows up to kHeavyRow a wave, and
-//   longer rows are cut into chunks of kRowChunk, one workgroup each,
-//   combined in chunk order: deterministic.
+//   longer rows are cut into chunks, one wave each, combined in chunk order:
+//   deterministic.
 // * Greedy partial Cholesky (PCG.cpp:38-103): per pivot an argmax over the
 //   Schur diagonal, the pivot row of A scattered into an n-vector, one
 //   product with A for the pivot's column of ADA^T, and a left-looking
 //   column update against the previous columns (column-major m x K factor,
 //   so the thread-per-row update reads coalesced).
-// * Preconditioner apply (PCG.cpp:183-196) with the factor in FP32: two
-//   passes over the m x K factor (a product and a transposed product).
+// * Preconditioner apply (PCG.cpp:183-196) with the factor in FP32: the
+//   product and the transposed product in one pass over the m x K factor.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -100,20 +100,37 @@ __global__ __launch_bounds__(256) void k_csr_medium(int32_t nmed, const int32_t*
     if (lane == 0) y[i] = s;
 }
 
+// A wave per chunk of a heavy row, eight terms per lane in flight.  Bound by
+// the gathers of x: listed by column block and XCD (RowSplitDev) they hit L2.
+// 12.1 million nonzeros of 1,181 rows, x of 32 MB: 70 us; chunks of 4,096
+// in row order, a workgroup each with one term per lane in flight, took 150 us.
 template <bool SQ>
-__global__ __launch_bounds__(256) void k_csr_chunk(const RowChunk* __restrict__ chunks,
+__global__ __launch_bounds__(256) void k_csr_chunk(int32_t nchunk, const RowChunk* __restrict__ chunks,
                                                    const int32_t* __restrict__ colind,
                                                    const double* __restrict__ val,
                                                    const double* __restrict__ x, double* __restrict__ part) {
-    __shared__ double red[kB];
-    const RowChunk c = chunks[blockIdx.x];
-    double acc = 0.0;
-    for (int64_t p = c.b + threadIdx.x; p < c.e; p += kB) {
-        const double v = val[p];
-        acc += (SQ ? v * v : v) * x[colind[p]];
+    const int32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (i >= nchunk) return;
+    const RowChunk c = chunks[i];
+    if (c.e <= c.b) return;   // padding
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int64_t p0 = c.b + lane; p0 < c.e; p0 += 512) {
+        double v[8], g[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int64_t q = p0 + 64 * u < c.e ? p0 + 64 * u : c.e - 1;
+            v[u] = val[q];
+            g[u] = x[colind[q]];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const double t = (SQ ? v[u] * v[u] : v[u]) * g[u];
+            a[u & 3] = (p0 + 64 * u < c.e) ? a[u & 3] + t : a[u & 3];
+        }
     }
-    const double s = block_sum(acc, red);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    const double s = wave_sum((a[0] + a[1]) + (a[2] + a[3]));
+    if (lane == 0) part[c.slot] = s;
 }
 
 // a wave per heavy row: its chunk partials summed lane-strided, fixed tree
@@ -311,9 +328,9 @@ __global__ void k_vdiv(int64_t n, const double* __restrict__ a, const double* __
     if (i < n) out[i] = a[i] / b[i];
 }
 
-__global__ void k_to_f32(int64_t n, const double* __restrict__ x, float* __restrict__ y) {
-    const int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x;
-    if (i < n) y[i] = (float)x[i];
+__global__ void k_to_f32(int32_t m, const double* __restrict__ x, float* __restrict__ y, int64_t ld) {
+    const int32_t i = blockIdx.x * kB + threadIdx.x;
+    if (i < m) y[blockIdx.y * ld + i] = (float)x[(int64_t)blockIdx.y * m + i];
 }
 
 // ------------------------------------------------------ preconditioner apply
@@ -339,7 +356,7 @@ __global__ __launch_bounds__(256) void k_pca_y1(int32_t K, const int32_t* __rest
 // z_j = (r_j - sum_c L(j,c) y1_c) / S_j off the pivots, 0 on them; the
 // factor in FP32 (the default) or FP64, the sums in FP64
 template <typename T>
-__global__ __launch_bounds__(256) void k_pca_t2(int32_t m, int32_t K, const int32_t* __restrict__ pos,
+__global__ __launch_bounds__(256) void k_pca_t2(int32_t m, int64_t ld, int32_t K, const int32_t* __restrict__ pos,
                                                 const T* __restrict__ L32, const double* __restrict__ y1g,
                                                 const double* __restrict__ S, const double* __restrict__ r,
                                                 double* __restrict__ z) {
@@ -352,19 +369,19 @@ __global__ __launch_bounds__(256) void k_pca_t2(int32_t m, int32_t K, const int3
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
     int32_t c = 0;
     for (; c + 3 < K; c += 4) {
-        a0 += (double)L32[(int64_t)c * m + j] * y1[c];
-        a1 += (double)L32[(int64_t)(c + 1) * m + j] * y1[c + 1];
-        a2 += (double)L32[(int64_t)(c + 2) * m + j] * y1[c + 2];
-        a3 += (double)L32[(int64_t)(c + 3) * m + j] * y1[c + 3];
+        a0 += (double)L32[(int64_t)c * ld + j] * y1[c];
+        a1 += (double)L32[(int64_t)(c + 1) * ld + j] * y1[c + 1];
+        a2 += (double)L32[(int64_t)(c + 2) * ld + j] * y1[c + 2];
+        a3 += (double)L32[(int64_t)(c + 3) * ld + j] * y1[c + 3];
     }
-    for (; c < K; ++c) a0 += (double)L32[(int64_t)c * m + j] * y1[c];
+    for (; c < K; ++c) a0 += (double)L32[(int64_t)c * ld + j] * y1[c];
     z[j] = (r[j] - ((a0 + a1) + (a2 + a3))) / S[j];
 }
 
 // ltpart[c * nb + b] = sum over the kLtRows rows of block b of L(j,c) z_j
 // (z is 0 on the pivots); a wave per column, 32 rows per lane in flight
 template <typename T>
-__global__ __launch_bounds__(256) void k_pca_lt(int32_t m, int32_t K, const T* __restrict__ L32,
+__global__ __launch_bounds__(256) void k_pca_lt(int32_t m, int64_t ld, int32_t K, const T* __restrict__ L32,
                                                 const double* __restrict__ z, double* __restrict__ ltpart) {
     __shared__ double zs[kLtRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -373,7 +390,7 @@ __global__ __launch_bounds__(256) void k_pca_lt(int32_t m, int32_t K, const T* _
     __syncthreads();
     const int64_t last = (int64_t)m - 1;
     for (int c = wave; c < K; c += 4) {
-        const T* Lc = L32 + (int64_t)c * m;
+        const T* Lc = L32 + (int64_t)c * ld;
         double a[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int u = 0; u < kLtRows / 64; ++u) {
@@ -403,20 +420,111 @@ __global__ __launch_bounds__(256) void k_pca_w(int32_t K, int32_t nb, const int3
     if (lane == 0) w[c] = y1[c] / S[perm[c]] - s;
 }
 
-// z(pivot i) = sum_{c >= i} X[c][i] w_c   (L11^-T w): a thread per i, the
-// reads of a row c coalesced across the threads, 8 terms in flight
-__global__ void k_pca_final(int32_t K, const int32_t* __restrict__ perm, const double* __restrict__ X,
-                            const double* __restrict__ w, double* __restrict__ z) {
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i >= K) return;
-    double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    int32_t c = i;
-    for (; c + 7 < K; c += 8) {
+// z_j = (r_j - sum_c L(j,c) y1_c) / S_j off the pivots, 0 on them, and
+// ltpart[c * nb + blk] = sum over the block's rows of L(j,c) z_j, in one pass
+// over the factor: a tile of 32 rows lies in the registers of a workgroup
+// (lane: a row and one of a pair of columns, NC pairs per wave) between its two
+// uses, and the sums of the second one stay in registers until the block has
+// walked all its tiles.  The next tile's loads are issued as each column is
+// used up.  Bound by reading the factor once.  NC columns of T and NC FP64 sums
+// per lane: with T = float and NC = 32 two workgroups share a CU.
+// m = 10^6, K = 500, FP32: 384 us (5.2 TB/s), where k_pca_t2 and k_pca_lt
+// read the factor twice in 347 + 342 us.
+template <typename T, int NC>
+__global__ __launch_bounds__(512, sizeof(T) * NC <= 128 ? 4 : 2) void k_pca_fused(int32_t m, int64_t ld, int32_t K, const int32_t* __restrict__ pos,
+                                                   const T* __restrict__ L, const double* __restrict__ y1g,
+                                                   const double* __restrict__ S, const double* __restrict__ r,
+                                                   double* __restrict__ z, double* __restrict__ ltpart) {
+    __shared__ double y1[16 * NC];
+    __shared__ double red[2][16][32];
+    const int tid = threadIdx.x, rl = tid & 31, hf = (tid >> 5) & 1, cg = tid >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int t = tid; t < 16 * NC; t += 512) y1[t] = t < K ? y1g[t] : 0.0;
+    // wave w holds columns 2 NC w + 2 i + (lane half); column pairs past the
+    // factor (of an even number of columns, a zero one after an odd K) repeat
+    // the last one: their y1 is 0 and their sums are not stored
+    const int cw = 2 * NC * wave, last = (K - 1) & ~1;
+    const double* yc = y1 + cw + hf;
+    const uint32_t half = hf * (uint32_t)ld;
+    double acc[NC];
+    T v[NC];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] += X[(int64_t)(c + u) * K + i] * w[c + u];
+    for (int i = 0; i < NC; ++i) acc[i] = 0.0;
+    const uint32_t step = gridDim.x * 32, um = (uint32_t)m;
+    uint32_t r0 = blockIdx.x * 32;   // below m + step < 2^32
+    auto load = [&](int i, uint32_t at) {
+        const T* col = L + min(cw + 2 * i, last) * ld;   // uniform over the wave
+        return col[at];
+    };
+    {
+        const uint32_t at = half + min(r0 + rl, um - 1);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[i] = load(i, at);
     }
-    for (; c < K; ++c) a[0] += X[(int64_t)c * K + i] * w[c];
-    z[perm[i]] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+    __syncthreads();
+    for (int buf = 0; r0 < um; r0 += step, buf ^= 1) {
+        const uint32_t j = min(r0 + rl, um - 1);
+        const double rj = r[j], sj = S[j];
+        const int32_t pj = pos[j];
+        double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+        for (int i = 0; i < NC; i += 2) {
+            s0 += (double)v[i] * yc[2 * i];
+            s1 += (double)v[i + 1] * yc[2 * i + 2];
+        }
+        red[buf][cg][rl] = s0 + s1;
+        // the FP32 tile is converted again below: kept as FP64 from here it
+        // would take twice the registers
+#pragma unroll
+        for (int i = 0; i < NC; ++i) asm volatile("" : "+v"(v[i]));
+        __syncthreads();
+        double q[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            q[g] = (red[buf][g][rl] + red[buf][g + 4][rl]) + (red[buf][g + 8][rl] + red[buf][g + 12][rl]);
+        const double zj = (r0 + rl < um && pj >= K) ? (rj - ((q[0] + q[1]) + (q[2] + q[3]))) / sj : 0.0;
+        if (cg == 0 && r0 + rl < um) z[j] = zj;
+        const uint32_t at = half + min(r0 + step + rl, um - 1);
+        // four columns at a time, so that the loads take the registers they free
+#pragma unroll
+        for (int i0 = 0; i0 < NC; i0 += 4) {
+#pragma unroll
+            for (int i = i0; i < i0 + 4; ++i) acc[i] += (double)v[i] * zj;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = i0; i < i0 + 4; ++i) v[i] = load(i, at);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        double s = acc[i];
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) s += __shfl_xor(s, off);
+        const int c = cw + 2 * i + hf;
+        if (rl == 0 && c < K) ltpart[(int64_t)c * gridDim.x + blockIdx.x] = s;
+    }
+}
+
+// z(pivot i) = sum_{c >= i} X[c][i] w_c   (L11^-T w): 64 pivots per workgroup,
+// 16 waves over the rows c of X (coalesced; zero above the diagonal).  K = 500:
+// 13 us, 75 us with a thread per pivot.
+__global__ __launch_bounds__(1024) void k_pca_final(int32_t K, const int32_t* __restrict__ perm,
+                                                    const double* __restrict__ X, const double* __restrict__ w,
+                                                    double* __restrict__ z) {
+    __shared__ double red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t i0 = blockIdx.x * 64, i = min(i0 + lane, K - 1);
+    double a = 0.0;
+#pragma unroll 8
+    for (int32_t c = i0 + wave; c < K; c += 16) a += X[(int64_t)c * K + i] * w[c];
+    red[wave][lane] = a;
+    __syncthreads();
+    if (wave != 0 || i0 + lane >= K) return;
+    a = 0.0;
+#pragma unroll
+    for (int g = 0; g < 16; ++g) a += red[g][lane];
+    z[perm[i]] = a;
 }
 
 // ---- conjugate gradients with the scalars on the device ----
@@ -512,20 +620,50 @@ __global__ void k_cg_init(double* __restrict__ s, double rr, double rz) {
 
 }  // namespace
 
-void build_row_split(int32_t m, const std::vector<int64_t>& rowptr, std::vector<RowChunk>& chunks,
-                     std::vector<int32_t>& hrow, std::vector<int32_t>& hptr, std::vector<int32_t>& mrow) {
+void build_row_split(int32_t m, int32_t n, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
+                     std::vector<RowChunk>& chunks, std::vector<int32_t>& hrow, std::vector<int32_t>& hptr,
+                     std::vector<int32_t>& mrow) {
     chunks.clear();
     hrow.clear();
     mrow.clear();
     hptr.assign(1, 0);
+    int64_t heavy = 0;
+    for (int32_t i = 0; i < m; ++i) {
+        const int64_t len = rowptr[i + 1] - rowptr[i];
+        if (len > kHeavyRow) heavy += len;
+        else if (len > kLightRow) mrow.push_back(i);
+    }
+    if (heavy == 0) return;
+    const int64_t len = std::min<int64_t>(kMaxChunk, std::max<int64_t>(kMinChunk, heavy / kChunkGoal));
+    // the chunks of every column block, row by row; partials numbered by row
+    std::vector<std::vector<RowChunk>> block((n + kColBlock - 1) / kColBlock);
+    int32_t slot = 0;
     for (int32_t i = 0; i < m; ++i) {
         const int64_t b = rowptr[i], e = rowptr[i + 1];
-        if (e - b <= kLightRow) continue;
-        if (e - b <= kHeavyRow) { mrow.push_back(i); continue; }
+        if (e - b <= kHeavyRow) continue;
         hrow.push_back(i);
-        for (int64_t p = b; p < e; p += kRowChunk) chunks.push_back({i, p, std::min(e, p + kRowChunk)});
-        hptr.push_back((int32_t)chunks.size());
+        int64_t p = b;
+        for (int64_t cb = 0; p < e; ++cb) {   // the row's columns ascend
+            const int64_t lim = (cb + 1) * (int64_t)kColBlock;
+            const int64_t q = lim >= n ? e : std::lower_bound(colind.begin() + p, colind.begin() + e, (int32_t)lim) - colind.begin();
+            for (; p < q; p += std::min(len, q - p)) block[cb].push_back({p, std::min(q, p + len), slot++});
+        }
+        hptr.push_back(slot);
     }
+    // eight contiguous runs of columns with equal nonzeros, one per XCD, dealt
+    // out in workgroups of four chunks in turn
+    std::vector<std::vector<RowChunk>> run(kXcds);
+    int64_t seen = 0;
+    for (const auto& bl : block)
+        for (const RowChunk& c : bl) {
+            run[std::min<int64_t>(kXcds - 1, seen * kXcds / heavy)].push_back(c);
+            seen += c.e - c.b;
+        }
+    size_t most = 0;
+    for (const auto& r : run) most = std::max(most, (r.size() + 3) / 4);
+    for (size_t w = 0; w < most; ++w)
+        for (const auto& r : run)
+            for (size_t k = 4 * w; k < 4 * w + 4; ++k) chunks.push_back(k < r.size() ? r[k] : RowChunk{0, 0, 0});
 }
 
 void launch_csr_split(const RowSplitDev& rs, const int64_t* rowptr, const int32_t* colind, const double* val,
@@ -538,10 +676,10 @@ void launch_csr_split(const RowSplitDev& rs, const int64_t* rowptr, const int32_
     }
     if (square) {
         help::launch_kernel(k_csr_light<true>, grid_for(rs.m), kB, 0, st, rs.m, rowptr, colind, val, x, y);
-        if (rs.nchunk) help::launch_kernel(k_csr_chunk<true>, rs.nchunk, kB, 0, st, rs.chunks, colind, val, x, rs.part);
+        if (rs.nchunk) help::launch_kernel(k_csr_chunk<true>, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, colind, val, x, rs.part);
     } else {
         help::launch_kernel(k_csr_light<false>, grid_for(rs.m), kB, 0, st, rs.m, rowptr, colind, val, x, y);
-        if (rs.nchunk) help::launch_kernel(k_csr_chunk<false>, rs.nchunk, kB, 0, st, rs.chunks, colind, val, x, rs.part);
+        if (rs.nchunk) help::launch_kernel(k_csr_chunk<false>, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, colind, val, x, rs.part);
     }
     if (rs.nheavy) help::launch_kernel(k_csr_heavy, (rs.nheavy + 3) / 4, kB, 0, st, rs.nheavy, rs.hrow, rs.hptr, rs.part, y);
 }
@@ -585,32 +723,59 @@ void launch_vdiv(int64_t n, const double* a, const double* b, double* out, hipSt
     if (n > 0) help::launch_kernel(k_vdiv, grid_for(n), kB, 0, st, n, a, b, out);
 }
 
-void launch_to_f32(int64_t n, const double* x, float* y, hipStream_t st) {
-    if (n > 0) help::launch_kernel(k_to_f32, grid_for(n), kB, 0, st, n, x, y);
+void launch_to_f32(int32_t m, int32_t K, const double* x, float* y, int64_t ld, hipStream_t st) {
+    if (m > 0 && K > 0) help::launch_kernel(k_to_f32, dim3(grid_for(m), K), kB, 0, st, m, x, y, ld);
+}
+
+// Columns per lane of the fused apply (16 groups of them): the factor's tile and
+// the FP64 sums of the transposed product take NC (sizeof(T) / 4 + 2) registers,
+// and NC = 64 spills, so K > 512 keeps the two passes.
+template <typename T>
+static int apply_cols(int32_t K) {
+    for (int nc = 8; nc <= 32; nc *= 2)
+        if (K <= 16 * nc) return nc;
+    return 0;
 }
 
 template <typename T>
-void launch_pc_apply(int32_t m, int32_t K, const int32_t* perm, const int32_t* pos, const T* L32,
+int pc_apply_blocks(int32_t m, int32_t K) {
+    if (apply_cols<T>(K)) return (int)std::min<int64_t>(kApplyBlocks, ((int64_t)m + 31) / 32);
+    return (int)(((int64_t)m + kLtRows - 1) / kLtRows);
+}
+
+template <typename T>
+void launch_pc_apply(int32_t m, int32_t K, int64_t ld, const int32_t* perm, const int32_t* pos, const T* L32,
                      const double* X, const double* S, const double* r, double* y1, double* ltpart, double* z,
                      hipStream_t st) {
     // K = 0: z = r / S
-    const int nb = (int)(((int64_t)m + kLtRows - 1) / kLtRows);
-    if (K > 0) help::launch_kernel(k_pca_y1, (K + 3) / 4, kB, 0, st, K, perm, X, r, y1);
-    help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, K, pos, L32, y1, S, r, z);
-    if (K > 0) {
-        help::launch_kernel(k_pca_lt<T>, nb, kB, 0, st, m, K, L32, z, ltpart);
-        double* w = y1 + kPcgMaxK;
-        help::launch_kernel(k_pca_w, (K + 3) / 4, kB, 0, st, K, nb, perm, y1, S, ltpart, w);
-        help::launch_kernel(k_pca_final, grid_for(K), kB, 0, st, K, perm, X, w, z);
+    if (K <= 0) {
+        help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, ld, K, pos, L32, y1, S, r, z);
+        return;
     }
+    const int nb = pc_apply_blocks<T>(m, K);
+    help::launch_kernel(k_pca_y1, (K + 3) / 4, kB, 0, st, K, perm, X, r, y1);
+    auto fused = [&](auto kern) { help::launch_kernel(kern, nb, 512, 0, st, m, ld, K, pos, L32, y1, S, r, z, ltpart); };
+    switch (apply_cols<T>(K)) {
+        case 8: fused(k_pca_fused<T, 8>); break;
+        case 16: fused(k_pca_fused<T, 16>); break;
+        case 32: fused(k_pca_fused<T, 32>); break;
+        default:
+            help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, ld, K, pos, L32, y1, S, r, z);
+            help::launch_kernel(k_pca_lt<T>, nb, kB, 0, st, m, ld, K, L32, z, ltpart);
+    }
+    double* w = y1 + kPcgMaxK;
+    help::launch_kernel(k_pca_w, (K + 3) / 4, kB, 0, st, K, nb, perm, y1, S, ltpart, w);
+    help::launch_kernel(k_pca_final, (K + 63) / 64, 1024, 0, st, K, perm, X, w, z);
 }
 
-template void launch_pc_apply<float>(int32_t, int32_t, const int32_t*, const int32_t*, const float*,
-                                      const double*, const double*, const double*, double*, double*, double*,
-                                      hipStream_t);
-template void launch_pc_apply<double>(int32_t, int32_t, const int32_t*, const int32_t*, const double*,
-                                       const double*, const double*, const double*, double*, double*, double*,
-                                       hipStream_t);
+#define HELP_INST(T)                                                                                         \
+    template int pc_apply_blocks<T>(int32_t, int32_t);                                                       \
+    template void launch_pc_apply<T>(int32_t, int32_t, int64_t, const int32_t*, const int32_t*, const T*,     \
+                                     const double*, const double*, const double*, double*, double*, double*,  \
+                                     hipStream_t);
+HELP_INST(float)
+HELP_INST(double)
+#undef HELP_INST
 
 void launch_cg_init(double* s, double rr, double rz, hipStream_t st) {
     help::launch_kernel(k_cg_init, 1, 64, 0, st, s, rr, rz);

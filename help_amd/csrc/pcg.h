@@ -13,31 +13,39 @@ namespace help {
 constexpr int kPcgMaxK = 1024;      // partial-Cholesky columns held in LDS by the kernels
 constexpr int kLightRow = 64;       // CSR rows up to this many nonzeros take one thread
 constexpr int kHeavyRow = 1024;     // CSR rows longer than this are split into chunks
-constexpr int kRowChunk = 4096;     // nonzeros per chunk of a heavy row
+constexpr int kMaxChunk = 2048;     // most nonzeros per chunk of a heavy row (a wave each)
+constexpr int kMinChunk = 256;
+constexpr int kChunkGoal = 8192;    // chunks that fill the chip (32 waves per CU)
+constexpr int kColBlock = 262144;   // columns per block of the heavy rows: 2 MB of x, half an XCD's L2
+constexpr int kXcds = 8;
 constexpr int kLtRows = 2048;       // rows per workgroup of the transposed factor product
+constexpr int kApplyBlocks = 512;   // most workgroups (and partials) of the fused apply: two per CU
 
 struct RowChunk {
-    int32_t row;
-    int64_t b, e;                   // nonzero range [b, e) of the row
+    int64_t b, e;                   // nonzero range [b, e) of one row; empty: padding
+    int32_t slot;                   // its place in the partial sums
 };
 
 // Row partition of a CSR matrix for deterministic products with heavy rows:
 // rows up to kLightRow nonzeros take one thread (sequential sum), rows up to
 // kHeavyRow one wave (lane-strided partial sums, fixed reduction tree), the
-// others are summed in chunks of kRowChunk by one workgroup each and
-// combined in chunk order.
+// others are summed in chunks by one wave each and combined in chunk order.
+// A chunk lies in one block of kColBlock columns, and the chunks are listed so
+// that each XCD (workgroups go to them in turn) walks its own contiguous run
+// of columns: the gathered part of x then stays in that XCD's L2.
 struct RowSplitDev {
     int32_t m = 0;
     int32_t nchunk = 0, nheavy = 0, nmed = 0;
     const int32_t* mrow = nullptr;   // medium rows
     const RowChunk* chunks = nullptr;
     const int32_t* hrow = nullptr;   // heavy rows
-    const int32_t* hptr = nullptr;   // chunk range of heavy row h: [hptr[h], hptr[h+1])
+    const int32_t* hptr = nullptr;   // partials of heavy row h: [hptr[h], hptr[h+1])
     double* part = nullptr;          // one partial per chunk
 };
 
-void build_row_split(int32_t m, const std::vector<int64_t>& rowptr, std::vector<RowChunk>& chunks,
-                     std::vector<int32_t>& hrow, std::vector<int32_t>& hptr, std::vector<int32_t>& mrow);
+void build_row_split(int32_t m, int32_t n, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
+                     std::vector<RowChunk>& chunks, std::vector<int32_t>& hrow, std::vector<int32_t>& hptr,
+                     std::vector<int32_t>& mrow);
 
 // y = A x (square = false) or y = (A .* A) x (square = true)
 void launch_csr_split(const RowSplitDev& rs, const int64_t* rowptr, const int32_t* colind,
@@ -63,13 +71,17 @@ void launch_pc_column(int32_t m, int32_t k, const int32_t* col, const int32_t* p
                       const double* w, const double* D, double* L, double* S, hipStream_t st);
 void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, double* L11,
                    double* X, hipStream_t st);
-void launch_to_f32(int64_t n, const double* x, float* y, hipStream_t st);
+// y (columns of ld >= m floats) = x (columns of m)
+void launch_to_f32(int32_t m, int32_t K, const double* x, float* y, int64_t ld, hipStream_t st);
 
 // ---- preconditioner apply z = M^-1 r (PCG.cpp:183-196) ----
-// y1: scratch of 2 * kPcgMaxK doubles; ltpart: K * ceil(m / kLtRows) doubles;
-// the m x K factor L32 in FP32 or FP64 (T = float / double)
+// y1: scratch of 2 * kPcgMaxK doubles; ltpart: K * pc_apply_blocks(m, K)
+// doubles; the m x K factor L32 in FP32 or FP64 (T = float / double), columns
+// ld apart
 template <typename T>
-void launch_pc_apply(int32_t m, int32_t K, const int32_t* perm, const int32_t* pos, const T* L32,
+int pc_apply_blocks(int32_t m, int32_t K);
+template <typename T>
+void launch_pc_apply(int32_t m, int32_t K, int64_t ld, const int32_t* perm, const int32_t* pos, const T* L32,
                      const double* X, const double* S, const double* r, double* y1, double* ltpart,
                      double* z, hipStream_t st);
 

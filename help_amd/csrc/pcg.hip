@@ -44,6 +44,7 @@ namespace help {
 
 struct PcgState {
     int32_t K = 0;
+    int64_t ld32 = 0;                // column stride of the FP32 factor: whole 128-byte lines
     DBuf<double> cg, part;           // CG scalars (kCgSlots) and reduction partials
     double* hpin = nullptr;          // pinned: the scalars of the last two iterations
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -68,8 +69,16 @@ void pcg_setup(help_gpu* h) {
     const int32_t m = h->m, n = h->n;
     P->K = std::max(0, std::min<int32_t>(std::min(h->opts.pcg_k, kPcgMaxK), m));
     const int64_t K = std::max<int32_t>(P->K, 1);
-    P->L.alloc((size_t)m * K);
-    if (h->opts.pcg_fp32_precond) P->L32.alloc((size_t)m * K);
+    // an even number of columns: the apply reads them in pairs, and a zero
+    // column follows an odd K
+    const int64_t K2 = (K + 1) / 2 * 2;
+    P->L.alloc((size_t)m * K2);
+    HIPCHK(hipMemsetAsync(P->L.p + (size_t)m * K, 0, sizeof(double) * (size_t)m * (K2 - K), st));
+    P->ld32 = ((int64_t)m + 31) / 32 * 32;
+    if (h->opts.pcg_fp32_precond) {
+        P->L32.alloc((size_t)P->ld32 * K2);
+        HIPCHK(hipMemsetAsync(P->L32.p + (size_t)P->ld32 * K, 0, sizeof(float) * (size_t)P->ld32 * (K2 - K), st));
+    }
     P->D.alloc(K);
     P->w.alloc(K);
     P->S.alloc(m);
@@ -78,7 +87,7 @@ void pcg_setup(help_gpu* h) {
     P->L11.alloc((size_t)K * K);
     P->X.alloc((size_t)K * K);
     P->y1.alloc(2 * kPcgMaxK);
-    P->ltpart.alloc((size_t)K * ((m + kLtRows - 1) / kLtRows));
+    P->ltpart.alloc((size_t)K * std::max(pc_apply_blocks<float>(m, P->K), pc_apply_blocks<double>(m, P->K)));
     P->pval.alloc(kArgmaxBlocks);
     P->pidx.alloc(kArgmaxBlocks);
     P->perm.alloc(m);
@@ -121,7 +130,7 @@ void pcg_renew(help_gpu* h) {
         launch_pc_column(m, k, P->col.p, P->pos.p, P->g.p, P->w.p, P->D.p, P->L.p, P->S.p, st);
     }
     launch_pc_l11(m, K, P->perm.p, P->L.p, P->L11.p, P->X.p, st);
-    if (h->opts.pcg_fp32_precond) launch_to_f32((int64_t)m * K, P->L.p, P->L32.p, st);
+    if (h->opts.pcg_fp32_precond) launch_to_f32(m, K, P->L.p, P->L32.p, P->ld32, st);
     HIPCHK(hipGetLastError());
 }
 
@@ -233,10 +242,10 @@ int pcg_solve(help_gpu* h, const double* rhs, const double* x0, double* x2, doub
 void pcg_precond(help_gpu* h, const double* v, double* out) {
     PcgState* P = h->pcg;
     if (h->opts.pcg_fp32_precond)
-        launch_pc_apply<float>(h->m, P->K, P->perm.p, P->pos.p, P->L32.p, P->X.p, P->S.p, v, P->y1.p,
+        launch_pc_apply<float>(h->m, P->K, P->ld32, P->perm.p, P->pos.p, P->L32.p, P->X.p, P->S.p, v, P->y1.p,
                                P->ltpart.p, out, h->st);
     else
-        launch_pc_apply<double>(h->m, P->K, P->perm.p, P->pos.p, P->L.p, P->X.p, P->S.p, v, P->y1.p,
+        launch_pc_apply<double>(h->m, P->K, h->m, P->perm.p, P->pos.p, P->L.p, P->X.p, P->S.p, v, P->y1.p,
                                 P->ltpart.p, out, h->st);
 }
 
@@ -252,10 +261,10 @@ void pcg_precond_noalloc(help_gpu* h, const double* v, double* out) {
                                  std::to_string(kNoAllocScratch));
     double* s = scratch_ptr();
     if (h->opts.pcg_fp32_precond)
-        launch_pc_apply<float>(h->m, P->K, P->perm.p, P->pos.p, P->L32.p, P->X.p, P->S.p, v, s,
+        launch_pc_apply<float>(h->m, P->K, P->ld32, P->perm.p, P->pos.p, P->L32.p, P->X.p, P->S.p, v, s,
                                s + 2 * kPcgMaxK, out, h->st);
     else
-        launch_pc_apply<double>(h->m, P->K, P->perm.p, P->pos.p, P->L.p, P->X.p, P->S.p, v, s,
+        launch_pc_apply<double>(h->m, P->K, h->m, P->perm.p, P->pos.p, P->L.p, P->X.p, P->S.p, v, s,
                                 s + 2 * kPcgMaxK, out, h->st);
 }
 

@@ -159,6 +159,58 @@ def test_preconditioner_apply_matches_oracle(name, maker, K, fp32):
     assert err <= (1e-5 if fp32 else 1e-12)
 
 
+@pytest.mark.parametrize("K", [1, 2, 127, 129, 256, 257, 512, 513])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_preconditioner_apply_column_counts(K, fp32):
+    """The one-pass apply holds 16 groups of 8, 16 or 32 columns (an odd K has a
+    zero column after it) and leaves K > 512 to two passes: K at these edges, m
+    not a multiple of its 32-row tiles, against the oracle within the bars of
+    test_preconditioner_apply_matches_oracle."""
+    inst = instances.random_lp(1237, 2400, 4, seed=61)
+    rng = np.random.default_rng(9)
+    d = np.exp(rng.uniform(-1, 1, inst.n) * np.log(10.0))
+    r = rng.standard_normal(inst.m)
+    _flush(f"pcg apply m={inst.m} K={K} fp32={fp32}")
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=K, pcg_fp32_precond=fp32)
+    be.construct(inst)
+    be.renew(d)
+    z = be.pcg_apply(r)
+    be.destruct()
+    rp, ci, pos = O.csr(inst)
+    cv = np.ascontiguousarray(inst.val[pos])
+    pc = O.PChol()
+    O.lib().or_pchol_build(inst.m, inst.n, O.i64(rp), O.i32(ci), O.d(cv), O.d(d), 0.0, 0.0, K, pc)
+    perm = np.ctypeslib.as_array(pc.perm, shape=(inst.m,)).copy()
+    rperm = np.ascontiguousarray(r[perm])
+    zp, work, zo = np.empty(inst.m), np.empty(2 * inst.m), np.empty(inst.m)
+    O.lib().or_pchol_apply(pc, O.d(rperm), O.d(zp), O.d(work))
+    O.lib().or_pchol_free(pc)
+    zo[perm] = zp
+    err = np.linalg.norm(z - zo) / np.linalg.norm(zo)
+    _flush(f"  rel err vs oracle {err:.3e}")
+    assert err <= (1e-5 if fp32 else 1e-12)
+
+
+def test_heavy_rows_in_column_blocks():
+    """Rows above 1,024 nonzeros are cut at column blocks (262,144 columns) and
+    into chunks dealt out to the XCDs: on an instance with three blocks, the
+    Schur diagonal before the first pivot (K = 0) is the diagonal of A D^-1 A^T
+    within the rounding of a sum of that many positive terms."""
+    inst = instances.zipf(2000, 600000, 6, 1.1, seed=62)
+    rng = np.random.default_rng(10)
+    d = np.exp(rng.uniform(-1, 1, inst.n) * np.log(10.0))
+    most = int(np.bincount(inst.rowind, minlength=inst.m).max())
+    _flush(f"heavy rows m={inst.m} n={inst.n} longest {most}")
+    assert most > 262144
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=0)
+    be.construct(inst)
+    be.renew(d)
+    _, _, S, _ = be.pcg_factor()
+    be.destruct()
+    ref = np.bincount(inst.rowind, inst.val ** 2 / np.repeat(d, np.diff(inst.colptr)), inst.m)
+    assert np.allclose(S, ref, rtol=most * np.finfo(float).eps, atol=0)
+
+
 def test_pcg_cap_reports_noconv():
     """A PCG solve stopped by pcg_max_iter short of pcg_tol returns
     HELP_ERR_NOCONV (with its last iterate and the residual in the stats),
