@@ -151,6 +151,17 @@ void build_schedules(help_gpu* h) {
         }
         return b;
     };
+    // the same for the panel columns alone
+    auto ea_panel_bytes = [&](int32_t s) {
+        double b = 0;
+        for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) {
+            const int32_t ch = S.child[t], cu = S.snrow[ch] - ncol(ch);
+            const int32_t* rel = S.relmap.data() + S.reloff[ch];
+            const double k = std::lower_bound(rel, rel + cu, ncol(s)) - rel;
+            b += 3.0 * 8.0 * k * (cu - (k - 1) / 2);
+        }
+        return b;
+    };
     // Phases, as soon as possible.  A small front is one SMALL launch; a
     // large front with P panels takes phases start .. start+P-1: extend-add
     // and panel 0 in the first, panel b in phase start+b, and the update
@@ -191,10 +202,29 @@ void build_schedules(help_gpu* h) {
         done[s] = r + npan[s] - 1;
         nphase = std::max(nphase, done[s] + 1);
     }
+    // A large front with few children, or with a large update matrix and up
+    // to kGatherKids of them, takes their update matrices where its own is
+    // written: the GEMM tile that forms U = (children) - L21 L21^T adds up the
+    // children's entries itself instead of reading back what an extend-add
+    // zeroed and read-modify-wrote.  Its extend-add then covers only the panel
+    // columns.  Same sums in the same order.  T = 200 staircase, nested
+    // dissection: extend-add 21.7 -> 4.0 ms, GEMM 34.5 -> 37.4 ms per renew
+    // (FP64).  A tile goes through its children one after the other, which
+    // costs a launch of few tiles more than the traffic saved: the 2,000-row
+    // random LP (fronts of up to 900 update rows with up to 20 children) took
+    // 2.39 ms per iteration gathered, 2.30 ms not.
+    auto gathered = [&](int32_t s) {
+        const int32_t kids = S.childptr[s + 1] - S.childptr[s];
+        return !smallf[s] && (kids <= 4 || (kids <= kGatherKids && S.snrow[s] - ncol(s) >= kGatherRows));
+    };
+    // its update matrix is parked between panels (kGemmFirst / kGemmNext)
+    auto parked = [&](int32_t s) { return folded(s, npan[s]) && (npan[s] + 1) / 2 > 1; };
     // Update-matrix placement.  Front s's update matrix is live from its
-    // first phase (its extend-add, or its small-front launch, zeroes it)
-    // through its parent's first phase (the parent's extend-add reads it),
-    // both inclusive; fronts whose lifetimes do not overlap share memory.
+    // first phase (its extend-add, or its small-front launch, zeroes it; a
+    // parked accumulator lies at the same offsets) or, gathered and not parked,
+    // from its last one (which writes it), through its parent's first phase
+    // (the parent's extend-add reads it) or, when the parent gathers, last
+    // phase, both inclusive; fronts whose lifetimes do not overlap share memory.
     // First fit over an address-ordered free list, phase by phase: the blocks
     // that died before the phase are freed, then its new ones are placed.
     {
@@ -203,8 +233,9 @@ void build_schedules(help_gpu* h) {
         for (int32_t s = 0; s < ns; ++s) {
             const int64_t cu = S.snrow[s] - ncol(s);
             if (cu <= 0) continue;
-            born[start[s]].push_back(s);
-            const int32_t last = S.sparent[s] >= 0 ? start[S.sparent[s]] : done[s];
+            born[gathered(s) && !parked(s) ? done[s] : start[s]].push_back(s);
+            const int32_t par = S.sparent[s];
+            const int32_t last = par < 0 ? done[s] : gathered(par) ? done[par] : start[par];
             dies[last + 1].push_back(s);
         }
         auto usize = [&](int32_t s) {
@@ -252,6 +283,26 @@ void build_schedules(help_gpu* h) {
             std::fprintf(stderr, "[help] update matrices: %lld elements placed (%lld without reuse)\n",
                          (long long)high, (long long)S.uoff[ns]);
     }
+    // children of the gathered fronts, and which of them touch each 16-row
+    // block of the front's update rows (bit t: child t)
+    std::vector<int32_t> g0(ns, -1), gblk(ns, 0);
+    std::vector<uint32_t>& gtouch = h->gtouch;
+    h->ginv_len = 0;
+    for (int32_t s = 0; s < ns; ++s) {
+        const int32_t nc = ncol(s), cu = S.snrow[s] - nc;
+        if (!gathered(s) || cu <= 0) continue;
+        g0[s] = (int32_t)h->gref.size();
+        gblk[s] = (int32_t)gtouch.size();
+        gtouch.resize(gtouch.size() + (cu + kTile - 1) / kTile * 4, 0);   // whole tiles
+        for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) {
+            const int32_t ch = S.child[t], chc = S.snrow[ch] - ncol(ch);
+            const int32_t* rel = S.relmap.data() + S.reloff[ch];
+            h->gref.push_back({h->uplan[ch], h->ginv_len, S.reloff[ch], chc, nc});
+            h->ginv_len += cu;
+            for (int32_t j = (int32_t)(std::lower_bound(rel, rel + chc, nc) - rel); j < chc; ++j)
+                gtouch[gblk[s] + (rel[j] - nc) / 16] |= 1u << (t - S.childptr[s]);
+        }
+    }
     // fronts by phase: small ones, large ones starting, large ones active
     // (some panel in the phase), large ones finishing
     std::vector<std::vector<int32_t>> at_small(nphase), at_start(nphase), at_active(nphase), at_done(nphase);
@@ -261,6 +312,57 @@ void build_schedules(help_gpu* h) {
         for (int32_t p = start[s]; p <= done[s]; ++p) at_active[p].push_back(s);
         at_done[done[s]].push_back(s);
     }
+    // GEMM tiles of a front's columns [cb, ce), rows down to c, by columns of
+    // tiles.  deal_tiles orders a launch's tiles: runs of whole tile columns of
+    // one front, the longest inner dimension first, dealt out to the XCDs
+    // (workgroups go to them in turn) by the least work so far.  The tiles of a
+    // run share panel rows in that XCD's L2, and the pieces of an
+    // update-matrix column that neighbouring tiles write meet there: 60,000
+    // tiles of 200 fronts with 16 columns were written at 3.74 TB/s by whole
+    // fronts, at 2.97 by single tile columns and at 2.89 by 4x4 squares (FP64).
+    // A run has at least a 64th of the launch, for the balance of the XCDs.
+    struct Run { int32_t off, count; double work; };   // work per tile
+    std::vector<Run> cols, runs;
+    std::vector<GemmTask> dealt;
+    constexpr int32_t kXcd = 8;
+    auto push_tiles = [&](GemmTask g, int32_t cb, int32_t ce, int32_t c, double& wg) {
+        for (int32_t c0 = cb; c0 < ce; c0 += kTile) {
+            const int32_t off = (int32_t)h->gemm.size();
+            for (int32_t r0 = c0; r0 < c; r0 += kTile) {
+                g.row0 = r0;
+                g.col0 = c0;
+                h->gemm.push_back(g);
+                wg += 2.0 * (g.k1 - g.k0) * tile_lower_entries(r0, c0, c, g.col_end);
+            }
+            cols.push_back({off, (int32_t)h->gemm.size() - off, (double)(g.k1 - g.k0 + kTile)});
+        }
+    };
+    auto deal_tiles = [&](int32_t go) {
+        const int32_t cnt = (int32_t)h->gemm.size() - go;
+        runs.clear();
+        for (const Run& q : cols) {
+            if (!runs.empty() && runs.back().count < cnt / 64 && runs.back().work == q.work &&
+                h->gemm[runs.back().off].s == h->gemm[q.off].s)
+                runs.back().count += q.count;
+            else
+                runs.push_back(q);
+        }
+        cols.clear();
+        if ((int32_t)runs.size() <= kXcd) return;
+        std::stable_sort(runs.begin(), runs.end(), [](const Run& a, const Run& b) { return a.work > b.work; });
+        std::vector<std::pair<double, std::vector<int32_t>>> lane(kXcd);
+        for (const Run& q : runs) {
+            auto it = std::min_element(lane.begin(), lane.end(),
+                                       [](const auto& a, const auto& b) { return a.first < b.first; });
+            it->first += q.work * q.count;
+            for (int32_t t = 0; t < q.count; ++t) it->second.push_back(q.off + t);
+        }
+        dealt.clear();
+        for (size_t i = 0; (int32_t)dealt.size() < cnt; ++i)
+            for (const auto& l : lane)
+                if (i < l.second.size()) dealt.push_back(h->gemm[l.second[i]]);
+        std::copy(dealt.begin(), dealt.end(), h->gemm.begin() + go);
+    };
     for (int32_t p = 0; p < nphase; ++p) {
         if (!at_small[p].empty()) {
             // fronts of at most 64 rows and 16 columns whose panel and
@@ -305,27 +407,29 @@ void build_schedules(help_gpu* h) {
         if (at_active[p].empty()) continue;
         // extend-add by kEaCols-column chunks of each starting front; the
         // same tasks first zero the front's update matrix (a childless front
-        // gets the tasks of its update-matrix columns for that alone)
+        // gets the tasks of its update-matrix columns for that alone).  A
+        // gathered front has tasks for its panel columns only.
         int32_t off = (int32_t)h->ea.size();
         double w = 0;
         std::vector<int32_t> chunk_cnt, chunk_fill;
         for (int32_t s : at_start[p]) {
             const int32_t c = S.snrow[s], nc = ncol(s);
-            const bool leaf = S.childptr[s + 1] == S.childptr[s];
-            if (leaf && c == nc) continue;
-            w += ea_bytes(s) + 4.0 * (c - nc) * (c - nc + 1);
+            const bool leaf = S.childptr[s + 1] == S.childptr[s], gat = gathered(s);
+            if (leaf && (gat || c == nc)) continue;
+            const int32_t cend = gat ? nc : c;   // columns of the front's tasks
+            w += gat ? ea_panel_bytes(s) : ea_bytes(s) + 4.0 * (c - nc) * (c - nc + 1);
             // each child's relative map is ascending: one walk over it cuts it
             // into the kEaCols-column chunks it touches, and the chunks' child
             // lists are filled child by child (child order within a chunk)
-            const int32_t nchunk = (c + kEaCols - 1) / kEaCols;
+            const int32_t nchunk = (cend + kEaCols - 1) / kEaCols;
             chunk_cnt.assign(nchunk + 1, 0);
             for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) {
                 const int32_t ch = S.child[t];
                 const int32_t chc = S.snrow[ch] - ncol(ch);
                 const int32_t* rel = S.relmap.data() + S.reloff[ch];
-                for (int32_t j = 0; j < chc;) {
+                for (int32_t j = 0; j < chc && rel[j] < cend;) {
                     const int32_t k = rel[j] / kEaCols;
-                    while (j < chc && rel[j] / kEaCols == k) ++j;
+                    while (j < chc && rel[j] < cend && rel[j] / kEaCols == k) ++j;
                     chunk_cnt[k + 1]++;
                 }
             }
@@ -337,16 +441,16 @@ void build_schedules(help_gpu* h) {
                 const int32_t ch = S.child[t];
                 const int32_t chc = S.snrow[ch] - ncol(ch);
                 const int32_t* rel = S.relmap.data() + S.reloff[ch];
-                for (int32_t j = 0; j < chc;) {
+                for (int32_t j = 0; j < chc && rel[j] < cend;) {
                     const int32_t k = rel[j] / kEaCols, lo = j;
-                    while (j < chc && rel[j] / kEaCols == k) ++j;
+                    while (j < chc && rel[j] < cend && rel[j] / kEaCols == k) ++j;
                     h->earef[base + chunk_fill[k]++] = {h->uplan[ch], S.reloff[ch], chc, lo, j};
                 }
             }
             // a task per chunk with children, and per update-matrix chunk
             // (its columns are zeroed there)
             for (int32_t k = leaf ? nc / kEaCols : 0; k < nchunk; ++k) {
-                const int32_t c0 = k * kEaCols, c1 = std::min(c, c0 + kEaCols);
+                const int32_t c0 = k * kEaCols, c1 = std::min(cend, c0 + kEaCols);
                 const int32_t nref = chunk_cnt[k + 1] - chunk_cnt[k];
                 if (nref == 0 && c1 <= nc) continue;
                 h->ea.push_back({s, c0, c1, base + chunk_cnt[k], nref, nc, c, S.loff[s], h->uplan[s]});
@@ -382,14 +486,7 @@ void build_schedules(help_gpu* h) {
             const int32_t pb = p - start[s], P = npan[s];
             const bool pair_first = (pb % 2 == 0) && pb + 1 < P;
             const int32_t kp = (pb % 2 == 1) ? b - kTile : b;   // first panel not yet applied
-            for (int32_t c0 = b + nb; c0 < nc; c0 += kTile) {
-                if (pair_first && c0 > b + nb) break;
-                const int32_t k0 = pair_first ? b : kp;
-                for (int32_t r0 = c0; r0 < c; r0 += kTile) {
-                    h->gemm.push_back({s, r0, c0, k0, b + nb, nc});
-                    wg += 2.0 * (b + nb - k0) * tile_lower_entries(r0, c0, c, nc);
-                }
-            }
+            push_tiles({s, 0, 0, pair_first ? b : kp, b + nb, nc}, b + nb, pair_first ? std::min(nc, b + nb + kTile) : nc, c, wg);
             if (folded(s, npan[s]) && !pair_first) {
                 // update points: the second panel of each pair and the last
                 const int32_t q = pb / 2, Q = (P + 1) / 2;
@@ -398,13 +495,7 @@ void build_schedules(help_gpu* h) {
                 else if (q == 0) mode = kGemmFirst;
                 else if (q == Q - 1) mode = kGemmLast;
                 if (Q > 1) h->use_uacc = true;
-                for (int32_t c0 = nc; c0 < c; c0 += kTile)
-                    for (int32_t r0 = c0; r0 < c; r0 += kTile) {
-                        GemmTask g{s, r0, c0, k0, k1, c};
-                        g.mode = mode;
-                        h->gemm.push_back(g);
-                        wg += 2.0 * (k1 - k0) * tile_lower_entries(r0, c0, c, c);
-                    }
+                push_tiles({s, 0, 0, k0, k1, c, mode}, nc, c, c, wg);
             }
         }
         // FP64: one fused launch for the phase's panels when its workgroups
@@ -423,20 +514,17 @@ void build_schedules(help_gpu* h) {
             h->fops.push_back(ot);
         }
         if ((int32_t)h->gemm.size() > go) h->fops.push_back({OP_GEMM, go, (int32_t)h->gemm.size() - go, wg});
+        deal_tiles(go);
         // U -= L21 L21^T with the whole panel as inner dimension, for the
         // fronts whose last panel is this phase's
         go = (int32_t)h->gemm.size();
         wg = 0;
         for (int32_t s : at_done[p]) {
             const int32_t nc = ncol(s), c = S.snrow[s];
-            if (folded(s, npan[s])) continue;
-            for (int32_t c0 = nc; c0 < c; c0 += kTile)
-                for (int32_t r0 = c0; r0 < c; r0 += kTile) {
-                    h->gemm.push_back({s, r0, c0, 0, nc, c});
-                    wg += 2.0 * nc * tile_lower_entries(r0, c0, c, c);
-                }
+            if (!folded(s, npan[s])) push_tiles({s, 0, 0, 0, nc, c}, nc, c, c, wg);
         }
         if ((int32_t)h->gemm.size() > go) h->fops.push_back({OP_GEMM, go, (int32_t)h->gemm.size() - go, wg});
+        deal_tiles(go);
         // Inverse blocks of the wide fronts, right-looking: task (i, j, k)
         // finalises X_kj (i = k) or adds L_ik X_kj to the partial sum of X_ij
         // (i > k), and every partial sum takes its terms in increasing k.
@@ -493,6 +581,12 @@ void build_schedules(help_gpu* h) {
         g.c = S.snrow[g.s];
         g.loff = S.loff[g.s];
         g.uoff = h->uplan[g.s];
+        if (g.col0 >= g.n && g0[g.s] >= 0) {
+            g.g0 = g0[g.s];
+            const uint32_t* touch = gtouch.data() + gblk[g.s] + (g.row0 - g.n) / 16;
+            g.gmask = touch[0] | touch[1] | touch[2] | touch[3];
+            g.gcol = gblk[g.s] + (g.col0 - g.n) / 16;
+        }
     }
     // triangular solves
     // algorithmic bytes of the solves: each stored factor entry is read once
@@ -669,6 +763,10 @@ void setup_device_factor(help_gpu* h) {
     h->d_big.upload(h->sbig, st);
     h->d_ea.upload(h->ea, st);
     h->d_earef.upload(h->earef, st);
+    h->d_gref.upload(h->gref, st);
+    h->d_gtouch.upload(h->gtouch, st);
+    h->d_ginv.alloc(std::max<int64_t>(1, h->ginv_len));
+    launch_gather_maps(h->d_gref.p, (int32_t)h->gref.size(), h->d_relmap.p, h->d_ginv.p, h->ginv_len, st);
     h->d_potrf.upload(h->potrf, st);
     h->d_panel.upload(h->panel, st);
     h->d_pcopy.upload(h->pcopy, st);
@@ -787,7 +885,9 @@ void run_factor(help_gpu* h, T* L, T* U, T* Dinv) {
                 launch_potrf_diag<T>(h->d_potrf.p + o.off, o.count, h->sym, L, Dinv, h->d_err.p, st);
                 break;
             case OP_TRSM: launch_trsm_rows<T>(h->d_trsm.p + o.off, o.count, h->sym, L, Dinv, st); break;
-            case OP_GEMM: launch_gemm<T>(h->d_gemm.p + o.off, o.count, h->sym, L, U, uacc_store<T>(h), st); break;
+            case OP_GEMM:
+                launch_gemm<T>(h->d_gemm.p + o.off, o.count, h->d_gref.p, h->d_ginv.p, h->d_gtouch.p, L, U, uacc_store<T>(h), st);
+                break;
             case OP_XINV: launch_xinv<T>(h->d_xtask.p + o.off, o.count, h->sym, L, Dinv, xinv_store<T>(h), xinv_partial<T>(h), h->st_side); break;
             default: break;
         }

@@ -54,8 +54,30 @@ struct GemmTask {
     // everything its addresses depend on
     int32_t n = 0, c = 0;
     int64_t loff = 0, uoff = 0;
+    // update-matrix tile of a front whose children are gathered (C starts
+    // from their sum instead of from memory): refs[g0 + t] is child t; bit t
+    // of gmask says that it has rows in the tile's, bit t of touch[gcol + w]
+    // that it has some in columns 16 w .. 16 w + 15 of the tile.  g0 < 0: C is
+    // read.
+    int32_t g0 = -1;
+    uint32_t gmask = 0;
+    int32_t gcol = 0;
+    int32_t pad = 0;
 };
 enum : int32_t { kGemmDirect = 0, kGemmFirst = 1, kGemmNext = 2, kGemmLast = 3 };
+// A child of a gathered front: its update matrix (chc rows and columns) and
+// the inverse of its relative map over the front's update rows: inv[i - n] is
+// the child's update row that lands on front row i, or -1.
+struct GatherRef {
+    int64_t uoff;
+    int64_t invoff;
+    int64_t reloff;
+    int32_t chc;
+    int32_t n;            // the front's columns
+};
+// children a front may have to be gathered: the bits of GemmTask::gmask
+constexpr int kGatherKids = 32;
+constexpr int kGatherRows = 1024;   // update rows from which more than four are gathered
 
 // Panel task: factor the diagonal block [b, b+nb) of front s (every task of
 // the step does it redundantly in LDS) and solve the rows of block rb below it.
@@ -176,7 +198,11 @@ template <typename T>
 void launch_trsm_rows(const PanelTask* tasks, int32_t count, DevSym sym, T* L, const T* Dinv,
                       hipStream_t st);
 template <typename T>
-void launch_gemm(const GemmTask* tasks, int32_t count, DevSym sym, T* L, T* U, T* Uacc, hipStream_t st);
+void launch_gemm(const GemmTask* tasks, int32_t count, const GatherRef* grefs, const int32_t* ginv,
+                 const uint32_t* gtouch, T* L, T* U, T* Uacc, hipStream_t st);
+// inv (len entries) of every gathered child from the relative maps
+void launch_gather_maps(const GatherRef* grefs, int32_t count, const int32_t* relmap, int32_t* inv, int64_t len,
+                        hipStream_t st);
 template <typename T>
 void launch_mfma_probe(const T* a, const T* b, T* out, hipStream_t st);
 // off-diagonal inverse blocks X_ij = -Dinv_i S_ij, S_ij = sum_{k=j}^{i-1} L_ik X_kj

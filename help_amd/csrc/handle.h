@@ -118,6 +118,9 @@ struct help_gpu {
     std::vector<int32_t> list_small, list_fwd, list_bwd;
     std::vector<EaTask> ea;
     std::vector<help::EaRef> earef;
+    std::vector<help::GatherRef> gref;
+    std::vector<uint32_t> gtouch;        // which of them touch each 16 update rows of the front
+    int64_t ginv_len = 0;
     std::vector<PanelTask> potrf, trsm, panel;
     std::vector<PanelTask> pcopy;   // diagonal blocks factored by fused panel launches
     std::vector<GemmTask> gemm;
@@ -165,6 +168,9 @@ struct help_gpu {
     DBuf<int8_t> d_big;
     DBuf<EaTask> d_ea;
     DBuf<help::EaRef> d_earef;
+    DBuf<help::GatherRef> d_gref;
+    DBuf<int32_t> d_ginv;
+    DBuf<uint32_t> d_gtouch;
     DBuf<PanelTask> d_potrf, d_trsm, d_panel, d_pcopy;
     DBuf<GemmTask> d_gemm;
     DBuf<SolveTask> d_fgemv, d_bgemv, d_fxs, d_bxs;

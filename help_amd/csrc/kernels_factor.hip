@@ -920,6 +920,44 @@ __global__ __launch_bounds__(256) void k_copy_diag(const PanelTask* __restrict__
     }
 }
 
+// cv[q] = the children's update-matrix entries on this lane's row and column q
+// of the wave's 16, added in child order from zero.  mask: the children that
+// touch the wave's rows and columns; rf, ri, cl: the first one's reference,
+// the child row that lands on this lane's row (-1: none) and, lanes 0 to 15,
+// the child columns that land on the wave's; iu, jl: the lane's row and column
+// in the maps.  A column's address is uniform over the wave and a lane's row
+// is an offset to it; the next child's reference and maps are loaded beside
+// this one's entries.  Entries outside the lower part or the front get an
+// unused value from inside the child's matrix.
+template <typename T>
+__device__ inline void gather_children(const GatherRef* __restrict__ grefs, const int32_t* __restrict__ ginv,
+                                       const T* U, int32_t g0, uint32_t mask, GatherRef rf, int32_t ri, int32_t cl,
+                                       int32_t iu, int32_t jl, T (&cv)[16]) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) cv[q] = T(0);
+    while (mask) {
+        mask &= mask - 1;
+        const GatherRef nx = grefs[g0 + __builtin_ctz(mask ? mask : 1u)];
+        const int32_t nri = ginv[nx.invoff + iu], ncl = ginv[nx.invoff + jl];
+        const T* Uc = U + rf.uoff;
+        T v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = T(0);
+        if (ri >= 0) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const T* col = Uc + (int64_t)max(__builtin_amdgcn_readlane(cl, q), 0) * rf.chc;
+                v[q] = col[(uint32_t)ri];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) cv[q] += __builtin_amdgcn_readlane(cl, q) >= 0 ? v[q] : T(0);
+        rf = nx;
+        ri = nri;
+        cl = ncl;
+    }
+}
+
 constexpr int kKc = 16;   // inner-dimension chunk staged in LDS
 
 // C[row0:+64, col0:+64] -= P[rows, k0:k1] * P[cols, k0:k1]^T, lower part only,
@@ -929,8 +967,9 @@ constexpr int kKc = 16;   // inner-dimension chunk staged in LDS
 // asked of the register allocation (the interior tiles' loads into LDS need
 // no staging registers).
 template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(const GemmTask* __restrict__ tasks, DevSym sym,
-                                              T* __restrict__ L, T* __restrict__ U, T* __restrict__ Uacc) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(const GemmTask* __restrict__ tasks,
+                                              const GatherRef* __restrict__ grefs, const int32_t* __restrict__ ginv,
+                                              const uint32_t* __restrict__ gtouch, T* __restrict__ L, T* U, T* __restrict__ Uacc) {
     typedef typename Mfma<T>::acc_t acc_t;
     constexpr int kPer = kKc / 4;
     // the double-buffered k chunks, and after the product the 64x64
@@ -968,6 +1007,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     const bool ok = i < c && j < tk.col_end && i >= j;
                     acc[a][b][r] = Ua[ok ? (int64_t)(j - n) * cu + (i - n) : 0];
                 }
+    }
+    // the first of the children that touch this wave's columns (gathered
+    // update matrix, below): its reference and maps arrive during the product
+    const int32_t iu = min(tk.row0 + lane, c - 1) - n;
+    const int32_t jl = min(tk.col0 + 16 * wave + (lane & 15), c - 1) - n;
+    uint32_t mask = 0;
+    GatherRef rf{};
+    int32_t ri = -1, cl = -1;
+    if (tk.g0 >= 0) mask = tk.gmask & gtouch[tk.gcol + __builtin_amdgcn_readfirstlane(wave)];
+    if (mask) {
+        rf = grefs[tk.g0 + __builtin_ctz(mask)];
+        ri = ginv[rf.invoff + iu];
+        cl = ginv[rf.invoff + jl];
     }
     if (tk.row0 + kTile <= c && tk.col0 + kTile <= c) {   // uniform over the workgroup
         // Interior tile: the chunks go from HBM straight into LDS
@@ -1121,13 +1173,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     bool okv[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
-        const int32_t tj = tj0 + q, j = tk.col0 + tj;
+        const int32_t j = tk.col0 + tj0 + q;
         okv[q] = i < c && j < tk.col_end && i >= j;
-        cv[q] = Ct[okv[q] ? tj * ld + ti : 0];
+    }
+    if (tk.g0 >= 0) {
+        gather_children<T>(grefs, ginv, U, tk.g0, mask, rf, ri, cl, iu, jl, cv);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) cv[q] = Ct[okv[q] ? (tj0 + q) * ld + ti : 0];
     }
 #pragma unroll
     for (int q = 0; q < 16; ++q)
         if (okv[q]) Ct[(tj0 + q) * ld + ti] = cv[q] - Cs[(tj0 + q) * kCLd + ti];
+}
+
+// inverse relative maps of the gathered children, a workgroup each (inv is -1
+// on entry)
+__global__ __launch_bounds__(256) void k_gather_maps(const GatherRef* __restrict__ grefs,
+                                                     const int32_t* __restrict__ relmap, int32_t* __restrict__ inv) {
+    const GatherRef rf = grefs[blockIdx.x];
+    for (int32_t t = threadIdx.x; t < rf.chc; t += 256) {
+        const int32_t r = relmap[rf.reloff + t];
+        if (r >= rf.n) inv[rf.invoff + r - rf.n] = t;
+    }
+}
+__global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int32_t v, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = v;
 }
 
 // X := X L_bb^-T for the 64 rows of block rb-1 below the diagonal block,
@@ -1360,8 +1432,9 @@ void launch_extend_add(const EaTask* tasks, int32_t count, const EaRef* refs, De
     else help::launch_kernel(k_extend_add<T, 4>, count, 256, 0, st, tasks, refs, sym, L, U);
 }
 template <typename T>
-void launch_gemm(const GemmTask* tasks, int32_t count, DevSym sym, T* L, T* U, T* Uacc, hipStream_t st) {
-    if (count > 0) help::launch_kernel(k_gemm<T>, count, 256, 0, st, tasks, sym, L, U, Uacc);
+void launch_gemm(const GemmTask* tasks, int32_t count, const GatherRef* grefs, const int32_t* ginv,
+                 const uint32_t* gtouch, T* L, T* U, T* Uacc, hipStream_t st) {
+    if (count > 0) help::launch_kernel(k_gemm<T>, count, 256, 0, st, tasks, grefs, ginv, gtouch, L, U, Uacc);
 }
 
 template <typename T>
@@ -1394,13 +1467,21 @@ void launch_xinv(const XTask* tasks, int32_t count, DevSym sym, const T* L, cons
     if (count > 0) help::launch_kernel(k_xinv<T>, count, 256, 0, st, tasks, sym, L, Dinv, X, S);
 }
 
+void launch_gather_maps(const GatherRef* grefs, int32_t count, const int32_t* relmap, int32_t* inv, int64_t len,
+                        hipStream_t st) {
+    if (count <= 0) return;
+    help::launch_kernel(k_fill_i32, (unsigned)((len + 255) / 256), 256, 0, st, inv, -1, len);
+    help::launch_kernel(k_gather_maps, count, 256, 0, st, grefs, relmap, inv);
+}
+
 #define HELP_INST(T)                                                                                \
     template void launch_small_fronts<T>(const int32_t*, int32_t, DevSym, T*, T*, T*, int32_t*,      \
                                          int32_t, hipStream_t);                                     \
     template void launch_small_wave<T>(const int32_t*, int32_t, DevSym, T*, T*, T*, int32_t*,        \
                                        int32_t, int32_t, hipStream_t);                              \
     template void launch_extend_add<T>(const EaTask*, int32_t, const EaRef*, DevSym, T*, T*, int32_t, hipStream_t); \
-    template void launch_gemm<T>(const GemmTask*, int32_t, DevSym, T*, T*, T*, hipStream_t);           \
+    template void launch_gemm<T>(const GemmTask*, int32_t, const GatherRef*, const int32_t*, const uint32_t*, T*, T*, T*, \
+                                 hipStream_t);                                                      \
     template void launch_potrf_diag<T>(const PanelTask*, int32_t, DevSym, T*, T*, int32_t*,        \
                                        hipStream_t);                                                \
     template void launch_trsm_rows<T>(const PanelTask*, int32_t, DevSym, T*, const T*, hipStream_t);     \

@@ -109,6 +109,40 @@ def test_factor_matches_oracle(be0, cfg0):
     assert worst <= 1e-12, worst
 
 
+@pytest.mark.parametrize("ordering", [L.ORDER_AMD, L.ORDER_ND])
+def test_factor_gathered_fronts(ordering):
+    """Fronts whose update-matrix tiles add up their children's entries
+    themselves: few children, and many (more than four, at least 1,024 update
+    rows), with update rows that are no multiple of a tile; L within 1e-12 of
+    the oracle's per column, as in test_factor_matches_oracle."""
+    inst = instances.staircase(3, 1000, 3000, 5, seed=27)
+    rng = np.random.default_rng(14)
+    d = log_uniform(rng, inst.n, -2, 2)
+    be = LinearEquation(ordering=ordering)
+    be.construct(inst)
+    sf, nr, _, tiled = be.supernodes()
+    perm, parent, _ = be.symbolic_arrays()
+    sn = np.repeat(np.arange(len(nr)), np.diff(sf))
+    up = parent[sf[1:] - 1]
+    kids = np.bincount(sn[up[up >= 0]], minlength=len(nr))
+    cu = nr - np.diff(sf)
+    many = (tiled == 1) & (kids > 4) & (cu >= 1024)
+    few = (tiled == 1) & (kids > 0) & (kids <= 4) & (cu > 0)
+    _flush(f"gathered fronts ordering={ordering}: {few.sum()} with few children, {many.sum()} with many")
+    assert many.any() and few.any() and (cu[many | few] % 64 != 0).any()
+    be.renew(d)
+    Lp, Li, Lx = _oracle_factor(inst, perm, d)
+    worst = 0.0
+    for j in list(range(0, inst.m, 37)) + [inst.m - 1]:
+        rows, vals = be.factor_column(j)
+        got = np.zeros(inst.m)
+        got[rows] = vals
+        got[Li[Lp[j]:Lp[j + 1]]] -= Lx[Lp[j]:Lp[j + 1]]
+        worst = max(worst, np.abs(got).max() / np.abs(Lx[Lp[j]:Lp[j + 1]]).max())
+    be.destruct()
+    assert worst <= 1e-12, worst
+
+
 @pytest.mark.parametrize("mode", [L.MODE_DIRECT_FP64, L.MODE_DIRECT_FP32])
 def test_solve_matches_oracle(cfg0, mode):
     be = LinearEquation(mode=mode)
