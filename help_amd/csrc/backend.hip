@@ -728,6 +728,7 @@ void setup_device_common(help_gpu* h) {
     h->rows.hrow = h->d_hrow.p;
     h->rows.hptr = h->d_hptr.p;
     h->rows.part = h->d_rpart.p;
+    h->rows.nparts = hptr.back();
     h->rows.nmed = (int32_t)mrow.size();
     h->rows.mrow = h->d_mrow.p;
 }

@@ -6,10 +6,10 @@
 //   longer rows are cut into chunks, one wave each, combined in chunk order:
 //   deterministic.
 // * Greedy partial Cholesky (PCG.cpp:38-103): per pivot an argmax over the
-//   Schur diagonal, the pivot row of A scattered into an n-vector, one
-//   product with A for the pivot's column of ADA^T, and a left-looking
-//   column update against the previous columns (column-major m x K factor,
-//   so the thread-per-row update reads coalesced).
+//   Schur diagonal; the candidates' rows of A scattered into n-vectors, their
+//   columns of ADA^T and their left-looking updates against the previous
+//   columns in blocks of kPcBlk (column-major m x K factor, so the
+//   thread-per-row update reads coalesced).
 // * Preconditioner apply (PCG.cpp:183-196) with the factor in FP32: the
 //   product and the transposed product in one pass over the m x K factor.
 #include <algorithm>
@@ -171,73 +171,304 @@ __device__ inline bool better(double v, int32_t i, double bv, int32_t bi) {
     return v > bv || (v == bv && i < bi);
 }
 
-__global__ __launch_bounds__(256) void k_pc_argmax_part(int32_t m, int32_t k, const int32_t* __restrict__ perm,
-                                                        const double* __restrict__ S, double* __restrict__ pval,
-                                                        int32_t* __restrict__ pidx) {
-    __shared__ double sv[kB];
-    __shared__ int32_t si[kB];
+// The pivots are taken kPcBlk at a time.  A block starts with kPcBlk
+// candidates, the largest Schur diagonals (ties to the lowest position); their
+// columns of A D^-1 A^T and their left-looking sums over all finished factor
+// columns are formed together, so the m x k factor and A are read once per
+// block instead of once per pivot.  Each step then takes the pivot as before,
+// the largest Schur diagonal of all, and adds the block's own columns; when
+// that pivot is none of the candidates the block ends there and the next one
+// starts with it.  The order of the pivots is the greedy one whatever the
+// candidates, and a column's sum over the earlier ones keeps its four
+// interleaved chains (PCG.cpp:85-102 in that order), so light rows round as
+// with one column at a time.  The state (PcState) stays on the device: every
+// kernel returns at once when its block has ended.
+// m = 10^6, K = 500 (zipf): 64.3 ms per build, 291 ms pivot by pivot (of which
+// the factor reads 178 ms and the products with A 100 ms).
+typedef PcBest Best;
+__device__ inline bool ahead(const Best& a, const Best& b) { return better(a.v, a.pos, b.v, b.pos); }
+
+__device__ inline Best block_best(Best x, Best* red) {
     const int t = threadIdx.x;
-    double bv = -HUGE_VAL;
-    int32_t bi = INT_MAX;
-    for (int64_t i = (int64_t)k + (int64_t)blockIdx.x * kB + t; i < m; i += (int64_t)gridDim.x * kB) {
-        const double v = S[perm[i]];
-        if (better(v, (int32_t)i, bv, bi)) { bv = v; bi = (int32_t)i; }
-    }
-    sv[t] = bv;
-    si[t] = bi;
+    red[t] = x;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
-        if (t < w && better(sv[t + w], si[t + w], sv[t], si[t])) { sv[t] = sv[t + w]; si[t] = si[t + w]; }
+        if (t < w && ahead(red[t + w], red[t])) red[t] = red[t + w];
         __syncthreads();
     }
-    if (t == 0) { pval[blockIdx.x] = sv[0]; pidx[blockIdx.x] = si[0]; }
-}
-
-__global__ __launch_bounds__(256) void k_pc_pick(int32_t nb, int32_t k, const double* __restrict__ pval,
-                                                 const int32_t* __restrict__ pidx, int32_t* __restrict__ perm,
-                                                 int32_t* __restrict__ pos, int32_t* __restrict__ col_out) {
-    __shared__ double sv[kB];
-    __shared__ int32_t si[kB];
-    const int t = threadIdx.x;
-    double bv = -HUGE_VAL;
-    int32_t bi = INT_MAX;
-    for (int b = t; b < nb; b += kB)
-        if (better(pval[b], pidx[b], bv, bi)) { bv = pval[b]; bi = pidx[b]; }
-    sv[t] = bv;
-    si[t] = bi;
+    const Best b = red[0];
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w && better(sv[t + w], si[t + w], sv[t], si[t])) { sv[t] = sv[t + w]; si[t] = si[t + w]; }
-        __syncthreads();
-    }
-    if (t == 0) {
-        int32_t cm = si[0] == INT_MAX ? k : si[0];
-        const int32_t a = perm[k], b = perm[cm];
-        perm[k] = b;
-        perm[cm] = a;
-        pos[a] = cm;
-        pos[b] = k;
-        *col_out = b;
+    return b;
+}
+
+// the block's kPcBlk best rows not yet pivoted, in order; the first one is also
+// its argmax partial
+__global__ __launch_bounds__(256) void k_pc_top_part(int32_t m, const int32_t* __restrict__ pos,
+                                                     const double* __restrict__ S, const PcState* __restrict__ st,
+                                                     PcBest* __restrict__ top, PcBest* __restrict__ arg) {
+    __shared__ Best red[kB];
+    const int32_t k = st->k;
+    const Best none = {-HUGE_VAL, INT_MAX, -1};
+    // this thread's best row strictly behind `last`
+    auto next = [&](const Best& last) {
+        Best b = none;
+        for (int64_t j = (int64_t)blockIdx.x * kB + threadIdx.x; j < m; j += (int64_t)gridDim.x * kB) {
+            const Best c = {S[j], pos[j], (int32_t)j};
+            if (c.pos >= k && ahead(last, c) && ahead(c, b)) b = c;
+        }
+        return b;
+    };
+    Best mine = next({HUGE_VAL, -1, -1});
+    for (int r = 0; r < kPcBlk; ++r) {
+        const Best b = block_best(mine, red);
+        if (threadIdx.x == 0) {
+            top[blockIdx.x * kPcBlk + r] = b;
+            if (r == 0) arg[blockIdx.x] = b;
+        }
+        if (b.row >= 0 && b.row == mine.row) mine = next(b);
     }
 }
 
-__global__ void k_pc_scatter(const int32_t* __restrict__ colp, const int64_t* __restrict__ rowptr,
+// the candidates of the next block out of nb blocks' best
+__global__ __launch_bounds__(256) void k_pc_top_pick(int32_t nb, int32_t K, const PcBest* __restrict__ top,
+                                                     PcState* __restrict__ st) {
+    constexpr int kPer = kTopBlocks / kB;   // lists per thread, each in order
+    __shared__ Best red[kB];
+    const Best none = {-HUGE_VAL, INT_MAX, -1};
+    int at[kPer];
+    Best head[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int b = threadIdx.x + u * kB;
+        at[u] = 0;
+        head[u] = b < nb ? top[b * kPcBlk] : none;
+    }
+    const int32_t force = st->force;
+    if (threadIdx.x == 0 && force >= 0) st->cand[0] = force;
+    for (int r = force >= 0 ? 1 : 0; r < kPcBlk; ++r) {
+        Best mine = none;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            if (head[u].row >= 0 && ahead(head[u], mine)) mine = head[u];
+        const Best b = block_best(mine, red);
+        if (threadIdx.x == 0) st->cand[r] = b.row;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            if (b.row >= 0 && head[u].row == b.row)
+                head[u] = ++at[u] < kPcBlk ? top[(threadIdx.x + u * kB) * kPcBlk + at[u]] : none;
+    }
+    if (threadIdx.x == 0) {
+        st->k0 = st->k;
+        st->stop = st->k >= K;
+        st->force = -1;
+    }
+}
+
+// sc[j][c] = A(cand_c, j) dinv_j on the candidates' rows (blockIdx.y = c), or 0
+__global__ void k_pc_scatter(const PcState* __restrict__ st, const int64_t* __restrict__ rowptr,
                              const int32_t* __restrict__ colind, const double* __restrict__ val,
                              const double* __restrict__ dinv, double* __restrict__ sc, int clear) {
-    const int32_t col = *colp;
+    const int c = blockIdx.y;
+    const int32_t col = st->cand[c];
+    if (st->stop || col < 0) return;
     const int64_t b = rowptr[col], e = rowptr[col + 1];
     for (int64_t p = b + (int64_t)blockIdx.x * kB + threadIdx.x; p < e; p += (int64_t)gridDim.x * kB) {
         const int32_t j = colind[p];
-        sc[j] = clear ? 0.0 : val[p] * dinv[j];
+        sc[(int64_t)j * kPcBlk + c] = clear ? 0.0 : val[p] * dinv[j];
     }
 }
 
-// w_r = D_r L(col, r) for r < k and D_k = g(col) + delta - sum_r w_r L(col, r)
-__global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t k, const int32_t* __restrict__ colp,
-                                                  const double* __restrict__ g, const double* __restrict__ L,
-                                                  double delta, double* __restrict__ D, double* __restrict__ w) {
+// g[c][i] = sum_p val[p] sc[colind[p]][c]: the products of A with all candidates'
+// vectors, the candidate on the low lanes, so a nonzero's gather is one
+// 64-byte line.  Rows by length as in the single products.
+__global__ __launch_bounds__(256) void k_pc_csr_light(int32_t m, const PcState* __restrict__ st,
+                                                      const int64_t* __restrict__ rowptr,
+                                                      const int32_t* __restrict__ colind,
+                                                      const double* __restrict__ val, const double* __restrict__ sc,
+                                                      double* __restrict__ g) {
+    const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
+    const int64_t i = t / kPcBlk;
+    const int c = (int)(t % kPcBlk);
+    if (st->stop || i >= m) return;
+    const int64_t b = rowptr[i], e = rowptr[i + 1];
+    if (e - b > kLightRow) return;
+    double acc = 0.0;
+    for (int64_t p = b; p < e; p += 4) {
+        double x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = p + u < e ? p + u : e - 1;
+            x[u] = val[q] * sc[(int64_t)colind[q] * kPcBlk + c];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = (p + u < e) ? acc + x[u] : acc;
+    }
+    g[(int64_t)c * m + i] = acc;
+}
+
+// sum over the nonzeros [b, e) of one wave, 64 / kPcBlk at a time; the sums end
+// up on the first kPcBlk lanes
+__device__ inline double wave_range(int64_t b, int64_t e, const int32_t* __restrict__ colind,
+                                     const double* __restrict__ val, const double* __restrict__ sc, int lane) {
+    constexpr int kN = 64 / kPcBlk;
+    const int c = lane & (kPcBlk - 1);
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int64_t p0 = b + lane / kPcBlk; p0 < e; p0 += 8 * kN) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int64_t q = p0 + kN * u < e ? p0 + kN * u : e - 1;
+            x[u] = val[q] * sc[(int64_t)colind[q] * kPcBlk + c];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[u & 3] = (p0 + kN * u < e) ? a[u & 3] + x[u] : a[u & 3];
+    }
+    double s = (a[0] + a[1]) + (a[2] + a[3]);
+    for (int off = 32; off >= kPcBlk; off >>= 1) s += __shfl_xor(s, off);
+    return s;
+}
+
+__global__ __launch_bounds__(256) void k_pc_csr_medium(int32_t m, int32_t nmed, const int32_t* __restrict__ mrow,
+                                                       const PcState* __restrict__ st,
+                                                       const int64_t* __restrict__ rowptr,
+                                                       const int32_t* __restrict__ colind,
+                                                       const double* __restrict__ val, const double* __restrict__ sc,
+                                                       double* __restrict__ g) {
+    const int32_t h = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (st->stop || h >= nmed) return;
+    const int32_t i = mrow[h];
+    const double s = wave_range(rowptr[i], rowptr[i + 1], colind, val, sc, lane);
+    if (lane < kPcBlk) g[(int64_t)lane * m + i] = s;
+}
+
+__global__ __launch_bounds__(256) void k_pc_csr_chunk(int32_t nchunk, const RowChunk* __restrict__ chunks,
+                                                      const PcState* __restrict__ st,
+                                                      const int32_t* __restrict__ colind,
+                                                      const double* __restrict__ val, const double* __restrict__ sc,
+                                                      double* __restrict__ part) {
+    const int32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (st->stop || i >= nchunk) return;
+    const RowChunk c = chunks[i];
+    if (c.e <= c.b) return;   // padding
+    const double s = wave_range(c.b, c.e, colind, val, sc, lane);
+    if (lane < kPcBlk) part[(int64_t)c.slot * kPcBlk + lane] = s;
+}
+
+// a workgroup per heavy row
+__global__ __launch_bounds__(256) void k_pc_csr_heavy(int32_t m, const int32_t* __restrict__ hrow,
+                                                      const int32_t* __restrict__ hptr,
+                                                      const PcState* __restrict__ st,
+                                                      const double* __restrict__ part, double* __restrict__ g) {
     __shared__ double red[kB];
-    const int32_t col = *colp;
+    const int t = threadIdx.x, c = t & (kPcBlk - 1);
+    if (st->stop) return;
+    double acc = 0.0;
+#pragma unroll 4
+    for (int32_t q = hptr[blockIdx.x] + t / kPcBlk; q < hptr[blockIdx.x + 1]; q += kB / kPcBlk)
+        acc += part[(int64_t)q * kPcBlk + c];
+    red[t] = acc;
+    __syncthreads();
+    for (int w = kB / 2; w >= kPcBlk; w >>= 1) {
+        if (t < w) red[t] += red[t + w];
+        __syncthreads();
+    }
+    if (t < kPcBlk) g[(int64_t)t * m + hrow[blockIdx.x]] = red[t];
+}
+
+// wb[r][c] = D_r L(cand_c, r) for the finished columns r
+__global__ void k_pc_weights(int32_t m, const PcState* __restrict__ st, const double* __restrict__ D,
+                             const double* __restrict__ L, double* __restrict__ wb) {
+    const int32_t t = blockIdx.x * kB + threadIdx.x;
+    const int32_t r = t / kPcBlk, c = t % kPcBlk;
+    if (st->stop || r >= st->k0) return;
+    const int32_t row = st->cand[c];
+    wb[t] = row >= 0 ? D[r] * L[(int64_t)r * m + row] : 0.0;
+}
+
+// acc[c][q][j] = sum over r < k0 - k0 % 4, r = q (mod 4), of L(j,r) wb[r][c]:
+// every finished column read once for all candidates, 4 kPcBlk chains per row in
+// registers.  Bound by reading the factor.
+__global__ __launch_bounds__(256) void k_pc_block(int32_t m, const PcState* __restrict__ st,
+                                                  const int32_t* __restrict__ pos, const double* __restrict__ wb,
+                                                  const double* __restrict__ L, double* __restrict__ acc) {
+    const int32_t j = blockIdx.x * kB + threadIdx.x;
+    if (st->stop || j >= m) return;
+    const int32_t k0 = st->k0, kb = k0 & ~3;
+    if (pos[j] < k0) return;
+    double a[kPcBlk][4];
+#pragma unroll
+    for (int c = 0; c < kPcBlk; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[c][q] = 0.0;
+    double l[2][4];   // this group of four columns and the next one
+#pragma unroll
+    for (int q = 0; q < 4; ++q) l[0][q] = L[(int64_t)q * m + j];
+    for (int32_t r = 0; r < kb; r += 8) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int32_t rr = r + 4 * h;
+            if (rr >= kb) break;
+            const int32_t nx = min(rr + 4, kb - 4);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) l[h ^ 1][q] = L[(int64_t)(nx + q) * m + j];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int c = 0; c < kPcBlk; ++c) a[c][q] += l[h][q] * wb[(rr + q) * kPcBlk + c];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < kPcBlk; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[(int64_t)(4 * c + q) * m + j] = a[c][q];
+}
+
+// The next pivot: the best of np partials.  Out of candidates or done: the block
+// stops.  Else it is swapped to position k, w_r = D_r L(col, r) for r < k and
+// D_k = g(col) - sum_r w_r L(col, r).
+__global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t K, int32_t np, const PcBest* __restrict__ arg,
+                                                  PcState* __restrict__ st, int32_t* __restrict__ perm,
+                                                  int32_t* __restrict__ pos, const double* __restrict__ g,
+                                                  const double* __restrict__ L, double* __restrict__ D,
+                                                  double* __restrict__ w) {
+    __shared__ Best redb[kB];
+    __shared__ double red[kB];
+    if (st->stop) return;
+    const int32_t k = st->k;
+    Best mine = {-HUGE_VAL, INT_MAX, -1};
+    for (int i = threadIdx.x; i < np; i += kB) {
+        const Best c = arg[i];
+        if (c.row >= 0 && ahead(c, mine)) mine = c;
+    }
+    Best b = block_best(mine, redb);
+    // no row is ahead of none (every value left is NaN): the row at position k
+    const bool lost = b.row < 0 && k < K;
+    if (lost) b = {0.0, k, perm[k]};
+    int ci = -1;
+#pragma unroll
+    for (int c = 0; c < kPcBlk; ++c)
+        if (k < K && st->cand[c] == b.row) ci = c;
+    __syncthreads();   // every thread has read the state
+    if (ci < 0) {
+        if (threadIdx.x == 0) {
+            st->stop = 1;
+            if (lost) st->force = b.row;
+        }
+        return;
+    }
+    const int32_t col = b.row;
+    if (threadIdx.x == 0) {
+        const int32_t a = perm[k];
+        perm[k] = col;
+        perm[b.pos] = a;
+        pos[a] = b.pos;
+        pos[col] = k;
+        st->col = col;
+        st->ci = ci;
+        st->k = k + 1;
+    }
     double acc = 0.0;
     for (int32_t r = threadIdx.x; r < k; r += kB) {
         const double l = L[(int64_t)r * m + col];
@@ -246,38 +477,49 @@ __global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t k, const in
         acc += wr * l;
     }
     const double s = block_sum(acc, red);
-    if (threadIdx.x == 0) D[k] = (g[col] + delta) - s;
+    if (threadIdx.x == 0) D[k] = g[(int64_t)ci * m + col] - s;
 }
 
 // column k of L over all rows: 1 at the pivot, 0 at earlier pivots, else
-// (g_j - sum_r L(j,r) w_r) / D_k; the Schur diagonal loses D_k L(j,k)^2
-__global__ __launch_bounds__(256) void k_pc_column(int32_t m, int32_t k, const int32_t* __restrict__ colp,
+// (g_j - sum_r L(j,r) w_r) / D_k; the Schur diagonal loses D_k L(j,k)^2; the
+// best row left of every block
+__global__ __launch_bounds__(256) void k_pc_column(int32_t m, const PcState* __restrict__ st,
                                                    const int32_t* __restrict__ pos, const double* __restrict__ g,
-                                                   const double* __restrict__ wg, const double* __restrict__ D,
-                                                   double* __restrict__ L, double* __restrict__ S) {
-    __shared__ double w[kPcgMaxK];
-    for (int r = threadIdx.x; r < k; r += kB) w[r] = wg[r];
-    __syncthreads();
-    const int32_t j = blockIdx.x * kB + threadIdx.x;
-    if (j >= m) return;
-    const int32_t col = *colp;
-    double* Lk = L + (int64_t)k * m;
-    if (j == col) { Lk[j] = 1.0; return; }
-    if (pos[j] < k) { Lk[j] = 0.0; return; }
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    int32_t r = 0;
-    for (; r + 3 < k; r += 4) {
-        a0 += L[(int64_t)r * m + j] * w[r];
-        a1 += L[(int64_t)(r + 1) * m + j] * w[r + 1];
-        a2 += L[(int64_t)(r + 2) * m + j] * w[r + 2];
-        a3 += L[(int64_t)(r + 3) * m + j] * w[r + 3];
-    }
-    for (; r < k; ++r) a0 += L[(int64_t)r * m + j] * w[r];
-    const double u = g[j] - ((a0 + a1) + (a2 + a3));
+                                                   const double* __restrict__ accs, const double* __restrict__ wg,
+                                                   const double* __restrict__ D, double* __restrict__ L,
+                                                   float* __restrict__ L32, int64_t ld32, double* __restrict__ S,
+                                                   PcBest* __restrict__ arg) {
+    __shared__ Best red[kB];
+    if (st->stop) return;
+    const int32_t k = st->k - 1, kb = st->k0 & ~3, col = st->col, ci = st->ci;
     const double dk = D[k];
-    const double l = u / dk;
-    Lk[j] = l;
-    S[j] -= dk * l * l;
+    Best best = {-HUGE_VAL, INT_MAX, -1};
+    for (int64_t j = (int64_t)blockIdx.x * kB + threadIdx.x; j < m; j += (int64_t)gridDim.x * kB) {
+        double l = 0.0;
+        const int32_t pj = pos[j];
+        if (j == col) {
+            l = 1.0;
+        } else if (pj >= k) {
+            double a[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = accs[(int64_t)(4 * ci + q) * m + j];
+            int32_t r = kb;
+            for (; r + 3 < k; r += 4)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) a[q] += L[(int64_t)(r + q) * m + j] * wg[r + q];
+            for (; r < k; ++r) a[0] += L[(int64_t)r * m + j] * wg[r];
+            const double u = g[(int64_t)ci * m + j] - ((a[0] + a[1]) + (a[2] + a[3]));
+            l = u / dk;
+            const double sj = S[j] - dk * l * l;
+            S[j] = sj;
+            const Best c = {sj, pj, (int32_t)j};
+            if (ahead(c, best)) best = c;
+        }
+        L[(int64_t)k * m + j] = l;
+        if (L32) L32[(int64_t)k * ld32 + j] = (float)l;
+    }
+    const Best b = block_best(best, red);
+    if (threadIdx.x == 0) arg[blockIdx.x] = b;
 }
 
 // L11 (row-major K x K, rows = pivots in order) and X = L11^-1 by columns:
@@ -326,11 +568,6 @@ __global__ void k_vdiv(int64_t n, const double* __restrict__ a, const double* __
                        double* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x;
     if (i < n) out[i] = a[i] / b[i];
-}
-
-__global__ void k_to_f32(int32_t m, const double* __restrict__ x, float* __restrict__ y, int64_t ld) {
-    const int32_t i = blockIdx.x * kB + threadIdx.x;
-    if (i < m) y[blockIdx.y * ld + i] = (float)x[(int64_t)blockIdx.y * m + i];
 }
 
 // ------------------------------------------------------ preconditioner apply
@@ -689,27 +926,29 @@ void launch_csc_t_scaled(int32_t n, const int64_t* colptr, const int32_t* rowind
     if (n > 0) help::launch_kernel(k_csc_ts, grid_for(n), kB, 0, st, n, colptr, rowind, val, dinv, x, t);
 }
 
-void launch_pc_argmax(int32_t m, int32_t k, const double* S, double* pval, int32_t* pidx, int32_t* perm,
-                      int32_t* pos, int32_t* col_out, hipStream_t st) {
-    const int nb = (int)std::min<int64_t>(kArgmaxBlocks, std::max<int64_t>(1, ((int64_t)m - k + kB - 1) / kB));
-    help::launch_kernel(k_pc_argmax_part, nb, kB, 0, st, m, k, perm, S, pval, pidx);
-    help::launch_kernel(k_pc_pick, 1, kB, 0, st, nb, k, pval, pidx, perm, pos, col_out);
-}
-
-void launch_pc_scatter(const int32_t* col, int32_t max_row_nnz, const int64_t* rowptr, const int32_t* colind,
-                       const double* val, const double* dinv, double* sc, bool clear, hipStream_t st) {
-    const int nb = (int)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)max_row_nnz + kB - 1) / kB));
-    help::launch_kernel(k_pc_scatter, nb, kB, 0, st, col, rowptr, colind, val, dinv, sc, clear ? 1 : 0);
-}
-
-void launch_pc_pivot(int32_t m, int32_t k, const int32_t* col, const double* g, const double* L, double delta,
-                     double* D, double* w, hipStream_t st) {
-    help::launch_kernel(k_pc_pivot, 1, kB, 0, st, m, k, col, g, L, delta, D, w);
-}
-
-void launch_pc_column(int32_t m, int32_t k, const int32_t* col, const int32_t* pos, const double* g,
-                      const double* w, const double* D, double* L, double* S, hipStream_t st) {
-    help::launch_kernel(k_pc_column, grid_for(m), kB, 0, st, m, k, col, pos, g, w, D, L, S);
+void launch_pc_block(const PcBuild& B, hipStream_t st) {
+    const int32_t m = B.rows.m, K = B.K;
+    const int nbt = (int)std::min<int64_t>(kTopBlocks, ((int64_t)m + kB - 1) / kB);
+    const int nbc = (int)std::min<int64_t>(kColumnBlocks, ((int64_t)m + kB - 1) / kB);
+    const RowSplitDev& rs = B.rows;
+    help::launch_kernel(k_pc_top_part, nbt, kB, 0, st, m, B.pos, B.S, B.state, B.top, B.arg);
+    help::launch_kernel(k_pc_top_pick, 1, kB, 0, st, nbt, K, B.top, B.state);
+    const int nbs = (int)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)B.max_row_nnz + kB - 1) / kB));
+    help::launch_kernel(k_pc_scatter, dim3(nbs, kPcBlk), kB, 0, st, B.state, B.rowptr, B.colind, B.val, B.dinv, B.sc, 0);
+    if (rs.nchunk)
+        help::launch_kernel(k_pc_csr_chunk, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, B.state, B.colind, B.val, B.sc, B.part);
+    if (rs.nmed)
+        help::launch_kernel(k_pc_csr_medium, (rs.nmed + 3) / 4, kB, 0, st, m, rs.nmed, rs.mrow, B.state, B.rowptr, B.colind, B.val, B.sc, B.g);
+    help::launch_kernel(k_pc_csr_light, grid_for((int64_t)m * kPcBlk), kB, 0, st, m, B.state, B.rowptr, B.colind, B.val, B.sc, B.g);
+    if (rs.nheavy)
+        help::launch_kernel(k_pc_csr_heavy, rs.nheavy, kB, 0, st, m, rs.hrow, rs.hptr, B.state, B.part, B.g);
+    help::launch_kernel(k_pc_scatter, dim3(nbs, kPcBlk), kB, 0, st, B.state, B.rowptr, B.colind, B.val, B.dinv, B.sc, 1);
+    help::launch_kernel(k_pc_weights, grid_for((int64_t)K * kPcBlk), kB, 0, st, m, B.state, B.D, B.L, B.wb);
+    help::launch_kernel(k_pc_block, grid_for(m), kB, 0, st, m, B.state, B.pos, B.wb, B.L, B.acc);
+    for (int s = 0; s < kPcBlk; ++s) {
+        help::launch_kernel(k_pc_pivot, 1, kB, 0, st, m, K, s == 0 ? nbt : nbc, B.arg, B.state, B.perm, B.pos, B.g, B.L, B.D, B.w);
+        help::launch_kernel(k_pc_column, nbc, kB, 0, st, m, B.state, B.pos, B.g, B.acc, B.w, B.D, B.L, B.L32, B.ld32, B.S, B.arg);
+    }
 }
 
 void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, double* L11, double* X,
@@ -721,10 +960,6 @@ void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, d
 
 void launch_vdiv(int64_t n, const double* a, const double* b, double* out, hipStream_t st) {
     if (n > 0) help::launch_kernel(k_vdiv, grid_for(n), kB, 0, st, n, a, b, out);
-}
-
-void launch_to_f32(int32_t m, int32_t K, const double* x, float* y, int64_t ld, hipStream_t st) {
-    if (m > 0 && K > 0) help::launch_kernel(k_to_f32, dim3(grid_for(m), K), kB, 0, st, m, x, y, ld);
 }
 
 // Columns per lane of the fused apply (16 groups of them): the factor's tile and

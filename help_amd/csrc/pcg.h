@@ -35,7 +35,7 @@ struct RowChunk {
 // of columns: the gathered part of x then stays in that XCD's L2.
 struct RowSplitDev {
     int32_t m = 0;
-    int32_t nchunk = 0, nheavy = 0, nmed = 0;
+    int32_t nchunk = 0, nheavy = 0, nmed = 0, nparts = 0;
     const int32_t* mrow = nullptr;   // medium rows
     const RowChunk* chunks = nullptr;
     const int32_t* hrow = nullptr;   // heavy rows
@@ -56,24 +56,41 @@ void launch_vdiv(int64_t n, const double* a, const double* b, double* out, hipSt
 void launch_csc_t_scaled(int32_t n, const int64_t* colptr, const int32_t* rowind, const double* val,
                          const double* dinv, const double* x, double* t, hipStream_t st);
 
-// ---- partial Cholesky build (one pivot per call sequence) ----
-constexpr int kArgmaxBlocks = 512;
-// picks the pivot of step k: the largest S over positions [k, m) (ties to
-// the lowest position), swaps it to position k, writes its row to col_out
-void launch_pc_argmax(int32_t m, int32_t k, const double* S, double* pval, int32_t* pidx,
-                      int32_t* perm, int32_t* pos, int32_t* col_out, hipStream_t st);
-void launch_pc_scatter(const int32_t* col, int32_t max_row_nnz, const int64_t* rowptr,
-                       const int32_t* colind, const double* val, const double* dinv, double* sc,
-                       bool clear, hipStream_t st);
-void launch_pc_pivot(int32_t m, int32_t k, const int32_t* col, const double* g, const double* L,
-                     double delta, double* D, double* w, hipStream_t st);
-void launch_pc_column(int32_t m, int32_t k, const int32_t* col, const int32_t* pos, const double* g,
-                      const double* w, const double* D, double* L, double* S, hipStream_t st);
+// ---- partial Cholesky build, kPcBlk pivots per call sequence ----
+constexpr int kPcBlk = 16;          // candidates (and most pivots) of a block
+constexpr int kTopBlocks = 512;
+constexpr int kColumnBlocks = 2048;
+struct PcState {
+    int32_t k;                      // pivots taken
+    int32_t k0;                     // ... when the block started
+    int32_t stop;                   // the block has ended
+    int32_t col, ci;                // the step's pivot row and its place among the candidates
+    int32_t force;                  // row to lead the next block's candidates, or -1
+    int32_t cand[kPcBlk];
+};
+struct PcBest {
+    double v;
+    int32_t pos, row;
+};
+struct PcBuild {
+    RowSplitDev rows;
+    const int64_t* rowptr;
+    const int32_t* colind;
+    const double *val, *dinv;
+    int32_t K, max_row_nnz;
+    int64_t ld32;
+    PcState* state;
+    PcBest *top, *arg;              // kTopBlocks * kPcBlk; max(kTopBlocks, kColumnBlocks)
+    int32_t *perm, *pos;
+    double *S, *D, *L, *w;
+    float* L32;                     // null: no FP32 copy
+    double *sc;                     // n * kPcBlk, zero between blocks
+    double *part;                   // partials of the heavy rows * kPcBlk
+    double *g, *acc, *wb;           // m * kPcBlk; 4 m kPcBlk; K * kPcBlk
+};
+void launch_pc_block(const PcBuild& B, hipStream_t st);
 void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, double* L11,
                    double* X, hipStream_t st);
-// y (columns of ld >= m floats) = x (columns of m)
-void launch_to_f32(int32_t m, int32_t K, const double* x, float* y, int64_t ld, hipStream_t st);
-
 // ---- preconditioner apply z = M^-1 r (PCG.cpp:183-196) ----
 // y1: scratch of 2 * kPcgMaxK doubles; ltpart: K * pc_apply_blocks(m, K)
 // doubles; the m x K factor L32 in FP32 or FP64 (T = float / double), columns

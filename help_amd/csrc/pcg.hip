@@ -6,6 +6,7 @@
 // with the preconditioner applied from the FP32 copy of the factor.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <string>
 
@@ -52,10 +53,14 @@ struct PcgState {
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
         if (hpin) (void)hipHostFree(hpin);
+        if (hstate) (void)hipHostFree(hstate);
     }
-    DBuf<double> L, D, S, w, g, sc, L11, X, y1, ltpart, pval;
+    DBuf<double> L, D, S, w, g, sc, acc, wb, bpart, L11, X, y1, ltpart;
     DBuf<float> L32;
-    DBuf<int32_t> perm, pos, col, pidx;
+    DBuf<int32_t> perm, pos;
+    DBuf<PcState> state;
+    DBuf<PcBest> top, arg;
+    PcState* hstate = nullptr;       // pinned
     DBuf<double> x, r, z, p, q, t;
     std::vector<int32_t> iota;
 };
@@ -82,17 +87,23 @@ void pcg_setup(help_gpu* h) {
     P->D.alloc(K);
     P->w.alloc(K);
     P->S.alloc(m);
-    P->g.alloc(m);
-    P->sc.alloc(n);
+    // the build's block of pivots: the candidates' vectors over the columns, the
+    // columns of A D^-1 A^T and their left-looking sums
+    P->sc.alloc((size_t)n * kPcBlk);
+    P->g.alloc((size_t)m * kPcBlk);
+    P->acc.alloc((size_t)m * kPcBlk * 4);
+    P->wb.alloc((size_t)K * kPcBlk);
+    P->bpart.alloc(std::max<size_t>(1, (size_t)h->rows.nparts * kPcBlk));
+    P->state.alloc(1);
+    P->top.alloc(kTopBlocks * kPcBlk);
+    P->arg.alloc(std::max(kTopBlocks, kColumnBlocks));
+    HIPCHK(hipHostMalloc((void**)&P->hstate, sizeof(PcState), hipHostMallocDefault));
     P->L11.alloc((size_t)K * K);
     P->X.alloc((size_t)K * K);
     P->y1.alloc(2 * kPcgMaxK);
     P->ltpart.alloc((size_t)K * std::max(pc_apply_blocks<float>(m, P->K), pc_apply_blocks<double>(m, P->K)));
-    P->pval.alloc(kArgmaxBlocks);
-    P->pidx.alloc(kArgmaxBlocks);
     P->perm.alloc(m);
     P->pos.alloc(m);
-    P->col.alloc(1);
     P->x.alloc(m); P->r.alloc(m); P->z.alloc(m); P->p.alloc(m); P->q.alloc(m);
     P->t.alloc(n);
     P->cg.alloc(kCgSlots);
@@ -101,7 +112,7 @@ void pcg_setup(help_gpu* h) {
     for (auto& e : P->ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     P->iota.resize(m);
     for (int32_t i = 0; i < m; ++i) P->iota[i] = i;
-    HIPCHK(hipMemsetAsync(P->sc.p, 0, sizeof(double) * n, st));
+    HIPCHK(hipMemsetAsync(P->sc.p, 0, sizeof(double) * n * kPcBlk, st));
     HIPCHK(hipStreamSynchronize(st));
 }
 
@@ -117,29 +128,41 @@ void pcg_renew(help_gpu* h) {
     launch_csr_split(h->rows, h->d_rowptr.p, h->d_colind.p, h->d_csrval.p, h->d_dinv.p, P->S.p, true, st);
     HIPCHK(hipMemcpyAsync(P->perm.p, P->iota.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(P->pos.p, P->iota.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice, st));
-    for (int32_t k = 0; k < K; ++k) {
-        launch_pc_argmax(m, k, P->S.p, P->pval.p, P->pidx.p, P->perm.p, P->pos.p, P->col.p, st);
-        // column of A D^-1 A^T at the pivot row: A (D^-1 a_col^T) (PCG.cpp:63-79)
-        launch_pc_scatter(P->col.p, h->max_row_nnz, h->d_rowptr.p, h->d_colind.p, h->d_csrval.p, h->d_dinv.p,
-                          P->sc.p, false, st);
-        launch_csr_split(h->rows, h->d_rowptr.p, h->d_colind.p, h->d_csrval.p, P->sc.p, P->g.p, false, st);
-        launch_pc_scatter(P->col.p, h->max_row_nnz, h->d_rowptr.p, h->d_colind.p, h->d_csrval.p, h->d_dinv.p,
-                          P->sc.p, true, st);
-        // left-looking update against the previous columns (PCG.cpp:85-102)
-        launch_pc_pivot(m, k, P->col.p, P->g.p, P->L.p, 0.0, P->D.p, P->w.p, st);
-        launch_pc_column(m, k, P->col.p, P->pos.p, P->g.p, P->w.p, P->D.p, P->L.p, P->S.p, st);
+    PcBuild B;
+    B.rows = h->rows;
+    B.rowptr = h->d_rowptr.p; B.colind = h->d_colind.p; B.val = h->d_csrval.p; B.dinv = h->d_dinv.p;
+    B.K = K; B.max_row_nnz = h->max_row_nnz; B.ld32 = P->ld32;
+    B.state = P->state.p; B.top = P->top.p; B.arg = P->arg.p;
+    B.perm = P->perm.p; B.pos = P->pos.p;
+    B.S = P->S.p; B.D = P->D.p; B.L = P->L.p; B.w = P->w.p; B.L32 = h->opts.pcg_fp32_precond ? P->L32.p : nullptr;
+    B.sc = P->sc.p; B.part = P->bpart.p; B.g = P->g.p; B.acc = P->acc.p; B.wb = P->wb.p;
+    std::memset(P->hstate, 0, sizeof(PcState));
+    P->hstate->force = -1;
+    HIPCHK(hipMemcpyAsync(P->state.p, P->hstate, sizeof(PcState), hipMemcpyHostToDevice, st));
+    // as many blocks as the pivots need if every candidate is taken; then, as
+    // long as pivots are missing, as many again as the rest needs.  A block
+    // takes at least one pivot, or names the row that leads the next one.
+    int32_t k = 0;
+    for (int64_t blocks = 0; k < K;) {
+        if (blocks > 2 * (int64_t)K + kPcBlk) throw HipError("partial Cholesky: no pivot taken", HELP_ERR_HIP);
+        for (int32_t b = 0; b < (K - k + kPcBlk - 1) / kPcBlk; ++b, ++blocks) launch_pc_block(B, st);
+        HIPCHK(hipMemcpyAsync(P->hstate, P->state.p, sizeof(PcState), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        k = P->hstate->k;
     }
     launch_pc_l11(m, K, P->perm.p, P->L.p, P->L11.p, P->X.p, st);
-    if (h->opts.pcg_fp32_precond) launch_to_f32(m, K, P->L.p, P->L32.p, P->ld32, st);
     HIPCHK(hipGetLastError());
 }
 
-// per pivot k: the product with A (12 nnz + 8 (n + m)), the left-looking
-// update reading k previous columns (8 m k) and writing one (8 m); the FP32
-// copy at the end (12 m K)
+// per block of kPcBlk pivots: A once (12 nnz) with kPcBlk vectors (8 (n + m)
+// each), the k finished columns once (8 m k) and the candidates' sums (32 m
+// each); per pivot its sums, the block's own columns (half of them on
+// average), the Schur diagonal and the new column in FP64 and FP32
 double pcg_build_bytes(const help_gpu* h) {
     const double nnz = (double)h->nnz, m = h->m, n = h->n, K = h->pcg ? h->pcg->K : 0;
-    return K * (12.0 * nnz + 8.0 * (n + m) + 8.0 * m) + 8.0 * m * K * (K - 1) / 2 + 12.0 * m * K;
+    const double blocks = K / kPcBlk;
+    return blocks * (12.0 * nnz + kPcBlk * (8.0 * (n + m) + 32.0 * m)) + 8.0 * m * K * blocks / 2 +
+           K * m * (32.0 + 8.0 + 4.0 * kPcBlk + 16.0 + 12.0);
 }
 
 // per iteration: A^T p scaled (12 nnz + 8 m + 16 n), A t (12 nnz + 8 n + 8 m),

@@ -60,6 +60,45 @@ def test_partial_cholesky_matches_oracle(name, maker, K):
     assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
 
 
+def _spread(inst, rng):
+    return np.exp(rng.uniform(-2, 2, inst.n) * np.log(10.0))
+
+
+def _shared_column(inst, rng):
+    """d so small on one column that its rows lead the Schur diagonal until the
+    first of them is taken: the others were candidates and fall behind"""
+    d = np.exp(rng.uniform(-0.5, 0.5, inst.n) * np.log(10.0))
+    d[3] = 1e-8
+    return d
+
+
+@pytest.mark.parametrize("name,maker,K,dfun", [
+    ("one pivot", lambda: instances.random_lp(300, 600, 4, seed=71), 1, _spread),
+    ("one block", lambda: instances.random_lp(300, 600, 4, seed=72), 16, _spread),
+    ("a block and one", lambda: instances.random_lp(300, 600, 4, seed=73), 17, _spread),
+    ("fewer rows than candidates", lambda: instances.random_lp(5, 9, 3, seed=74), 5, _spread),
+    ("ties", lambda: instances.mcf(side=6, commodities=2, pairs=3, seed=75), 40, lambda inst, rng: np.ones(inst.n)),
+    ("candidates that fall behind", lambda: instances.random_lp(400, 700, 12, seed=76), 37, _shared_column),
+    ("zipf-heavy-rows", lambda: instances.zipf(3000, 9000, 6, 1.1, seed=77), 50, _spread)])
+def test_partial_cholesky_blocks_match_oracle(name, maker, K, dfun):
+    """The build takes its pivots from blocks of 16 candidates: the greedy order
+    of the oracle all the same, and the factor within the bars of
+    test_partial_cholesky_matches_oracle."""
+    inst = maker()
+    d = dfun(inst, np.random.default_rng(5))
+    _flush(f"pcg factor blocks, {name}: m={inst.m} n={inst.n} K={K}")
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=K)
+    be.construct(inst)
+    be.renew(d)
+    perm, D, S, Lg = be.pcg_factor()
+    be.destruct()
+    operm, oD, oS, oL = _oracle_pchol(inst, d, K)
+    assert np.array_equal(perm, operm)
+    assert np.allclose(D, oD, rtol=1e-11, atol=0)
+    assert np.allclose(S, oS, rtol=1e-9, atol=1e-12 * np.abs(oS).max())
+    assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
+
+
 def test_pcg_solve_matches_dense():
     inst = instances.random_lp(400, 800, 4, seed=23)
     rng = np.random.default_rng(2)
