@@ -498,8 +498,8 @@ void build_schedules(help_gpu* h) {
                 push_tiles({s, 0, 0, k0, k1, c, mode}, nc, c, c, wg);
             }
         }
-        // FP64: one fused launch for the phase's panels when its workgroups
-        // (one per row block, 104 KB of LDS each) fit the chip at once
+        // one fused launch for the phase's panels when its workgroups (one per
+        // row block, 110 KB of LDS each in FP64) fit the chip at once
         const int32_t npa = (int32_t)h->panel.size() - pa;
         const bool fuse = npa <= kFusedPanelMax;
         Op op{OP_POTRF, po, (int32_t)h->potrf.size() - po, wp};
@@ -576,6 +576,13 @@ void build_schedules(help_gpu* h) {
                 h->fops.push_back({OP_XINV, xo, (int32_t)h->xtask.size() - xo, wx});
         }
     }
+    for (std::vector<PanelTask>* v : {&h->potrf, &h->panel, &h->trsm, &h->pcopy})
+        for (PanelTask& t : *v) {
+            t.n = ncol(t.s);
+            t.c = S.snrow[t.s];
+            t.loff = S.loff[t.s];
+            t.doff = h->dinvoff[t.s] + (int64_t)(t.b / kTile) * kTile * kTile;
+        }
     for (GemmTask& g : h->gemm) {
         g.n = ncol(g.s);
         g.c = S.snrow[g.s];
@@ -795,6 +802,7 @@ void setup_device_factor(help_gpu* h) {
         h->d_scale.alloc(h->m);
         h->d_L32.alloc(std::max<int64_t>(1, nl));
         h->d_Dinv32.alloc(std::max<int64_t>(1, nd));
+        if (!h->pcopy.empty()) h->d_Lstage32.alloc(std::max<int64_t>(1, nd));
         if (h->use_xinv) {
             h->d_X32.alloc(std::max<int64_t>(1, h->xoff[S.nsuper]));
             h->d_S32.alloc(std::max<int64_t>(1, h->xoff[S.nsuper]));
@@ -835,6 +843,11 @@ T* xinv_store(help_gpu* h) {
     return (T*)h->d_X64.p;
 }
 template <typename T>
+T* lstage_store(help_gpu* h) {
+    if (std::is_same<T, float>::value) return (T*)h->d_Lstage32.p;
+    return (T*)h->d_Lstage64.p;
+}
+template <typename T>
 T* uacc_store(help_gpu* h) {
     return (T*)h->d_Uaccbuf.p;
 }
@@ -862,8 +875,7 @@ void run_factor(help_gpu* h, T* L, T* U, T* Dinv) {
             side_used = true;
         }
         forked = side;
-        const bool fused = std::is_same<T, double>::value &&
-                           ((o.kind == OP_POTRF && o.xcount > 0) || (o.kind == OP_TRSM && o.fused));
+        const bool fused = (o.kind == OP_POTRF && o.xcount > 0) || (o.kind == OP_TRSM && o.fused);
         if (fused && o.kind == OP_TRSM) continue;   // done by the fused panel launch
         ProfScope ps(h, o.kind, fused ? o.work2 : o.work);
         switch (o.kind) {
@@ -876,16 +888,13 @@ void run_factor(help_gpu* h, T* L, T* U, T* Dinv) {
                 break;
             case OP_EA: launch_extend_add<T>(h->d_ea.p + o.off, o.count, h->d_earef.p, h->sym, L, U, o.depth, st); break;
             case OP_POTRF:
-                if constexpr (std::is_same<T, double>::value) {
-                    if (fused) {
-                        launch_panel_fp64(h->d_panel.p + o.xoff, o.xcount, h->sym, L, Dinv, h->d_Lstage64.p,
-                                          h->d_err.p, st);
-                        break;
-                    }
+                if (fused) {
+                    launch_panel<T>(h->d_panel.p + o.xoff, o.xcount, L, Dinv, lstage_store<T>(h), h->d_err.p, st);
+                    break;
                 }
-                launch_potrf_diag<T>(h->d_potrf.p + o.off, o.count, h->sym, L, Dinv, h->d_err.p, st);
+                launch_potrf_diag<T>(h->d_potrf.p + o.off, o.count, L, Dinv, h->d_err.p, st);
                 break;
-            case OP_TRSM: launch_trsm_rows<T>(h->d_trsm.p + o.off, o.count, h->sym, L, Dinv, st); break;
+            case OP_TRSM: launch_trsm_rows<T>(h->d_trsm.p + o.off, o.count, L, Dinv, st); break;
             case OP_GEMM:
                 launch_gemm<T>(h->d_gemm.p + o.off, o.count, h->d_gref.p, h->d_ginv.p, h->d_gtouch.p, L, U, uacc_store<T>(h), st);
                 break;
@@ -893,12 +902,10 @@ void run_factor(help_gpu* h, T* L, T* U, T* Dinv) {
             default: break;
         }
     }
-    if constexpr (std::is_same<T, double>::value) {
-        // the fused panels' L11 blocks into L (nothing reads them from L
-        // during the factorization)
-        if (!h->pcopy.empty())
-            launch_copy_diag_fp64(h->d_pcopy.p, (int32_t)h->pcopy.size(), h->sym, h->d_Lstage64.p, L, st);
-    }
+    // the fused panels' L11 blocks into L (nothing reads them from L during
+    // the factorization)
+    if (!h->pcopy.empty())
+        launch_copy_diag<T>(h->d_pcopy.p, (int32_t)h->pcopy.size(), lstage_store<T>(h), L, st);
     if (side_used) {
         HIPCHK(hipEventRecord(h->ev_side[1], h->st_side));
         HIPCHK(hipStreamWaitEvent(st, h->ev_side[1], 0));

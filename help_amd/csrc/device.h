@@ -85,6 +85,10 @@ struct PanelTask {
     int32_t s;
     int32_t b;            // first panel column
     int32_t rb;           // 0: write back the diagonal block; >=1: row block rb-1
+    // the front's sizes and storage offsets (filled when the schedule is built)
+    int32_t n = 0, c = 0;
+    int64_t loff = 0;
+    int64_t doff = 0;     // the block's offset in Dinv
 };
 
 // Extend-add task: add every child's update matrix into the columns
@@ -111,7 +115,7 @@ struct EaRef {
 };
 
 constexpr int kTile = 64;      // GEMM tile and panel width
-// most workgroups of a fused FP64 panel launch (one per CU: 104 KB of LDS)
+// most workgroups of a fused panel launch (FP64: one per CU, 110 KB of LDS)
 constexpr int kFusedPanelMax = 240;
 constexpr int kSmallRows = 256;
 constexpr int kSmallElems = 4032;  // panel elements of a small front; with the 64x65
@@ -181,21 +185,22 @@ void launch_extend_add(const EaTask* tasks, int32_t count, const EaRef* refs, De
 constexpr int kEaDeepRows = 2048;   // launches with a front this tall take 8 rows per lane in flight
 // factor the 64x64 diagonal block at column b and store its inverse
 template <typename T>
-void launch_potrf_diag(const PanelTask* tasks, int32_t count, DevSym sym, T* L, T* Dinv,
+void launch_potrf_diag(const PanelTask* tasks, int32_t count, T* L, T* Dinv,
                        int32_t* err, hipStream_t st);
-// FP64: the diagonal block and one row block per task (PanelTask.rb >= 1;
+// the diagonal block and one row block per task (PanelTask.rb >= 1;
 // rb = 0 for a panel with no rows below), each task factoring the block
 // redundantly; the task with rb <= 1 stores Dinv and L11, the latter into
 // Lstage (Dinv layout), because the other tasks of the launch may still be
 // reading the unfactored block from L
-void launch_panel_fp64(const PanelTask* tasks, int32_t count, DevSym sym, double* L, double* Dinv,
-                       double* Lstage, int32_t* err, hipStream_t st);
+template <typename T>
+void launch_panel(const PanelTask* tasks, int32_t count, T* L, T* Dinv, T* Lstage, int32_t* err,
+                  hipStream_t st);
 // L11 blocks (s, b) from Lstage into L
-void launch_copy_diag_fp64(const PanelTask* tasks, int32_t count, DevSym sym, const double* Lstage,
-                           double* L, hipStream_t st);
+template <typename T>
+void launch_copy_diag(const PanelTask* tasks, int32_t count, const T* Lstage, T* L, hipStream_t st);
 // panel rows below the diagonal block times the stored inverse (MFMA)
 template <typename T>
-void launch_trsm_rows(const PanelTask* tasks, int32_t count, DevSym sym, T* L, const T* Dinv,
+void launch_trsm_rows(const PanelTask* tasks, int32_t count, T* L, const T* Dinv,
                       hipStream_t st);
 template <typename T>
 void launch_gemm(const GemmTask* tasks, int32_t count, const GatherRef* grefs, const int32_t* ginv,

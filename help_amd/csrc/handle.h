@@ -66,7 +66,7 @@ struct Op {
     int32_t lds = 0;   // dynamic LDS elements per workgroup (small fronts)
     int32_t ntiny = 0; // solves: leading supernodes of the list solved one per wave
     int32_t xoff = 0, xcount = 0;   // solves: the level's wide-supernode block tasks;
-                                    // FP64 factor: the phase's fused panel tasks
+                                    // the factor: the phase's fused panel tasks
                                     // (POTRF; its TRSM op then has fused set)
     double work2 = 0;  // flops of the fused panel launch
     int32_t wave = 0;  // lanes per front or supernode of the one-wave forms (64 or 32):
@@ -160,6 +160,7 @@ struct help_gpu {
     // one buffer each for both precisions (FP32 uses its first half)
     DBuf<double> d_Ubuf, d_Uaccbuf;
     DBuf<double> d_Lstage64;   // L11 of the fused panels (Dinv layout) until the final copy
+    DBuf<float> d_Lstage32;
     // FP32 mode: symmetric diagonal scaling of the factored matrix
     std::vector<int32_t> slot_row;
     DBuf<int32_t> d_slot_row, d_slot_col;

@@ -14,10 +14,10 @@
 // Small fronts (c <= 256, c*n <= 7680): one workgroup per front does the
 // extend-add, the dense partial factorization in LDS, the diagonal-block
 // inverses and the update SYRK.
-// Large fronts: extend-add by column chunks, then for each 64-column panel a
-// two-wave diagonal-block Cholesky + inverse, the panel rows times the
-// inverse on MFMA, an MFMA GEMM on the trailing panel columns, and finally
-// one MFMA SYRK for U with the full inner dimension n.
+// Large fronts: extend-add by column chunks, then for each 64-column panel the
+// diagonal block's Cholesky + inverse and the panel rows times the inverse on
+// MFMA, an MFMA GEMM on the trailing panel columns, and finally one MFMA SYRK
+// for U with the full inner dimension n.
 #include <type_traits>
 
 #include "device.h"
@@ -423,225 +423,6 @@ __global__ __launch_bounds__(256) void k_extend_add(const EaTask* __restrict__ t
     }
 }
 
-// ------------------------------------ diagonal block Cholesky + inverse
-// Elimination with unit multipliers on the augmented block [A | I]: step j
-// stores m_ij = a_ij / d_j in place, updates the trailing lower part
-// (a_ik -= d_j m_ij m_kj) and applies the same row operation to the identity
-// (x_ik -= m_ij x_jk).  At the end A holds L_u (unit) and D, X holds L_u^-1,
-// so L = L_u D^1/2 and L^-1 = D^-1/2 L_u^-1.  The block is padded with the
-// identity to 64, which leaves the leading nb x nb results unchanged.
-template <typename T>
-__device__ void factor_invert_block(const T* __restrict__ src, int64_t lds, int32_t nb,
-                                    T* __restrict__ Ldst, T* __restrict__ Db, T* A, T* X,
-                                    int32_t* err) {
-    constexpr int ld = kTile + 1;
-    const int tid = threadIdx.x;
-    const int row = tid & 63, part = tid >> 6;
-    for (int idx = tid; idx < kTile * kTile; idx += 256) {
-        int j = idx >> 6, i = idx & 63;
-        T v = (i == j) ? T(1) : T(0);
-        if (i < nb && j < nb && i >= j) v = src[(int64_t)j * lds + i];
-        A[j * ld + i] = v;
-        X[j * ld + i] = (i == j) ? T(1) : T(0);
-    }
-    __syncthreads();
-    for (int j = 0; j < kTile; ++j) {
-        T piv = A[j * ld + j];
-        if (!(piv > T(0))) {
-            if (tid == 0 && j < nb) atomicAdd(err, 1);
-            piv = Huge<T>::v;
-        }
-        __syncthreads();
-        if (part == 0) {
-            if (row > j) A[j * ld + row] /= piv;
-            else if (row == j) A[j * ld + j] = piv;
-        }
-        __syncthreads();
-        if (row > j) {
-            const T mi = A[j * ld + row];
-            for (int k = part; k <= row; k += 4) {
-                if (k > j) A[k * ld + row] -= piv * mi * A[j * ld + k];
-                else X[k * ld + row] -= mi * X[k * ld + j];
-            }
-        }
-        __syncthreads();
-    }
-    for (int idx = tid; idx < kTile * kTile; idx += 256) {
-        int j = idx >> 6, i = idx & 63;
-        if (i >= nb || j >= nb) continue;
-        const T sdj = sqrt(A[j * ld + j]);
-        if (i >= j) Ldst[(int64_t)j * lds + i] = (i == j) ? sdj : A[j * ld + i] * sdj;
-        Db[j * nb + i] = (i >= j) ? X[j * ld + i] / sqrt(A[i * ld + i]) : T(0);
-    }
-}
-
-// Diagonal block of a panel: LDL^T of the nb x nb block (identity padding to
-// 64) with L11 = L_unit diag(sqrt(d)) written in place and its inverse
-// Dinv = diag(1/sqrt(d)) L_unit^-1 written to the block's Dinv slot.
-//
-// Two waves with 2D register blocking: lane (bi, bk) = (lane >> 3, lane & 7)
-// holds the 8x8 block of rows 8bi.. and columns 8bk.. .
-//  * Wave 0 factors.  Step j publishes column j of the Schur complement to
-//    LDS (the lanes of column block j/8 write it), every lane reads its 8
-//    row values and 8 column values and applies a -= (raw_r / d_j) raw_k to
-//    its whole block.  That is exact on the trailing matrix (r, k > j); the
-//    other entries it touches are never read again (finished columns are
-//    already published, rows above j only own upper-triangle entries), so
-//    the step needs no masks and no branches.  L11 is formed at the end from
-//    the published columns.
-//  * Wave 1 forms X = L_unit^-1 in the same layout: step j waits for wave 0
-//    to publish step j (LDS flag; wave 0 never waits), takes l_rj for its
-//    rows from the published column, and subtracts l_rj X[j][:] (row j of X
-//    is final at step j and published by its owners).
-// 8 steps are unrolled so every register index is static; the publishing
-// stores are branch-free (non-owner lanes write a dump row), and the output
-// stores are unconditional (elements outside nb x nb go to an LDS slot
-// through the generic address space).
-template <typename T>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void k_potrf_diag(const PanelTask* __restrict__ tasks, DevSym sym, T* __restrict__ L, T* __restrict__ Dinv,
-                  int32_t* __restrict__ err) {
-    constexpr int kS = kTile + 1;
-    __shared__ T S[kTile * kS];            // input staging, then X for the Dinv output
-    __shared__ T cbt[kTile * kTile];       // column j of the Schur complement at step j
-    __shared__ T rps[kTile], pivs[kTile], sdv[kTile];
-    __shared__ T xrow[kTile];
-    __shared__ T dump[2][kTile * 8];
-    __shared__ int flag;
-    const PanelTask tk = tasks[blockIdx.x];
-    const int32_t s = tk.s, b = tk.b;
-    const int32_t n = sym.sfirst[s + 1] - sym.sfirst[s];
-    const int32_t c = sym.snrow[s];
-    const int nb = min(kTile, n - b);
-    T* P = L + sym.loff[s] + (int64_t)b * c + b;
-    T* Db = Dinv + dinv_block_offset(sym, s, b);
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int bi = lane >> 3, bk = lane & 7;
-    {
-        // lower triangle, identity outside nb, zero above; clamped loads
-        const int r = lane, rr = min(r, nb - 1);
-        T v[kTile / 2];
-#pragma unroll
-        for (int t = 0; t < kTile / 2; ++t) {
-            const int k = w + 2 * t;
-            v[t] = P[(int64_t)min(k, nb - 1) * c + rr];
-        }
-#pragma unroll
-        for (int t = 0; t < kTile / 2; ++t) {
-            const int k = w + 2 * t;
-            S[k * kS + r] = (r < nb && k < nb) ? ((r >= k) ? v[t] : T(0)) : ((r == k) ? T(1) : T(0));
-        }
-        if (tid == 0) flag = 0;
-    }
-    __syncthreads();
-    if (w == 0) {
-        T a[8][8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int v = 0; v < 8; ++v) a[u][v] = S[(8 * bk + v) * kS + 8 * bi + u];
-        int nbad = 0;
-        for (int jb = 0; jb < 8; ++jb) {
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const int j = 8 * jb + jj;
-                T* col = cbt + j * kTile;
-                T* dst = (bk == jb) ? col + 8 * bi : dump[0] + 8 * lane;
-#pragma unroll
-                for (int u = 0; u < 8; ++u) dst[u] = a[u][jj];
-                wave_sync();
-                T piv = col[j];
-                T raw[8], cc[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) raw[u] = col[8 * bi + u];
-#pragma unroll
-                for (int v = 0; v < 8; ++v) cc[v] = col[8 * bk + v];
-                const bool bad = !(piv > T(0));
-                nbad += (bad && j < nb) ? 1 : 0;
-                piv = bad ? Huge<T>::v : piv;
-                const T rp = T(1) / piv;
-                T m[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) m[u] = raw[u] * rp;
-                // the next column first: it is published at the next step
-                if (jj < 7) {
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) a[u][jj + 1] -= m[u] * cc[jj + 1];
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-#pragma unroll
-                    for (int v = 0; v < 8; ++v)
-                        if (v != jj + 1) a[u][v] -= m[u] * cc[v];
-                rps[j] = rp;
-                pivs[j] = piv;
-                __hip_atomic_store(&flag, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-        }
-        if (lane == 0 && nbad) atomicAdd(err, nbad);
-        // L11[r][k] = l_rk sqrt(d_k) = raw_r(step k) / d_k * sqrt(d_k)
-        const int r = lane;
-        sdv[r] = sqrt(pivs[r]);
-        wave_sync();
-        T* trash = dump[0] + lane;
-#pragma unroll
-        for (int k = 0; k < kTile; ++k) {
-            const T sk = sdv[k];
-            const T f = (r > k) ? rps[k] * sk : T(0);
-            T v = cbt[k * kTile + r] * f;
-            v = (r == k) ? sk : v;
-            T* dst = (r < nb && k < nb) ? P + (int64_t)k * c + r : trash;
-            *dst = v;
-        }
-    } else {
-        T x[8][8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int v = 0; v < 8; ++v) x[u][v] = (8 * bi + u == 8 * bk + v) ? T(1) : T(0);
-        for (int jb = 0; jb < 8; ++jb) {
-            const bool lo = bi > jb, hi = bi >= jb;    // row 8bi+u > j for u <= jj / u > jj
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const int j = 8 * jb + jj;
-                T* dx = (bi == jb) ? xrow + 8 * bk : dump[1] + 8 * lane;
-#pragma unroll
-                for (int v = 0; v < 8; ++v) dx[v] = x[jj][v];
-                while (__hip_atomic_load(&flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <= j)
-                    __builtin_amdgcn_s_sleep(1);
-                const T rp = rps[j];
-                T m[8], xr[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const T mv = cbt[j * kTile + 8 * bi + u] * rp;
-                    m[u] = ((u > jj) ? hi : lo) ? mv : T(0);
-                }
-#pragma unroll
-                for (int v = 0; v < 8; ++v) xr[v] = xrow[8 * bk + v];
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-#pragma unroll
-                    for (int v = 0; v < 8; ++v) x[u][v] -= m[u] * xr[v];
-                wave_sync();
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int v = 0; v < 8; ++v) S[(8 * bk + v) * kS + 8 * bi + u] = x[u][v];
-        wave_sync();
-        const int r = lane;
-        const T isd = T(1) / sqrt(pivs[r]);
-        T* trash = dump[1] + lane;
-#pragma unroll
-        for (int k = 0; k < kTile; ++k) {
-            const T v = S[k * kS + r] * ((r >= k) ? isd : T(0));
-            T* dst = (r < nb && k < nb) ? Db + k * nb + r : trash;
-            *dst = v;
-        }
-    }
-}
-
 // ------------------------------------------------------------- MFMA GEMM
 // 4 waves, each a 32x32 quarter of a 64x64 tile built from 2x2 MFMA 16x16x4
 // blocks.  Lane layout (measured on gfx950 by help_selftest_mfma): A[i][k] in
@@ -687,65 +468,77 @@ __device__ inline void mfma_tile(const T* As, const T* Bs, int kc, int lane, int
 }
 
 // ------------------------- diagonal block, blocked form with MFMA updates
-// Same result as k_potrf_diag (L11 = L_unit diag(sqrt(d)) in place, Dinv =
-// diag(1/sqrt(d)) L_unit^-1), LDL^T by 4-column panels.  The 64x64 block and
-// X = L_unit^-1 live in MFMA accumulator layout: wave w holds the 16x16
-// tiles (w, 0..3) of each.  Block step kb, panel owner wave ow = kb/4:
-//  * wave ow reads column block kb from S with the rows on the lanes and
-//    factors it: pivot and in-panel values come from other lanes by
-//    readlane, the multipliers m = a/d go to Mn (negated) and the unscaled
-//    columns to Uf.  It then finishes the panel's 4 rows of X: they leave
-//    its accumulators through XR, take the unit-lower 4x4 substitution with
-//    the columns on the lanes, and go to XF (final, column-major) and back
-//    to XR;
-//  * barrier; every tile row below the panel applies A -= m U^T and
-//    X -= m XR as one V_MFMA_F64_16X16X4_F64 per live tile (K = the 4 panel
-//    columns) and stores its part of column block kb+1 to S; barrier.
-// Two barriers per 4 pivots instead of per-pivot publishing, and the
-// trailing updates run on the matrix cores.
+// Diagonal block of a panel: LDL^T of the nb x nb block (identity padding to
+// 64) by 4-column panels with L11 = L_unit diag(sqrt(d)) written in place and
+// its inverse Dinv = diag(1/sqrt(d)) X, X = L_unit^-1, written to the block's
+// Dinv slot.  The 64x64 block and X live in MFMA accumulator layout: wave
+// w < 4 holds the 16x16 tiles (w, 0..3) of each; wave 4 factors the panels.
+// Step kb, between two barriers each:
+//  * wave 4 reads column block kb from S with the rows on the lanes and
+//    factors it: pivot and in-panel values come from other lanes by readlane,
+//    the multipliers m = a/d go to Mn (negated) and the unscaled columns to Uf.
+//    Meanwhile waves 0 to 3 apply step kb-1 to the column tiles that the next
+//    panel is not in, A -= m U^T, one MFMA per live tile (K = the 4 panel
+//    columns), and step kb-2 to X (first); then the wave that owns rows 4(kb-1).. of X
+//    finishes them: they leave its accumulators through XR, take the
+//    unit-lower 4x4 substitution with the columns on the lanes, and go to XF
+//    (final, column-major) and back to XR;
+//  * waves 0 to 3 apply step kb to the one column tile that panel kb+1 is in
+//    and store that panel's columns to S.
+// The dependent chain is a panel's 4 pivots, one MFMA and two barriers per
+// step; X and the other tiles run beside it.  Every accumulator takes its
+// terms in the order of kb.
 // kTrsm: the task also carries row block rb - 1 below the diagonal block
 // (every task of a panel factors the block redundantly; the task with
 // rb <= 1 writes L11, Dinv and the pivot count).  Its 64 rows are loaded
 // before the factorization and solved at the end as k_trsm_gemm does,
 // X * Dinv^T on MFMA with Dinv taken from LDS: the same products and
 // order, so the same values, without a launch of its own.
+// Bound by the chain.  A launch of 120 tasks with the row block: FP64 20.7 us
+// (31.3 us when the owner of the next panel's rows applied all its updates
+// before factoring it and the row block was staged at the end), FP32 19.9 us
+// (26.3 us plus a launch of k_trsm_gemm when two waves passed single columns
+// through LDS).
 __device__ inline double read_lane(double v, int l) {
     const long long b = __builtin_bit_cast(long long, v);
     const int lo = __builtin_amdgcn_readlane((int)b, l);
     const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
 }
+__device__ inline float read_lane(float v, int l) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
 
-template <bool kTrsm>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void k_potrf_mfma(const PanelTask* __restrict__ tasks, DevSym sym, double* __restrict__ L,
-                  double* __restrict__ Dinv, double* __restrict__ Lstage, int32_t* __restrict__ err) {
-    typedef double T;
-    typedef Mfma<double>::acc_t acc_t;
+template <typename T, bool kTrsm>
+__global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_potrf_mfma(const PanelTask* __restrict__ tasks, T* __restrict__ L,
+                  T* __restrict__ Dinv, T* __restrict__ Lstage, int32_t* __restrict__ err) {
+    typedef typename Mfma<T>::acc_t acc_t;
     constexpr int kS = kTile + 1;
     __shared__ T S[kTile * kS];
     __shared__ T Uf[kTile * kTile];        // column j before scaling (step j), Uf[j*64 + r]
     __shared__ T XF[kTile * kTile];        // final X, column-major
-    __shared__ T Mn[kTile * 4];            // -m of the current panel, Mn[r*4 + jj]
-    __shared__ T XR[4 * kTile];            // the current panel's rows of X
-    __shared__ T rps[kTile], pivs[kTile], sdv[kTile];
+    __shared__ T Mn[3][kTile * 4];         // -m of panel kb in Mn[kb % 3], [r*4 + jj]
+    __shared__ T XR[2][4 * kTile];         // panel kb's rows of X in XR[kb % 2]
+    __shared__ T rps[kTile], pivs[kTile], sdv[kTile], isdv[kTile];
+    __shared__ T As[kTrsm ? kTile * kTile : 1];   // the row block, As[k*64 + i]
     const PanelTask tk = tasks[blockIdx.x];
-    const int32_t s = tk.s, b = tk.b;
-    const int32_t n = sym.sfirst[s + 1] - sym.sfirst[s];
-    const int32_t c = sym.snrow[s];
+    const int32_t b = tk.b, n = tk.n, c = tk.c;
     const int nb = min(kTile, n - b);
-    T* P = L + sym.loff[s] + (int64_t)b * c + b;
-    T* Db = Dinv + dinv_block_offset(sym, s, b);
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    T* P = L + tk.loff + (int64_t)b * c + b;
+    T* Db = Dinv + tk.doff;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const bool upd = wave < 4;
     const int lc = lane & 15, lk = lane >> 4;
     const bool owner = !kTrsm || tk.rb <= 1;
     const bool rows = kTrsm && tk.rb >= 1;
     const int32_t r0 = b + nb + (tk.rb - 1) * kTile;
-    T* Lp = L + sym.loff[s];
+    T* Lp = L + tk.loff;
     // the row block's entries (as k_trsm_gemm loads them), in flight
     // during the factorization
     T va[kTile * kTile / 256];
-    if (rows) {
+    if (rows && upd) {
         const int32_t ri = min(r0 + lane, c - 1);
 #pragma unroll
         for (int q = 0; q < kTile * kTile / 256; ++q) {
@@ -753,7 +546,7 @@ void k_potrf_mfma(const PanelTask* __restrict__ tasks, DevSym sym, double* __res
             va[q] = Lp[(int64_t)(b + kc) * c + ri];
         }
     }
-    {
+    if (upd) {
         // lower triangle, identity outside nb, zero above; clamped loads
         const int r = lane, rr = min(r, nb - 1);
         T v[16];
@@ -768,152 +561,216 @@ void k_potrf_mfma(const PanelTask* __restrict__ tasks, DevSym sym, double* __res
             S[k * kS + r] = (r < nb && k < nb) ? ((r >= k) ? v[q] : T(0)) : ((r == k) ? T(1) : T(0));
         }
     }
+    if (rows && upd) {
+#pragma unroll
+        for (int q = 0; q < kTile * kTile / 256; ++q) {
+            const int k = wave + 4 * q;
+            As[k * kTile + lane] = (k < nb && r0 + lane < c) ? va[q] : T(0);
+        }
+    }
     __syncthreads();
     acc_t acc[4], xacc[4];
+    if (upd) {
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
+        for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 16 * wave + Mfma<double>::row(lane, r), col = 16 * tj + lc;
-            acc[tj][r] = S[col * kS + row];
-            xacc[tj][r] = (row == col) ? T(1) : T(0);
-        }
-    int nbad = 0;
-    for (int kb = 0; kb < 16; ++kb) {
-        if (wave == (kb >> 2)) {
-            T p[4];
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) p[jj] = S[(4 * kb + jj) * kS + lane];
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                const int j = 4 * kb + jj;
-                T d = read_lane(p[jj], j);
-                T akj[4];
-#pragma unroll
-                for (int kk = jj + 1; kk < 4; ++kk) akj[kk] = read_lane(p[jj], 4 * kb + kk);
-                const bool bad = !(d > T(0));
-                nbad += (bad && j < nb) ? 1 : 0;
-                d = bad ? Huge<T>::v : d;
-                const T rp = T(1) / d;
-                const T m = p[jj] * rp;
-                Uf[j * kTile + lane] = p[jj];
-                Mn[lane * 4 + jj] = -m;
-#pragma unroll
-                for (int kk = jj + 1; kk < 4; ++kk) p[kk] -= m * akj[kk];
-                if (lane == 0) { rps[j] = rp; pivs[j] = d; }
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * wave + Mfma<T>::row(lane, r), col = 16 * tj + lc;
+                acc[tj][r] = S[col * kS + row];
+                xacc[tj][r] = (row == col) ? T(1) : T(0);
             }
-            // the panel's rows of X (rows 4(kb%4).. of this wave's tiles)
+    }
+    int nbad = 0;
+    // A -= m U^T of step kb on column tile tj
+    auto apply_a = [&](int kb, int tj, T aop) {
+        const T bop = Uf[(4 * kb + lk) * kTile + 16 * tj + lc];
+        acc[tj] = Mfma<T>::fma(aop, bop, acc[tj]);
+    };
+    // X -= m XR of step kb
+    auto apply_x = [&](int kb) {
+        if (16 * wave + 15 < 4 * kb + 4) return;
+        const T xop = (16 * wave + lc > 4 * kb + 3) ? Mn[kb % 3][(16 * wave + lc) * 4 + lk] : T(0);
 #pragma unroll
-            for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = Mfma<double>::row(lane, r);
-                    if ((row >> 2) == (kb & 3)) XR[(row & 3) * kTile + 16 * tj + lc] = xacc[tj][r];
-                }
-            wave_sync();
-            T xs[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) xs[u] = XR[u * kTile + lane];
+        for (int tj = 0; tj < 4; ++tj)
+            if (tj <= wave && 16 * tj <= 4 * kb + 3)   // nonzero part of X (uniform)
+                xacc[tj] = Mfma<T>::fma(xop, XR[kb & 1][lk * kTile + 16 * tj + lc], xacc[tj]);
+    };
+    // rows 4 kb .. 4 kb + 3 of X
+    auto finish_x = [&](int kb) {
+        if (wave != (kb >> 2)) return;
+        T* xr = XR[kb & 1];
+        const T* mn = Mn[kb % 3];
+        if constexpr (sizeof(T) == 4) {
+            // FP32: a lane holds the four rows of a column
+            T m[4][4];
 #pragma unroll
             for (int u = 1; u < 4; ++u)
 #pragma unroll
-                for (int up = 0; up < u; ++up) xs[u] += Mn[(4 * kb + u) * 4 + up] * xs[up];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                XR[u * kTile + lane] = xs[u];
-                XF[lane * kTile + 4 * kb + u] = xs[u];
-            }
-        }
-        __syncthreads();
-        if (16 * wave + 15 >= 4 * kb + 4) {
-            const T aop = Mn[(16 * wave + lc) * 4 + lk];
-            const T xop = (16 * wave + lc > 4 * kb + 3) ? aop : T(0);
+                for (int up = 0; up < u; ++up) m[u][up] = mn[(4 * kb + u) * 4 + up];
+            if (lk != (kb & 3)) return;
 #pragma unroll
             for (int tj = 0; tj < 4; ++tj) {
-                if (16 * tj + 15 >= 4 * kb + 4) {          // live columns (uniform)
-                    const T bop = Uf[(4 * kb + lk) * kTile + 16 * tj + lc];
-                    acc[tj] = Mfma<double>::fma(aop, bop, acc[tj]);
+                T xs[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    xs[u] = xacc[tj][u];
+#pragma unroll
+                    for (int up = 0; up < u; ++up) xs[u] += m[u][up] * xs[up];
                 }
-                if (tj <= wave && 16 * tj <= 4 * kb + 3) {  // nonzero part of X (uniform)
-                    const T bx = XR[lk * kTile + 16 * tj + lc];
-                    xacc[tj] = Mfma<double>::fma(xop, bx, xacc[tj]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    xr[u * kTile + 16 * tj + lc] = xs[u];
+                    XF[(16 * tj + lc) * kTile + 4 * kb + u] = xs[u];
                 }
             }
-            if (kb + 1 < 16) {
-                const int tj1 = (kb + 1) >> 2, jc = 4 * ((kb + 1) & 3);
-                if (lc >= jc && lc < jc + 4) {
+            return;
+        }
 #pragma unroll
-                    for (int tj = 0; tj < 4; ++tj)
-                        if (tj == tj1)
+        for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                S[(16 * tj + lc) * kS + 16 * wave + Mfma<double>::row(lane, r)] = acc[tj][r];
+            for (int r = 0; r < 4; ++r) {
+                const int row = Mfma<T>::row(lane, r);
+                if ((row >> 2) == (kb & 3)) xr[(row & 3) * kTile + 16 * tj + lc] = xacc[tj][r];
+            }
+        wave_sync();
+        T xs[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xs[u] = xr[u * kTile + lane];
+#pragma unroll
+        for (int u = 1; u < 4; ++u)
+#pragma unroll
+            for (int up = 0; up < u; ++up) xs[u] += mn[(4 * kb + u) * 4 + up] * xs[up];
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            xr[u * kTile + lane] = xs[u];
+            XF[lane * kTile + 4 * kb + u] = xs[u];
+        }
+    };
+    for (int kb = 0; kb <= 16; ++kb) {
+        if (!upd) {
+            if (kb < 16) {
+                T p[4];
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) p[jj] = S[(4 * kb + jj) * kS + lane];
+                T* mn = Mn[kb % 3];
+#pragma unroll
+                for (int jj = 0; jj < 4; ++jj) {
+                    const int j = 4 * kb + jj;
+                    T d = read_lane(p[jj], j);
+                    T akj[4];
+#pragma unroll
+                    for (int kk = jj + 1; kk < 4; ++kk) akj[kk] = read_lane(p[jj], 4 * kb + kk);
+                    const bool bad = !(d > T(0));
+                    nbad += (bad && j < nb) ? 1 : 0;
+                    d = bad ? Huge<T>::v : d;
+                    const T rp = T(1) / d;
+                    const T m = p[jj] * rp;
+#pragma unroll
+                    for (int kk = jj + 1; kk < 4; ++kk) p[kk] -= m * akj[kk];
+                    Uf[j * kTile + lane] = p[jj];
+                    mn[lane * 4 + jj] = -m;
+                    if (lane == 0) { rps[j] = rp; pivs[j] = d; }
                 }
             }
+        } else {
+            if (kb >= 2) apply_x(kb - 2);
+            if (kb >= 1 && kb < 16 && 16 * wave + 15 >= 4 * kb) {   // the rest of step kb - 1
+                const T aop = Mn[(kb - 1) % 3][(16 * wave + lc) * 4 + lk];
+#pragma unroll
+                for (int tj = 0; tj < 4; ++tj)
+                    if (tj != (kb >> 2) && 16 * tj + 15 >= 4 * kb) apply_a(kb - 1, tj, aop);
+            }
+            if (kb >= 1) finish_x(kb - 1);
+        }
+        __syncthreads();
+        if (kb >= 15) continue;   // (after the last panel only X is left)
+        if (upd && 16 * wave + 15 >= 4 * kb + 4) {
+            const T aop = Mn[kb % 3][(16 * wave + lc) * 4 + lk];
+            const int tj1 = (kb + 1) >> 2, jc = 4 * ((kb + 1) & 3);
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj)
+                if (tj == tj1) {
+                    apply_a(kb, tj, aop);
+                    if (lc >= jc && lc < jc + 4) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            S[(16 * tj + lc) * kS + 16 * wave + Mfma<T>::row(lane, r)] = acc[tj][r];
+                    }
+                }
         }
         __syncthreads();
     }
-    if (owner && t == 0 && nbad) atomicAdd(err, nbad);
-    if (t < kTile) sdv[t] = sqrt(pivs[t]);
+    if (owner && t == 256 && nbad) atomicAdd(err, nbad);
+    // (all at once: taken per step beside the panels they lengthened every step)
+    if (t < kTile) {
+        const T sd = sqrt(pivs[t]);
+        sdv[t] = sd;
+        isdv[t] = T(1) / sd;
+    }
     __syncthreads();
+    if (!upd) return;
     // L11[r][k] = raw_r(step k) / d_k * sqrt(d_k); Dinv[r][k] = X[r][k] / sqrt(d_r)
-    const int r = lane;
-    const T isd = T(1) / sdv[r];
+    if (owner) {
+        const int r = lane;
+        const T isd = isdv[r];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int k = wave + 4 * q;
-        const T sk = sdv[k];
-        const T f = (r > k) ? rps[k] * sk : T(0);
-        T v = Uf[k * kTile + r] * f;
-        v = (r == k) ? sk : v;
-        if (kTrsm) {
-            if (owner && r < nb && k < nb) Lstage[dinv_block_offset(sym, s, b) + k * nb + r] = v;
-        } else {
-            if (r < nb && k < nb) P[(int64_t)k * c + r] = v;
-        }
-        const T xv = XF[k * kTile + r] * ((r >= k) ? isd : T(0));
-        if (owner && r < nb && k < nb) Db[k * nb + r] = xv;
-    }
-    if (!rows) return;   // uniform over the workgroup
-    // row block: As[k][i] = X[i][k] in S's storage, Bs[k][j] = Dinv[j][k]
-    // (the values just written to Db) in Uf's storage
-    __syncthreads();
-    T* As = S;
-    T* Bs = Uf;
-#pragma unroll
-    for (int q = 0; q < kTile * kTile / 256; ++q) {
-        const int k = wave + 4 * q;
-        As[k * kTile + lane] = (k < nb && r0 + lane < c) ? va[q] : T(0);
-        const T xv = XF[k * kTile + r] * ((r >= k) ? isd : T(0));
-        Bs[k * kTile + lane] = (k < nb && lane < nb) ? xv : T(0);
-    }
-    __syncthreads();
-    acc_t tacc[2][2];
-    for (int a = 0; a < 2; ++a)
-        for (int q = 0; q < 2; ++q) tacc[a][q] = acc_t{0, 0, 0, 0};
-    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-    mfma_tile<T>(As, Bs, kTile, lane, wr, wc, tacc);
-    for (int a = 0; a < 2; ++a)
-        for (int q = 0; q < 2; ++q)
-            for (int rr = 0; rr < 4; ++rr) {
-                const int32_t i = wr + a * 16 + Mfma<T>::row(lane, rr);
-                const int32_t j = wc + q * 16 + (lane & 15);
-                if (r0 + i >= c || j >= nb) continue;
-                Lp[(int64_t)(b + j) * c + r0 + i] = tacc[a][q][rr];
+        for (int q = 0; q < 16; ++q) {
+            const int k = wave + 4 * q;
+            const T sk = sdv[k];
+            const T f = (r > k) ? rps[k] * sk : T(0);
+            T v = Uf[k * kTile + r] * f;
+            v = (r == k) ? sk : v;
+            if (r < nb && k < nb) {
+                if (kTrsm) Lstage[tk.doff + k * nb + r] = v;
+                else P[(int64_t)k * c + r] = v;
+                Db[k * nb + r] = XF[k * kTile + r] * ((r >= k) ? isd : T(0));
             }
+        }
+    }
+    if (!rows) return;
+    // the row block times Dinv^T, as D[j][i] = sum_k Dinv[j][k] X[i][k]: wave w
+    // takes rows i = 16 w .. of the block, so a lane stores 16 consecutive
+    // rows' neighbours; Dinv comes from XF as it was stored, and only its
+    // lower part (k <= j) enters
+    acc_t tacc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) tacc[q] = acc_t{0, 0, 0, 0};
+    T isd4[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) isd4[q] = isdv[16 * q + lc];
+#pragma unroll
+    for (int kk = 0; kk < kTile; kk += 4) {
+        const int kr = kk + lk;
+        const T x = As[kr * kTile + 16 * wave + lc];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (kk < 16 * (q + 1)) {
+                const T dv = XF[kr * kTile + 16 * q + lc] * ((16 * q + lc >= kr) ? isd4[q] : T(0));
+                tacc[q] = Mfma<T>::fma(dv, x, tacc[q]);
+            }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+            const int32_t i = 16 * wave + lc;
+            const int32_t j = 16 * q + Mfma<T>::row(lane, rr);
+            if (r0 + i >= c || j >= nb) continue;
+            Lp[(int64_t)(b + j) * c + r0 + i] = tacc[q][rr];
+        }
 }
 
 // L11 block (s, b), nb x nb column-major at the Dinv offset of the block,
 // back into the front's panel
-__global__ __launch_bounds__(256) void k_copy_diag(const PanelTask* __restrict__ tasks, DevSym sym,
-                                                   const double* __restrict__ Lstage, double* __restrict__ L) {
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy_diag(const PanelTask* __restrict__ tasks,
+                                                   const T* __restrict__ Lstage, T* __restrict__ L) {
     const PanelTask tk = tasks[blockIdx.x];
-    const int32_t s = tk.s, b = tk.b;
-    const int32_t n = sym.sfirst[s + 1] - sym.sfirst[s];
-    const int32_t c = sym.snrow[s];
-    const int nb = min(kTile, n - b);
-    const double* src = Lstage + dinv_block_offset(sym, s, b);
-    double* P = L + sym.loff[s] + (int64_t)b * c + b;
+    const int32_t b = tk.b, c = tk.c;
+    const int nb = min(kTile, tk.n - b);
+    const T* src = Lstage + tk.doff;
+    T* P = L + tk.loff + (int64_t)b * c + b;
     for (int idx = threadIdx.x; idx < nb * nb; idx += 256) {
         const int k = idx / nb, r = idx - k * nb;
         P[(int64_t)k * c + r] = src[idx];
@@ -1205,19 +1062,17 @@ __global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int32
 // X := X L_bb^-T for the 64 rows of block rb-1 below the diagonal block,
 // computed as X * (L_bb^-1)^T on MFMA in place.
 template <typename T>
-__global__ __launch_bounds__(256) void k_trsm_gemm(const PanelTask* __restrict__ tasks, DevSym sym,
+__global__ __launch_bounds__(256) void k_trsm_gemm(const PanelTask* __restrict__ tasks,
                                                    T* __restrict__ L, const T* __restrict__ Dinv) {
     typedef typename Mfma<T>::acc_t acc_t;
     __shared__ T As[kTile * kTile];
     __shared__ T Bs[kTile * kTile];
     const PanelTask tk = tasks[blockIdx.x];
-    const int32_t s = tk.s, b = tk.b;
-    const int32_t n = sym.sfirst[s + 1] - sym.sfirst[s];
-    const int32_t c = sym.snrow[s];
+    const int32_t b = tk.b, n = tk.n, c = tk.c;
     const int32_t nb = min(kTile, n - b);
     const int32_t r0 = b + nb + (tk.rb - 1) * kTile;
-    T* Lp = L + sym.loff[s];
-    const T* Db = Dinv + dinv_block_offset(sym, s, b);
+    T* Lp = L + tk.loff;
+    const T* Db = Dinv + tk.doff;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
@@ -1438,28 +1293,24 @@ void launch_gemm(const GemmTask* tasks, int32_t count, const GatherRef* grefs, c
 }
 
 template <typename T>
-void launch_potrf_diag(const PanelTask* tasks, int32_t count, DevSym sym, T* L, T* Dinv, int32_t* err,
+void launch_potrf_diag(const PanelTask* tasks, int32_t count, T* L, T* Dinv, int32_t* err,
                        hipStream_t st) {
     if (count <= 0) return;
-    // FP64: the blocked MFMA form; FP32 keeps the two-wave register-blocked form
-    if constexpr (std::is_same<T, double>::value)
-        help::launch_kernel(k_potrf_mfma<false>, count, 256, 0, st, tasks, sym, L, Dinv, (double*)nullptr, err);
-    else
-        help::launch_kernel(k_potrf_diag<T>, count, 128, 0, st, tasks, sym, L, Dinv, err);
-}
-void launch_panel_fp64(const PanelTask* tasks, int32_t count, DevSym sym, double* L, double* Dinv,
-                       double* Lstage, int32_t* err, hipStream_t st) {
-    if (count > 0)
-        help::launch_kernel(k_potrf_mfma<true>, count, 256, 0, st, tasks, sym, L, Dinv, Lstage, err);
-}
-void launch_copy_diag_fp64(const PanelTask* tasks, int32_t count, DevSym sym, const double* Lstage,
-                           double* L, hipStream_t st) {
-    if (count > 0) help::launch_kernel(k_copy_diag, count, 256, 0, st, tasks, sym, Lstage, L);
+    help::launch_kernel(k_potrf_mfma<T, false>, count, 320, 0, st, tasks, L, Dinv, (T*)nullptr, err);
 }
 template <typename T>
-void launch_trsm_rows(const PanelTask* tasks, int32_t count, DevSym sym, T* L, const T* Dinv,
+void launch_panel(const PanelTask* tasks, int32_t count, T* L, T* Dinv, T* Lstage, int32_t* err,
+                  hipStream_t st) {
+    if (count > 0) help::launch_kernel(k_potrf_mfma<T, true>, count, 320, 0, st, tasks, L, Dinv, Lstage, err);
+}
+template <typename T>
+void launch_copy_diag(const PanelTask* tasks, int32_t count, const T* Lstage, T* L, hipStream_t st) {
+    if (count > 0) help::launch_kernel(k_copy_diag<T>, count, 256, 0, st, tasks, Lstage, L);
+}
+template <typename T>
+void launch_trsm_rows(const PanelTask* tasks, int32_t count, T* L, const T* Dinv,
                       hipStream_t st) {
-    if (count > 0) help::launch_kernel(k_trsm_gemm<T>, count, 256, 0, st, tasks, sym, L, Dinv);
+    if (count > 0) help::launch_kernel(k_trsm_gemm<T>, count, 256, 0, st, tasks, L, Dinv);
 }
 template <typename T>
 void launch_xinv(const XTask* tasks, int32_t count, DevSym sym, const T* L, const T* Dinv, T* X, T* S,
@@ -1482,9 +1333,11 @@ void launch_gather_maps(const GatherRef* grefs, int32_t count, const int32_t* re
     template void launch_extend_add<T>(const EaTask*, int32_t, const EaRef*, DevSym, T*, T*, int32_t, hipStream_t); \
     template void launch_gemm<T>(const GemmTask*, int32_t, const GatherRef*, const int32_t*, const uint32_t*, T*, T*, T*, \
                                  hipStream_t);                                                      \
-    template void launch_potrf_diag<T>(const PanelTask*, int32_t, DevSym, T*, T*, int32_t*,        \
+    template void launch_potrf_diag<T>(const PanelTask*, int32_t, T*, T*, int32_t*,        \
                                        hipStream_t);                                                \
-    template void launch_trsm_rows<T>(const PanelTask*, int32_t, DevSym, T*, const T*, hipStream_t);     \
+    template void launch_panel<T>(const PanelTask*, int32_t, T*, T*, T*, int32_t*, hipStream_t); \
+    template void launch_copy_diag<T>(const PanelTask*, int32_t, const T*, T*, hipStream_t);     \
+    template void launch_trsm_rows<T>(const PanelTask*, int32_t, T*, const T*, hipStream_t);     \
     template void launch_xinv<T>(const XTask*, int32_t, DevSym, const T*, const T*, T*, T*, hipStream_t);
 HELP_INST(double)
 HELP_INST(float)

@@ -109,6 +109,33 @@ def test_factor_matches_oracle(be0, cfg0):
     assert worst <= 1e-12, worst
 
 
+@pytest.mark.parametrize("mode", [L.MODE_DIRECT_FP64, L.MODE_DIRECT_FP32])
+@pytest.mark.parametrize("m", [1, 3, 4, 5, 16, 17, 63, 64, 65, 127, 128, 129, 193])
+def test_panel_sizes(mode, m):
+    """The diagonal-block kernel at its edges (4-column panels, 16-row tiles,
+    64-column blocks and their row blocks), every front through the tiled
+    kernels: a dense-ish random LP's solution within 1e-10 of the oracle's; in
+    FP32 that takes at most 4 refinement steps (each gains about six digits
+    with a factor that is right)."""
+    inst = instances.random_lp(m, 4 * m + 4, min(m, 12), seed=80 + m)
+    rng = np.random.default_rng(m)
+    d = log_uniform(rng, inst.n, -1, 1)
+    b1, b2 = rng.standard_normal(inst.n), rng.standard_normal(inst.m)
+    be = LinearEquation(mode=mode, front_path=1)
+    be.construct(inst)
+    perm, _, _ = be.symbolic_arrays()
+    be.renew(d)
+    x1, x2 = be.solve(d, b1, b2)
+    steps, tiny, bits = be.solve_stats.refine_steps, be.renew_stats.n_tiny_pivots, be.renew_stats.factor_bits
+    be.destruct()
+    _flush(f"panel m={m} mode={mode}: {steps} refinement steps")
+    Lp, Li, Lx = _oracle_factor(inst, perm, d)
+    o1, o2 = O.solve_kkt(inst, perm, Lp, Li, Lx, d, b1, b2)
+    assert tiny == 0 and bits == (64 if mode == L.MODE_DIRECT_FP64 else 32) and steps <= 4
+    assert np.linalg.norm(x2 - o2) <= 1e-10 * np.linalg.norm(o2)
+    assert np.linalg.norm(x1 - o1) <= 1e-10 * np.linalg.norm(o1)
+
+
 @pytest.mark.parametrize("ordering", [L.ORDER_AMD, L.ORDER_ND])
 def test_factor_gathered_fronts(ordering):
     """Fronts whose update-matrix tiles add up their children's entries
