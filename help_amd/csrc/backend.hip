@@ -117,6 +117,40 @@ bool is_big_solve(int32_t c, int32_t ncol) {
     return (c - ncol) > 128 && (int64_t)ncol * (c - ncol) > 32768;
 }
 
+// Places of the update vectors in W (SolveMaps): supernode by supernode, its
+// rows' lists one after the other, each in child order.
+void solve_maps(const Supernodal& S, std::vector<int64_t>& gptr, std::vector<int64_t>& wslot) {
+    const int32_t ns = S.nsuper;
+    auto update_rows = [&](int32_t s) { return (int64_t)S.snrow[s] - (S.sfirst[s + 1] - S.sfirst[s]); };
+    std::vector<int64_t> base(ns + 1, 0);
+    for (int32_t s = 0; s < ns; ++s) {
+        base[s + 1] = base[s];
+        for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) base[s + 1] += update_rows(S.child[t]);
+    }
+    gptr.assign(S.rowoff[ns] + 1, 0);
+    gptr[S.rowoff[ns]] = base[ns];
+    wslot.assign(S.reloff[ns], 0);
+    std::vector<int64_t> at;
+    for (int32_t s = 0; s < ns; ++s) {
+        at.assign((size_t)S.snrow[s] + 1, 0);
+        for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) {
+            const int32_t ch = S.child[t];
+            const int32_t* rel = S.relmap.data() + S.reloff[ch];
+            for (int64_t u = 0; u < update_rows(ch); ++u) ++at[rel[u] + 1];
+        }
+        at[0] = base[s];
+        for (int32_t r = 0; r < S.snrow[s]; ++r) {
+            at[r + 1] += at[r];
+            gptr[S.rowoff[s] + r] = at[r];
+        }
+        for (int32_t t = S.childptr[s]; t < S.childptr[s + 1]; ++t) {
+            const int32_t ch = S.child[t];
+            const int32_t* rel = S.relmap.data() + S.reloff[ch];
+            for (int64_t u = 0; u < update_rows(ch); ++u) wslot[S.reloff[ch] + u] = at[rel[u]]++;
+        }
+    }
+}
+
 void build_schedules(help_gpu* h) {
     const Supernodal& S = h->S;
     h->sbig.assign(S.nsuper, 0);
@@ -605,7 +639,11 @@ void build_schedules(help_gpu* h) {
     };
     // each level's list of supernodes that are not wide: the tiny ones (one
     // wave each) first; wide supernodes go to per-block tasks instead
-    auto level_list = [&](int32_t l, std::vector<int32_t>& out) {
+    auto task = [&](int32_t s, int32_t blk) {
+        return SolveTask{S.loff[s], h->dinvoff[s], h->xoff[s], S.reloff[s], S.rowoff[s],
+                         S.sfirst[s], ncol(s), S.snrow[s], blk, h->sbig[s], s};
+    };
+    auto level_list = [&](int32_t l, std::vector<SolveTask>& out) {
         int32_t ntiny = 0;
         for (int pass = 0; pass < 2; ++pass)
             for (int32_t t = S.levelptr[l]; t < S.levelptr[l + 1]; ++t) {
@@ -613,7 +651,7 @@ void build_schedules(help_gpu* h) {
                 if (wide(s)) continue;
                 bool tiny = S.snrow[s] <= kTinyRows;
                 if (tiny != (pass == 0)) continue;
-                out.push_back(s);
+                out.push_back(task(s, 0));
                 ntiny += tiny;
             }
         return ntiny;
@@ -626,13 +664,16 @@ void build_schedules(help_gpu* h) {
     };
     // lanes per tiny supernode for a level of tiny supernodes only: 32 (two
     // per wave) when every one has at most 32 rows, else 64
-    auto tiny_lanes = [&](const std::vector<int32_t>& lst, int32_t off, int32_t count, int32_t ntiny,
+    auto tiny_lanes = [&](const std::vector<SolveTask>& lst, int32_t off, int32_t count, int32_t ntiny,
                           int32_t nx) {
         if (ntiny != count || nx != 0) return 64;
         for (int32_t t = off; t < off + count; ++t)
-            if (S.snrow[lst[t]] > 32) return 64;
+            if (lst[t].c > 32) return 64;
         return 32;
     };
+    for (int32_t s = 0; s < S.nsuper; ++s)
+        h->sbig[s] = wide(s) ? 2 : is_big_solve(S.snrow[s], ncol(s)) ? 1 : 0;
+    solve_maps(S, h->gptr, h->wslot);
     for (int32_t l = 0; l < S.nlevels; ++l) {
         int32_t off = (int32_t)h->list_fwd.size(), to = (int32_t)h->fgemv.size(), xo = (int32_t)h->fxs.size();
         double w = 0, wg = 0;
@@ -640,17 +681,16 @@ void build_schedules(help_gpu* h) {
         for (int32_t t = S.levelptr[l]; t < S.levelptr[l + 1]; ++t) {
             int32_t s = S.levelsn[t];
             int32_t nc = S.sfirst[s + 1] - S.sfirst[s], c = S.snrow[s];
-            bool big = is_big_solve(c, nc) || wide(s);
+            const bool big = h->sbig[s] != 0;
             if (wide(s)) {
                 w += xinv_bytes(s);
-                for (int32_t i = 0; i < nblk_of(s); ++i) h->fxs.push_back({s, i});
+                for (int32_t i = 0; i < nblk_of(s); ++i) h->fxs.push_back(task(s, i));
             } else {
                 w += tri_bytes(s, !big);
             }
             if (big) {
-                h->sbig[s] = wide(s) ? 2 : 1;
                 wg += wsz * (double)(c - nc) * nc;
-                for (int32_t b = 0; nc + b * 64 < c; ++b) h->fgemv.push_back({s, b});
+                for (int32_t b = 0; nc + b * 64 < c; ++b) h->fgemv.push_back(task(s, b));
             }
         }
         Op o{OP_FWD, off, (int32_t)h->list_fwd.size() - off, w, 0, ntiny};
@@ -669,13 +709,13 @@ void build_schedules(help_gpu* h) {
             int32_t nc = S.sfirst[s + 1] - S.sfirst[s], c = S.snrow[s];
             if (wide(s)) {
                 w += xinv_bytes(s);
-                for (int32_t j = 0; j < nblk_of(s); ++j) h->bxs.push_back({s, j});
+                for (int32_t j = 0; j < nblk_of(s); ++j) h->bxs.push_back(task(s, j));
             } else {
                 w += tri_bytes(s, !h->sbig[s]);
             }
             if (h->sbig[s]) {
                 wg += wsz * (double)(c - nc) * nc;
-                for (int32_t b = 0; b * 16 < nc; ++b) h->bgemv.push_back({s, b});
+                for (int32_t b = 0; b * 16 < nc; ++b) h->bgemv.push_back(task(s, b));
             }
         }
         if ((int32_t)h->bgemv.size() > to) h->sops_bwd.push_back({OP_BWD_GEMV, to, (int32_t)h->bgemv.size() - to, wg});
@@ -768,7 +808,8 @@ void setup_device_factor(help_gpu* h) {
     h->d_list_small.upload(h->list_small, st);
     h->d_list_fwd.upload(h->list_fwd, st);
     h->d_list_bwd.upload(h->list_bwd, st);
-    h->d_big.upload(h->sbig, st);
+    h->d_gptr.upload(h->gptr, st);
+    h->d_wslot.upload(h->wslot, st);
     h->d_ea.upload(h->ea, st);
     h->d_earef.upload(h->earef, st);
     h->d_gref.upload(h->gref, st);
@@ -826,6 +867,7 @@ void setup_device_factor(help_gpu* h) {
     y.relmap = h->d_relmap.p; y.childptr = h->d_childptr.p; y.child = h->d_child.p;
     y.dinvoff = h->d_dinvoff.p;
     y.xoff = h->d_xoff.p;
+    h->smaps = {h->d_gptr.p, h->d_wslot.p, h->d_rowidx.p};
 }
 
 void setup_device(help_gpu* h) {
@@ -930,18 +972,18 @@ void run_trisolve(help_gpu* h, const T* L, const T* Dinv, double* x, int nrhs = 
     for (const Op& o : h->sops_fwd) {
         ProfScope ps(h, o.kind, o.work * nrhs);
         if (o.kind == OP_FWD)
-            launch_fwd_level<T>(h->d_list_fwd.p + o.off, o.count, o.ntiny, h->d_fxs.p + o.xoff, o.xcount, h->sym,
-                                h->d_big.p, L, Dinv, X, x, y, h->d_W.p, nrhs, rs, st, o.wave);
+            launch_fwd_level<T>(h->d_list_fwd.p + o.off, o.count, o.ntiny, h->d_fxs.p + o.xoff, o.xcount, h->smaps,
+                                L, Dinv, X, x, y, h->d_W.p, nrhs, rs, st, o.wave);
         else
-            launch_fwd_gemv<T>(h->d_fgemv.p + o.off, o.count, h->sym, L, y, h->d_W.p, nrhs, rs, st);
+            launch_fwd_gemv<T>(h->d_fgemv.p + o.off, o.count, h->smaps, L, y, h->d_W.p, nrhs, rs, st);
     }
     for (const Op& o : h->sops_bwd) {
         ProfScope ps(h, o.kind, o.work * nrhs);
         if (o.kind == OP_BWD)
-            launch_bwd_level<T>(h->d_list_bwd.p + o.off, o.count, o.ntiny, h->d_bxs.p + o.xoff, o.xcount, h->sym,
-                                h->d_big.p, L, Dinv, X, y, h->d_t.p, x, nrhs, rs, st, o.wave);
+            launch_bwd_level<T>(h->d_list_bwd.p + o.off, o.count, o.ntiny, h->d_bxs.p + o.xoff, o.xcount, h->smaps,
+                                L, Dinv, X, y, h->d_t.p, x, nrhs, rs, st, o.wave);
         else
-            launch_bwd_gemv<T>(h->d_bgemv.p + o.off, o.count, h->sym, L, x, h->d_t.p, nrhs, rs, st);
+            launch_bwd_gemv<T>(h->d_bgemv.p + o.off, o.count, h->smaps, L, x, h->d_t.p, nrhs, rs, st);
     }
     h->prof_fp32 = false;
     HIPCHK(hipGetLastError());

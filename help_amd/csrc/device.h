@@ -221,25 +221,39 @@ void launch_xinv(const XTask* tasks, int32_t count, DevSym sym, const T* L, cons
 // ---- supernodal triangular solves (kernels_solve.hip) ----
 constexpr int kMaxSnCols = 2048;   // supernodes are split to at most this many columns
 
-// Row/column block task of a big supernode in the triangular solves.
+// Task of the triangular solves: a supernode, or one row or column block of a
+// big or wide one, with the supernode's sizes and storage offsets copied from
+// the symbolic structure (one 64-byte load instead of a chain of lookups).
 struct SolveTask {
+    int64_t loff, dinvoff, xoff, reloff, rowoff;
+    int32_t f, n, c;      // first column, columns, rows
+    int32_t blk;          // 64-row block of L21 or L11 (forward) / 16-column block of L21 or
+                          // 64-column block of L11 (backward)
+    int32_t big;          // != 0: the L21 products are left to the gemv kernels
     int32_t s;
-    int32_t blk;          // 64-row block of L21 (forward) / 64-column block (backward)
+};
+// Where the update vectors lie: child entry u of supernode s is
+// W[wslot[reloff[s] + u]], and the entries that land on row r of supernode s
+// are W[gptr[rowoff[s] + r] .. gptr[rowoff[s] + r + 1]), in child order.
+struct SolveMaps {
+    const int64_t* gptr;      // one per entry of rowidx, and the end
+    const int64_t* wslot;     // one per update row
+    const int32_t* rowidx;
 };
 constexpr int kTinyRows = 64;      // supernodes with at most this many rows take one wave
 // The forward solve L y = b reads b and writes y, the backward solve
 // L^T x = y reads y and writes x (x may share b's storage).  Per level:
 // launch_fwd_level, then launch_fwd_gemv for the L21 products of big
 // supernodes; launch_bwd_gemv, then launch_bwd_level.
-// launch_fwd_level / launch_bwd_level: `list` holds the level's supernodes
-// that are not wide, its first `ntiny` with snrow <= kTinyRows (one wave
-// each, four per workgroup), the rest one workgroup each; `xt` holds one task
+// launch_fwd_level / launch_bwd_level: `tasks` holds the level's supernodes
+// that are not wide, its first `ntiny` with c <= kTinyRows (one wave each),
+// the rest one workgroup each; `xt` holds one task
 // per 64-row (forward) or 64-column (backward) block of the level's wide
 // supernodes, solved with the explicit inverse of L11:
 //   forward  y_s(block i) = sum_{j<=i} X_ij g_s(block j), g_s = b_s minus the
 //            children's update vectors;
 //   backward x_s(block j) = sum_{i>=j} X_ij^T (y_s - t_s)(block i).
-// Supernodes with big[s] != 0 leave their L21 products to the gemv kernels.
+// Supernodes with big != 0 leave their L21 products to the gemv kernels.
 // tiny_lanes = 32 (a level of tiny supernodes only, all with at most 32
 // rows): two supernodes per wave, 32 lanes each, same per-lane arithmetic.
 // Every launch solves nrhs right-hand sides at once (blockIdx.y): right-hand
@@ -250,20 +264,20 @@ struct RhsStride {
     int64_t w = 0;   // W
 };
 template <typename T>
-void launch_fwd_level(const int32_t* list, int32_t count, int32_t ntiny, const SolveTask* xt, int32_t nx,
-                      DevSym sym, const int8_t* big, const T* L, const T* Dinv, const T* X, const double* b,
-                      double* y, double* W, int nrhs, RhsStride rs, hipStream_t st, int tiny_lanes = 64);
+void launch_fwd_level(const SolveTask* tasks, int32_t count, int32_t ntiny, const SolveTask* xt, int32_t nx,
+                      SolveMaps mp, const T* L, const T* Dinv, const T* X, const double* b, double* y, double* W,
+                      int nrhs, RhsStride rs, hipStream_t st, int tiny_lanes = 64);
 template <typename T>
-void launch_bwd_level(const int32_t* list, int32_t count, int32_t ntiny, const SolveTask* xt, int32_t nx,
-                      DevSym sym, const int8_t* big, const T* L, const T* Dinv, const T* X, const double* y,
-                      const double* t, double* x, int nrhs, RhsStride rs, hipStream_t st, int tiny_lanes = 64);
-// Forward, big supernodes: W_s += L21 y_s by 64-row blocks.
+void launch_bwd_level(const SolveTask* tasks, int32_t count, int32_t ntiny, const SolveTask* xt, int32_t nx,
+                      SolveMaps mp, const T* L, const T* Dinv, const T* X, const double* y, const double* t,
+                      double* x, int nrhs, RhsStride rs, hipStream_t st, int tiny_lanes = 64);
+// Forward, big supernodes: W_s = the children's entries + L21 y_s by 64-row blocks.
 template <typename T>
-void launch_fwd_gemv(const SolveTask* tasks, int32_t count, DevSym sym, const T* L,
-                     const double* y, double* W, int nrhs, RhsStride rs, hipStream_t st);
+void launch_fwd_gemv(const SolveTask* tasks, int32_t count, SolveMaps mp, const T* L, const double* y, double* W,
+                     int nrhs, RhsStride rs, hipStream_t st);
 // Backward, big supernodes: t[f+j] = sum_{i>=n} L21(i,j) x[row_i] by 16-column blocks.
 template <typename T>
-void launch_bwd_gemv(const SolveTask* tasks, int32_t count, DevSym sym, const T* L,
-                     const double* x, double* t, int nrhs, RhsStride rs, hipStream_t st);
+void launch_bwd_gemv(const SolveTask* tasks, int32_t count, SolveMaps mp, const T* L, const double* x, double* t,
+                     int nrhs, RhsStride rs, hipStream_t st);
 
 }  // namespace help

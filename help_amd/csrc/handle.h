@@ -115,7 +115,7 @@ struct help_gpu {
     std::vector<int8_t> sbig;
     // schedules
     std::vector<Op> fops, sops_fwd, sops_bwd;
-    std::vector<int32_t> list_small, list_fwd, list_bwd;
+    std::vector<int32_t> list_small;
     std::vector<EaTask> ea;
     std::vector<help::EaRef> earef;
     std::vector<help::GatherRef> gref;
@@ -124,7 +124,8 @@ struct help_gpu {
     std::vector<PanelTask> potrf, trsm, panel;
     std::vector<PanelTask> pcopy;   // diagonal blocks factored by fused panel launches
     std::vector<GemmTask> gemm;
-    std::vector<SolveTask> fgemv, bgemv;
+    std::vector<SolveTask> list_fwd, list_bwd, fgemv, bgemv;
+    std::vector<int64_t> gptr, wslot;    // places of the update vectors (SolveMaps)
     // explicit inverse of L11 for supernodes wider than one 64-column block
     bool use_xinv = false;
     bool use_uacc = false;   // some update matrix is built over several panels (Uacc)
@@ -151,7 +152,7 @@ struct help_gpu {
     DBuf<int64_t> d_colptr, d_rowptr, d_pairptr, d_dest, d_diagpos, d_loff, d_uoff, d_rowoff, d_reloff,
         d_dinvoff;
     DBuf<int32_t> d_rowind, d_colind, d_pair_p, d_pair_q, d_colof, d_iperm, d_sfirst, d_snrow,
-        d_rowidx, d_relmap, d_childptr, d_child, d_list_small, d_list_fwd, d_list_bwd, d_err;
+        d_rowidx, d_relmap, d_childptr, d_child, d_list_small, d_err;
     DBuf<double> d_val, d_csrval, d_d, d_dinv, d_b1, d_b2, d_x1, d_x2, d_rp, d_W, d_t, d_tn, d_r,
         d_c, d_z, d_p, d_q, d_part, d_scal, d_slotvals;
     DBuf<double> d_wnz;   // A_ij / d_j per nonzero (the assembly's first factor)
@@ -166,7 +167,6 @@ struct help_gpu {
     DBuf<int32_t> d_slot_row, d_slot_col;
     DBuf<double> d_scale;
     DBuf<float> d_L32, d_Dinv32;
-    DBuf<int8_t> d_big;
     DBuf<EaTask> d_ea;
     DBuf<help::EaRef> d_earef;
     DBuf<help::GatherRef> d_gref;
@@ -174,7 +174,9 @@ struct help_gpu {
     DBuf<uint32_t> d_gtouch;
     DBuf<PanelTask> d_potrf, d_trsm, d_panel, d_pcopy;
     DBuf<GemmTask> d_gemm;
-    DBuf<SolveTask> d_fgemv, d_bgemv, d_fxs, d_bxs;
+    DBuf<SolveTask> d_list_fwd, d_list_bwd, d_fgemv, d_bgemv, d_fxs, d_bxs;
+    DBuf<int64_t> d_gptr, d_wslot;
+    help::SolveMaps smaps{};
     DBuf<XTask> d_xtask;
     DBuf<int64_t> d_xoff;
     DBuf<float> d_X32, d_S32;              // inverse blocks and their partial sums

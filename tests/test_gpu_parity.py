@@ -17,7 +17,7 @@ import pytest
 
 import oracle_bind as O
 from conftest import log_uniform
-from help_amd import LinearEquation, instances
+from help_amd import Instance, LinearEquation, instances
 from help_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
@@ -134,6 +134,84 @@ def test_panel_sizes(mode, m):
     assert tiny == 0 and bits == (64 if mode == L.MODE_DIRECT_FP64 else 32) and steps <= 4
     assert np.linalg.norm(x2 - o2) <= 1e-10 * np.linalg.norm(o2)
     assert np.linalg.norm(x1 - o1) <= 1e-10 * np.linalg.norm(o1)
+
+
+def _from_columns(m, cols, vals):
+    colptr = np.concatenate(([0], np.cumsum([len(c) for c in cols]))).astype(np.int64)
+    return Instance(m, len(cols), colptr, np.concatenate(cols).astype(np.int32), np.concatenate(vals),
+                    np.ones(m), np.ones(len(cols)))
+
+
+@pytest.mark.parametrize("mode", [L.MODE_DIRECT_FP64, L.MODE_DIRECT_FP32])
+def test_solve_many_wide_supernodes(mode):
+    """A level with more blocks of wide supernodes than the launch rule splits
+    (320 independent dense blocks of 65 to 130 rows; with two right-hand sides
+    as with one), against the oracle within 1e-10 and single solves bit for
+    bit."""
+    rng = np.random.default_rng(31)
+    cols, vals, m = [], [], 0
+    for b in range(320):
+        k = 65 + (b * 7) % 66
+        for j in range(k + 3):
+            cols.append(m + np.sort(rng.choice(k, min(k, 24), replace=False)))
+            vals.append(rng.standard_normal(len(cols[-1])))
+        m += k
+    cols += [np.array([i]) for i in range(m)]
+    vals += [np.ones(1)] * m
+    inst = _from_columns(m, cols, vals)
+    d = log_uniform(rng, inst.n, -1, 1)
+    b1a, b1b = rng.standard_normal(inst.n), rng.standard_normal(inst.n)
+    b2a, b2b = rng.standard_normal(m), rng.standard_normal(m)
+    be = LinearEquation(mode=mode)
+    be.construct(inst)
+    sf, _, lv, _ = be.supernodes()
+    nblk = (np.diff(sf) + 63) // 64
+    wide = max(nblk[(lv == l) & (nblk > 1)].sum() for l in np.unique(lv))
+    perm, _, _ = be.symbolic_arrays()
+    _flush(f"many wide mode={mode}: m={m}, {wide} blocks in one level")
+    assert wide > 512
+    be.renew(d)
+    (x1a, x2a), (x1b, x2b) = be.solve2(d, b1a, b2a, b1b, b2b)
+    y1a, y2a = be.solve(d, b1a, b2a)
+    y1b, y2b = be.solve(d, b1b, b2b)
+    be.destruct()
+    for u, v in ((x1a, y1a), (x2a, y2a), (x1b, y1b), (x2b, y2b)):
+        assert np.array_equal(u, v)
+    Lp, Li, Lx = _oracle_factor(inst, perm, d)
+    o1, o2 = O.solve_kkt(inst, perm, Lp, Li, Lx, d, b1a, b2a)
+    assert np.linalg.norm(x2a - o2) <= 1e-10 * np.linalg.norm(o2)
+    assert np.linalg.norm(x1a - o1) <= 1e-10 * np.linalg.norm(o1)
+
+
+@pytest.mark.parametrize("mode,hub", [(L.MODE_DIRECT_FP32, 4300), (L.MODE_DIRECT_FP64, 6200)])
+def test_solve_tall_fronts(mode, hub):
+    """Fronts with more rows than the backward solve holds in LDS: narrow ones
+    (three leaves below a dense block of `hub` rows) and, in FP64, the wide
+    ones of the block; the solution of the normal equations within 1e-10 of a
+    dense solve in FP64."""
+    rng = np.random.default_rng(hub)
+    leaves = 3
+    m = hub + leaves
+    cols = [np.concatenate(([i], np.arange(leaves, m))) for i in range(leaves)] + [np.array([i]) for i in range(m)]
+    vals = [rng.standard_normal(len(c)) for c in cols[:leaves]] + [np.ones(1)] * m
+    inst = _from_columns(m, cols, vals)
+    d = log_uniform(rng, inst.n, -1, 1)
+    b2 = rng.standard_normal(m)
+    be = LinearEquation(mode=mode)
+    be.construct(inst)
+    sf, nr, _, _ = be.supernodes()
+    _flush(f"tall fronts mode={mode}: rows {nr[:5]} columns {np.diff(sf)[:5]}")
+    assert nr[0] > hub
+    be.renew(d)
+    _, x2 = be.solve(d, np.zeros(inst.n), b2)
+    be.destruct()
+    V = np.zeros((m, leaves))
+    for j in range(leaves):
+        V[cols[j], j] = vals[j]
+    M = (V / d[:leaves]) @ V.T
+    M[np.arange(m), np.arange(m)] += 1.0 / d[leaves:] + 1e-5
+    o2 = np.linalg.solve(M, b2)
+    assert min(np.linalg.norm(x2 - o2), np.linalg.norm(x2 + o2)) <= 1e-10 * np.linalg.norm(o2)
 
 
 @pytest.mark.parametrize("ordering", [L.ORDER_AMD, L.ORDER_ND])
