@@ -10,7 +10,7 @@ import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
 import oracle_bind as O
-from help_amd import LinearEquation, instances
+from help_amd import Instance, LinearEquation, instances
 from help_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
@@ -248,6 +248,35 @@ def test_heavy_rows_in_column_blocks():
     be.destruct()
     ref = np.bincount(inst.rowind, inst.val ** 2 / np.repeat(d, np.diff(inst.colptr)), inst.m)
     assert np.allclose(S, ref, rtol=most * np.finfo(float).eps, atol=0)
+
+
+def test_column_products_in_chunks():
+    """A^T x adds each column from LDS chunks of 1,024 nonzeros: columns that
+    end inside, at and beyond a chunk (one of 2,500), 256 to a workgroup with a
+    last partial one; the solution's residual by a CPU product at the stop
+    tolerance (1e-10, within ten times it for the recursive residual), and x1
+    from x2 within the rounding of sums of at most 2,500 terms."""
+    rng = np.random.default_rng(17)
+    m = 2500
+    lens = np.concatenate(([1024, 1, 1023, 2500, 1, 2, 3, 1025], rng.integers(1, 12, 700), [m - 1, 4]))
+    cols = [np.sort(rng.choice(m, k, replace=False)) for k in lens] + [np.array([i]) for i in range(m)]
+    vals = [rng.standard_normal(len(c)) / np.sqrt(len(c)) for c in cols[:len(lens)]] + [np.ones(1)] * m
+    inst = Instance(m, len(cols), np.concatenate(([0], np.cumsum([len(c) for c in cols]))).astype(np.int64),
+                    np.concatenate(cols).astype(np.int32), np.concatenate(vals), np.ones(m), np.ones(len(cols)))
+    assert inst.n % 256 != 0
+    A = _csc(inst)
+    d = np.exp(rng.uniform(-1, 1, inst.n) * np.log(10.0))
+    b1, b2 = rng.standard_normal(inst.n), rng.standard_normal(m)
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=20, pcg_tol=1e-10, pcg_max_iter=5000)
+    be.construct(inst)
+    be.renew(d)
+    x1, x2 = be.solve(d, b1, b2)
+    be.destruct()
+    r = A @ (b1 / d) - b2
+    rel = np.linalg.norm(r - A @ ((A.T @ x2) / d)) / np.linalg.norm(r)
+    bs = np.linalg.norm(x1 - (b1 - A.T @ x2) / d) / np.linalg.norm(x1)
+    _flush(f"column chunks: relative residual {rel:.2e}, back-substitution {bs:.1e}")
+    assert rel <= 1e-9 and bs <= 1e-12
 
 
 def test_pcg_cap_reports_noconv():
