@@ -37,11 +37,6 @@ __device__ inline float round_bf16(float x) {
     return __uint_as_float(u & 0xffff0000u);
 }
 
-__device__ inline float wave_sum_f(float v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 // ---------------------------------------------------------------- features
 __global__ void k_feat_row(int32_t m, const double* __restrict__ g, const double* __restrict__ r, double rs,
                            double mu, float* __restrict__ xr) {
@@ -64,13 +59,22 @@ __global__ void k_feat_col(int32_t n, const double* __restrict__ dinv, double nu
 
 // mode 0: part[b] = sum of log(x) over x > 0, part[nblk + b] = their count;
 // mode 1: part[b] = sum of x^2
-__global__ __launch_bounds__(256) void k_logsum(int64_t n, const double* __restrict__ x, int mode,
-                                                double* __restrict__ part) {
+// Partial sums of the input statistics, blockIdx.y = 0: log g_i and the
+// count of g_i > 0, 1: the same for 1/d, 2: r_i^2 (rows of gridDim.x partials
+// in that order).  Bound by the launches and the copy to the host: one of
+// each for the three.
+__global__ __launch_bounds__(256) void k_stats(int64_t m, int64_t n, const double* __restrict__ g,
+                                               const double* __restrict__ dinv, const double* __restrict__ r,
+                                               double* __restrict__ part) {
     __shared__ double s0[kB], s1[kB];
+    const int what = blockIdx.y;
+    const double* x = what == 0 ? g : what == 1 ? dinv : r;
+    const int64_t cnt = what == 1 ? n : m;
+    part += 2 * what * gridDim.x;
     double a = 0.0, c = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x; i < n; i += (int64_t)gridDim.x * kB) {
+    for (int64_t i = (int64_t)blockIdx.x * kB + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * kB) {
         const double v = x[i];
-        if (mode == 0) {
+        if (what < 2) {
             if (v > 0) { a += log(v); c += 1.0; }
         } else {
             a += v * v;
@@ -85,7 +89,7 @@ __global__ __launch_bounds__(256) void k_logsum(int64_t n, const double* __restr
     }
     if (threadIdx.x == 0) {
         part[blockIdx.x] = s0[0];
-        if (mode == 0) part[gridDim.x + blockIdx.x] = s1[0];
+        if (what < 2) part[gridDim.x + blockIdx.x] = s1[0];
     }
 }
 
@@ -296,16 +300,31 @@ __global__ __launch_bounds__(256) void k_mean(int32_t N, const int64_t* __restri
     store8(out + node * kNnH + f, acc);
 }
 
+// y_i = z_i wo + bo: eight lanes per row, eight features each, so a wave takes
+// eight rows with one load; the features' sum keeps its butterfly (features 32,
+// 16, 8 apart over the lanes, then 4, 2, 1 apart in a lane).  180 thousand
+// rows in BF16: 12 us, 50 us with a wave per row.
 template <typename AT>
 __global__ __launch_bounds__(256) void k_output(int32_t m, const AT* __restrict__ z, const float* __restrict__ wo,
                                                 const float* __restrict__ bo, const double* __restrict__ g,
                                                 double rs, float* __restrict__ y, double* __restrict__ x0) {
-    const int lane = threadIdx.x & 63;
-    const int32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= m) return;
-    const float v = wave_sum_f(ldv(z[(int64_t)row * kNnH + lane]) * wo[lane]);
-    if (lane == 0) {
-        const float yy = v + bo[0];
+    const int f = 8 * (threadIdx.x & 7);
+    const int64_t row = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+    if (row >= m) return;   // (eight lanes together)
+    float v[8];
+    load8(z + row * kNnH + f, v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] *= wo[f + k];
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] += __shfl_xor(v[k], off);
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < off; ++k) v[k] += v[k + off];
+    if (f == 0) {
+        const float yy = v[0] + bo[0];
         y[row] = yy;
         if (x0) x0[row] = g[row] > 0 ? (double)yy * rs / g[row] : 0.0;
     }
@@ -667,8 +686,9 @@ void nn_features(int32_t m, int32_t n, const double* g, const double* r, const d
     help::launch_kernel(k_feat_col, grid_for(n), kB, 0, st, n, dinv, nu, xc);
 }
 
-void nn_logsum_partials(int64_t n, const double* x, int mode, double* part, int nblk, hipStream_t st) {
-    help::launch_kernel(k_logsum, nblk, kB, 0, st, n, x, mode, part);
+void nn_stats_partials(int64_t m, int64_t n, const double* g, const double* dinv, const double* r, double* part,
+                       int nblk, hipStream_t st) {
+    help::launch_kernel(k_stats, dim3(nblk, 3), kB, 0, st, m, n, g, dinv, r, part);
 }
 
 template <typename AT, typename IT>
@@ -705,7 +725,7 @@ void nn_mean(int32_t N, const int64_t* ptr, const int32_t* idx, const double* va
 template <typename AT>
 void nn_output(int32_t m, const AT* z, const float* wo, const float* bo, const double* g, double rs, float* y,
                double* x0, hipStream_t st) {
-    if (m > 0) help::launch_kernel(k_output<AT>, (m + 3) / 4, kB, 0, st, m, z, wo, bo, g, rs, y, x0);
+    if (m > 0) help::launch_kernel(k_output<AT>, (m + 31) / 32, kB, 0, st, m, z, wo, bo, g, rs, y, x0);
 }
 
 void nn_loss_partials(int32_t m, const float* y, const double* dy, const double* g, double rs, double* part,

@@ -49,7 +49,9 @@ struct Bf16 { uint16_t v; };
 // ---- kernels (kernels_mpnn.hip); AT = float or Bf16 activation storage ----
 void nn_features(int32_t m, int32_t n, const double* g, const double* r, const double* dinv, double rs,
                  double mu, double nu, float* xr, float* xc, hipStream_t st);
-void nn_logsum_partials(int64_t n, const double* x, int mode, double* part, int nblk, hipStream_t st);
+// 5 nblk partial sums: log g and its count, log 1/d and its count, r^2
+void nn_stats_partials(int64_t m, int64_t n, const double* g, const double* dinv, const double* r, double* part,
+                       int nblk, hipStream_t st);
 template <typename AT, typename IT>
 void nn_dense(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const float* W, const float* b, AT* out,
               hipStream_t st);

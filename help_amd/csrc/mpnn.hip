@@ -56,7 +56,7 @@ void ensure_workspace(help_mpnn* net, int32_t m, int32_t n) {
     net->cap_n = N;
     const int64_t MN = std::max(M, N);
     net->dd.alloc(N); net->dinv.alloc(N); net->dr.alloc(M); net->ddy.alloc(M); net->g.alloc(M); net->x0.alloc(M);
-    net->stat.alloc(2 * kStatBlocks);
+    net->stat.alloc(5 * kStatBlocks);
     net->y.alloc(M); net->dyv.alloc(M);
     net->xr.alloc(M * help::kNnFR); net->xc.alloc(N * help::kNnFC);
     net->R1.alloc(M * kNnH); net->R2.alloc(M * kNnH);
@@ -79,18 +79,20 @@ struct Acts {
     }
 };
 
-double host_sum(help_mpnn* net, hipStream_t st, int64_t n, const double* x, int mode, double* count) {
-    help::nn_logsum_partials(n, x, mode, net->stat.p, kStatBlocks, st);
-    std::vector<double> h(2 * kStatBlocks);
-    HIPCHK(hipMemcpyAsync(h.data(), net->stat.p, sizeof(double) * (mode == 0 ? 2 : 1) * kStatBlocks,
-                          hipMemcpyDeviceToHost, st));
+// The input statistics: mean logs of g and 1/d (over their positive entries)
+// and the root mean square of r, their partial sums copied back together.
+void input_stats(help_mpnn* net, hipStream_t st, int32_t m, int32_t n, const double* r) {
+    double* p = net->stat.p;
+    help::nn_stats_partials(m, n, net->g.p, net->dinv.p, r, p, kStatBlocks, st);
+    std::vector<double> h(5 * kStatBlocks);
+    HIPCHK(hipMemcpyAsync(h.data(), p, sizeof(double) * 5 * kStatBlocks, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
-    double s = 0, c = 0;
-    for (int b = 0; b < kStatBlocks; ++b) s += h[b];
-    if (mode == 0)
-        for (int b = 0; b < kStatBlocks; ++b) c += h[kStatBlocks + b];
-    if (count) *count = c;
-    return s;
+    double s[5] = {0, 0, 0, 0, 0};
+    for (int q = 0; q < 5; ++q)
+        for (int b = 0; b < kStatBlocks; ++b) s[q] += h[q * kStatBlocks + b];
+    net->mu = s[1] > 0 ? s[0] / s[1] : 0.0;
+    net->nu = s[3] > 0 ? s[2] / s[3] : 0.0;
+    net->rs = s[4] > 0 ? std::sqrt(s[4] / m) : 1.0;
 }
 
 // forward pass; d, r device vectors of the handle's size; x0 out (device)
@@ -103,13 +105,7 @@ void forward(help_mpnn* net, help_gpu* h, const double* d, const double* r, doub
     net->last_n = n;
     help::launch_dinv(d, net->dinv.p, n, st);
     help::launch_csr_split(h->rows, h->d_rowptr.p, h->d_colind.p, h->d_csrval.p, net->dinv.p, net->g.p, true, st);
-    double cnt = 0;
-    const double lg = host_sum(net, st, m, net->g.p, 0, &cnt);
-    net->mu = cnt > 0 ? lg / cnt : 0.0;
-    const double ld = host_sum(net, st, n, net->dinv.p, 0, &cnt);
-    net->nu = cnt > 0 ? ld / cnt : 0.0;
-    const double r2 = host_sum(net, st, m, r, 1, nullptr);
-    net->rs = r2 > 0 ? std::sqrt(r2 / m) : 1.0;
+    input_stats(net, st, m, n, r);
     help::nn_features(m, n, net->g.p, r, net->dinv.p, net->rs, net->mu, net->nu, net->xr.p, net->xc.p, st);
     Acts<AT> a(net);
     const float* W = net->pw.p;
