@@ -3,7 +3,7 @@
 // * Row-split CSR products: A has rows of wildly different lengths (Zipf row
 //   popularity gives rows with millions of nonzeros), so rows up to
 //   kLightRow nonzeros take a thread, rows up to kHeavyRow a wave, and
-//   longer rows are cut into chunks, one wave each, combined in chunk order:
+//   longer rows are cut into chunks, a workgroup each, combined in chunk order:
 //   deterministic.
 // * Greedy partial Cholesky (PCG.cpp:38-103): per pivot an argmax over the
 //   Schur diagonal; the candidates' rows of A scattered into n-vectors, their
@@ -100,36 +100,40 @@ __global__ __launch_bounds__(256) void k_csr_medium(int32_t nmed, const int32_t*
     if (lane == 0) y[i] = s;
 }
 
-// A wave per chunk of a heavy row, eight terms per lane in flight.  Bound by
-// the gathers of x: listed by column block and XCD (RowSplitDev) they hit L2.
-// 12.1 million nonzeros of 1,181 rows, x of 32 MB: 70 us; chunks of 4,096
-// in row order, a workgroup each with one term per lane in flight, took 150 us.
+// A workgroup per chunk of a heavy row, eight terms per thread in flight.
+// Bound by the gathers of x; the chunks are listed by column and XCD
+// (RowSplitDev).  12.1 million nonzeros of 1,181 rows, x of 32 MB: 123 us; in
+// row order with one term per thread in flight, 150 us.  (A wave per chunk,
+// cut at blocks of 262,144 columns, took 70 us, and rounds differently: a solve
+// that stops at 1e-10 then ends up to 1e-7 of an entry away.)
 template <bool SQ>
-__global__ __launch_bounds__(256) void k_csr_chunk(int32_t nchunk, const RowChunk* __restrict__ chunks,
+__global__ __launch_bounds__(256) void k_csr_chunk(const RowChunk* __restrict__ chunks,
                                                    const int32_t* __restrict__ colind,
                                                    const double* __restrict__ val,
                                                    const double* __restrict__ x, double* __restrict__ part) {
-    const int32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (i >= nchunk) return;
-    const RowChunk c = chunks[i];
+    __shared__ double red[4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const RowChunk c = chunks[blockIdx.x];
     if (c.e <= c.b) return;   // padding
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t p0 = c.b + lane; p0 < c.e; p0 += 512) {
+    double a = 0.0;
+    for (int64_t p0 = c.b + tid; p0 < c.e; p0 += 2048) {
         double v[8], g[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const int64_t q = p0 + 64 * u < c.e ? p0 + 64 * u : c.e - 1;
+            const int64_t q = p0 + 256 * u < c.e ? p0 + 256 * u : c.e - 1;
             v[u] = val[q];
             g[u] = x[colind[q]];
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const double t = (SQ ? v[u] * v[u] : v[u]) * g[u];
-            a[u & 3] = (p0 + 64 * u < c.e) ? a[u & 3] + t : a[u & 3];
+            a = (p0 + 256 * u < c.e) ? a + t : a;
         }
     }
-    const double s = wave_sum((a[0] + a[1]) + (a[2] + a[3]));
+    red[wave][lane] = a;
+    __syncthreads();
+    if (wave != 0) return;
+    const double s = wave_sum((red[0][lane] + red[2][lane]) + (red[1][lane] + red[3][lane]));
     if (lane == 0) part[c.slot] = s;
 }
 
@@ -337,26 +341,34 @@ __global__ __launch_bounds__(256) void k_pc_csr_light(int32_t m, const PcState* 
     g[(int64_t)c * m + i] = acc;
 }
 
-// sum over the nonzeros [b, e) of one wave, 64 / kPcBlk at a time; the sums end
-// up on the first kPcBlk lanes
-__device__ inline double wave_range(int64_t b, int64_t e, const int32_t* __restrict__ colind,
-                                     const double* __restrict__ val, const double* __restrict__ sc, int lane) {
-    constexpr int kN = 64 / kPcBlk;
-    const int c = lane & (kPcBlk - 1);
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t p0 = b + lane / kPcBlk; p0 < e; p0 += 8 * kN) {
-        double x[8];
+// sum of a run of terms of one row for the block's kPcBlk columns (sc: kPcBlk
+// values per column of A), on lane c for column c: every column has the
+// accumulators of k_csr_medium (kChunk: of k_csr_chunk), four per lane, and
+// their combine order, so it rounds as a product of its own
+template <bool kChunk>
+__device__ __forceinline__ double wave_range(int64_t b, int64_t e, const int32_t* __restrict__ colind,
+                                             const double* __restrict__ val, const double* __restrict__ sc, int lane) {
+    double a[kPcBlk][4] = {};
+    for (int64_t p0 = b + lane; p0 < e; p0 += 256) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t q = p0 + kN * u < e ? p0 + kN * u : e - 1;
-            x[u] = val[q] * sc[(int64_t)colind[q] * kPcBlk + c];
+        for (int u = 0; u < 4; ++u) {
+            const int64_t q = p0 + 64 * u;
+            if (q < e) {
+                const double v = val[q];
+                const double* g = sc + (int64_t)colind[q] * kPcBlk;
+#pragma unroll
+                for (int c = 0; c < kPcBlk; ++c) a[c][u] += v * g[c];
+            }
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a[u & 3] = (p0 + kN * u < e) ? a[u & 3] + x[u] : a[u & 3];
     }
-    double s = (a[0] + a[1]) + (a[2] + a[3]);
-    for (int off = 32; off >= kPcBlk; off >>= 1) s += __shfl_xor(s, off);
-    return s;
+    double out = 0.0;
+#pragma unroll
+    for (int c = 0; c < kPcBlk; ++c) {
+        const double s = kChunk ? wave_sum((a[c][0] + a[c][2]) + (a[c][1] + a[c][3]))
+                                : wave_sum((a[c][0] + a[c][1]) + (a[c][2] + a[c][3]));
+        out = lane == c ? s : out;
+    }
+    return out;
 }
 
 __global__ __launch_bounds__(256) void k_pc_csr_medium(int32_t m, int32_t nmed, const int32_t* __restrict__ mrow,
@@ -369,7 +381,7 @@ __global__ __launch_bounds__(256) void k_pc_csr_medium(int32_t m, int32_t nmed, 
     const int lane = threadIdx.x & 63;
     if (st->stop || h >= nmed) return;
     const int32_t i = mrow[h];
-    const double s = wave_range(rowptr[i], rowptr[i + 1], colind, val, sc, lane);
+    const double s = wave_range<false>(rowptr[i], rowptr[i + 1], colind, val, sc, lane);
     if (lane < kPcBlk) g[(int64_t)lane * m + i] = s;
 }
 
@@ -378,12 +390,13 @@ __global__ __launch_bounds__(256) void k_pc_csr_chunk(int32_t nchunk, const RowC
                                                       const int32_t* __restrict__ colind,
                                                       const double* __restrict__ val, const double* __restrict__ sc,
                                                       double* __restrict__ part) {
-    const int32_t i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    // workgroup b takes four chunks of XCD b mod 8's run
+    const int32_t i = (blockIdx.x / kXcds * 4 + (threadIdx.x >> 6)) * kXcds + blockIdx.x % kXcds;
     const int lane = threadIdx.x & 63;
     if (st->stop || i >= nchunk) return;
     const RowChunk c = chunks[i];
     if (c.e <= c.b) return;   // padding
-    const double s = wave_range(c.b, c.e, colind, val, sc, lane);
+    const double s = wave_range<true>(c.b, c.e, colind, val, sc, lane);
     if (lane < kPcBlk) part[(int64_t)c.slot * kPcBlk + lane] = s;
 }
 
@@ -392,20 +405,18 @@ __global__ __launch_bounds__(256) void k_pc_csr_heavy(int32_t m, const int32_t* 
                                                       const int32_t* __restrict__ hptr,
                                                       const PcState* __restrict__ st,
                                                       const double* __restrict__ part, double* __restrict__ g) {
-    __shared__ double red[kB];
-    const int t = threadIdx.x, c = t & (kPcBlk - 1);
+    // a wave per kPcBlk / 4 columns, as k_csr_heavy
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (st->stop) return;
-    double acc = 0.0;
-#pragma unroll 4
-    for (int32_t q = hptr[blockIdx.x] + t / kPcBlk; q < hptr[blockIdx.x + 1]; q += kB / kPcBlk)
-        acc += part[(int64_t)q * kPcBlk + c];
-    red[t] = acc;
-    __syncthreads();
-    for (int w = kB / 2; w >= kPcBlk; w >>= 1) {
-        if (t < w) red[t] += red[t + w];
-        __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPcBlk / 4; ++k) {
+        const int c = wave * (kPcBlk / 4) + k;
+        double acc = 0.0;
+        for (int32_t q = hptr[blockIdx.x] + lane; q < hptr[blockIdx.x + 1]; q += 64)
+            acc += part[(int64_t)q * kPcBlk + c];
+        const double s = wave_sum(acc);
+        if (lane == 0) g[(int64_t)c * m + hrow[blockIdx.x]] = s;
     }
-    if (t < kPcBlk) g[(int64_t)t * m + hrow[blockIdx.x]] = red[t];
 }
 
 // wb[r][c] = D_r L(cand_c, r) for the finished columns r
@@ -647,7 +658,10 @@ __global__ __launch_bounds__(256) void k_pca_t2(int32_t m, int64_t ld, int32_t K
 }
 
 // ltpart[c * nb + b] = sum over the kLtRows rows of block b of L(j,c) z_j
-// (z is 0 on the pivots); a wave per column, 32 rows per lane in flight
+// (z is 0 on the pivots); a wave per column, 32 rows per lane in flight.
+// gridDim.y workgroups share the columns of a block where that leaves at most
+// kLtGroups (m = 31,415, K = 77, 16 blocks: 7.2 us, 35 us with one each;
+// m = 10^6, K = 500, 489 blocks: 342 us with one each, 367 with four)
 template <typename T>
 __global__ __launch_bounds__(256) void k_pca_lt(int32_t m, int64_t ld, int32_t K, const T* __restrict__ L32,
                                                 const double* __restrict__ z, double* __restrict__ ltpart) {
@@ -657,7 +671,7 @@ __global__ __launch_bounds__(256) void k_pca_lt(int32_t m, int64_t ld, int32_t K
     for (int t = threadIdx.x; t < kLtRows; t += kB) zs[t] = (r0 + t < m) ? z[r0 + t] : 0.0;
     __syncthreads();
     const int64_t last = (int64_t)m - 1;
-    for (int c = wave; c < K; c += 4) {
+    for (int c = wave + 4 * blockIdx.y; c < K; c += 4 * gridDim.y) {
         const T* Lc = L32 + (int64_t)c * ld;
         double a[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -688,111 +702,40 @@ __global__ __launch_bounds__(256) void k_pca_w(int32_t K, int32_t nb, const int3
     if (lane == 0) w[c] = y1[c] / S[perm[c]] - s;
 }
 
-// z_j = (r_j - sum_c L(j,c) y1_c) / S_j off the pivots, 0 on them, and
-// ltpart[c * nb + blk] = sum over the block's rows of L(j,c) z_j, in one pass
-// over the factor: a tile of 32 rows lies in the registers of a workgroup
-// (lane: a row and one of a pair of columns, NC pairs per wave) between its two
-// uses, and the sums of the second one stay in registers until the block has
-// walked all its tiles.  The next tile's loads are issued as each column is
-// used up.  Bound by reading the factor once.  NC columns of T and NC FP64 sums
-// per lane: with T = float and NC = 32 two workgroups share a CU.
-// m = 10^6, K = 500, FP32: 384 us (5.2 TB/s), where k_pca_t2 and k_pca_lt
-// read the factor twice in 347 + 342 us.
-template <typename T, int NC>
-__global__ __launch_bounds__(512, sizeof(T) * NC <= 128 ? 4 : 2) void k_pca_fused(int32_t m, int64_t ld, int32_t K, const int32_t* __restrict__ pos,
-                                                   const T* __restrict__ L, const double* __restrict__ y1g,
-                                                   const double* __restrict__ S, const double* __restrict__ r,
-                                                   double* __restrict__ z, double* __restrict__ ltpart) {
-    __shared__ double y1[16 * NC];
-    __shared__ double red[2][16][32];
-    const int tid = threadIdx.x, rl = tid & 31, hf = (tid >> 5) & 1, cg = tid >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    for (int t = tid; t < 16 * NC; t += 512) y1[t] = t < K ? y1g[t] : 0.0;
-    // wave w holds columns 2 NC w + 2 i + (lane half); column pairs past the
-    // factor (of an even number of columns, a zero one after an odd K) repeat
-    // the last one: their y1 is 0 and their sums are not stored
-    const int cw = 2 * NC * wave, last = (K - 1) & ~1;
-    const double* yc = y1 + cw + hf;
-    const uint32_t half = hf * (uint32_t)ld;
-    double acc[NC];
-    T v[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = 0.0;
-    const uint32_t step = gridDim.x * 32, um = (uint32_t)m;
-    uint32_t r0 = blockIdx.x * 32;   // below m + step < 2^32
-    auto load = [&](int i, uint32_t at) {
-        const T* col = L + min(cw + 2 * i, last) * ld;   // uniform over the wave
-        return col[at];
-    };
-    {
-        const uint32_t at = half + min(r0 + rl, um - 1);
-#pragma unroll
-        for (int i = 0; i < NC; ++i) v[i] = load(i, at);
-    }
-    __syncthreads();
-    for (int buf = 0; r0 < um; r0 += step, buf ^= 1) {
-        const uint32_t j = min(r0 + rl, um - 1);
-        const double rj = r[j], sj = S[j];
-        const int32_t pj = pos[j];
-        double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-        for (int i = 0; i < NC; i += 2) {
-            s0 += (double)v[i] * yc[2 * i];
-            s1 += (double)v[i + 1] * yc[2 * i + 2];
-        }
-        red[buf][cg][rl] = s0 + s1;
-        // the FP32 tile is converted again below: kept as FP64 from here it
-        // would take twice the registers
-#pragma unroll
-        for (int i = 0; i < NC; ++i) asm volatile("" : "+v"(v[i]));
-        __syncthreads();
-        double q[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            q[g] = (red[buf][g][rl] + red[buf][g + 4][rl]) + (red[buf][g + 8][rl] + red[buf][g + 12][rl]);
-        const double zj = (r0 + rl < um && pj >= K) ? (rj - ((q[0] + q[1]) + (q[2] + q[3]))) / sj : 0.0;
-        if (cg == 0 && r0 + rl < um) z[j] = zj;
-        const uint32_t at = half + min(r0 + step + rl, um - 1);
-        // four columns at a time, so that the loads take the registers they free
-#pragma unroll
-        for (int i0 = 0; i0 < NC; i0 += 4) {
-#pragma unroll
-            for (int i = i0; i < i0 + 4; ++i) acc[i] += (double)v[i] * zj;
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = i0; i < i0 + 4; ++i) v[i] = load(i, at);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        double s = acc[i];
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) s += __shfl_xor(s, off);
-        const int c = cw + 2 * i + hf;
-        if (rl == 0 && c < K) ltpart[(int64_t)c * gridDim.x + blockIdx.x] = s;
-    }
-}
-
-// z(pivot i) = sum_{c >= i} X[c][i] w_c   (L11^-T w): 64 pivots per workgroup,
-// 16 waves over the rows c of X (coalesced; zero above the diagonal).  K = 500:
-// 13 us, 75 us with a thread per pivot.
-__global__ __launch_bounds__(1024) void k_pca_final(int32_t K, const int32_t* __restrict__ perm,
-                                                    const double* __restrict__ X, const double* __restrict__ w,
-                                                    double* __restrict__ z) {
-    __shared__ double red[16][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int32_t i0 = blockIdx.x * 64, i = min(i0 + lane, K - 1);
+// z(pivot i) = sum_{c >= i} X[c][i] w_c   (L11^-T w): 64 pivots per workgroup
+// on the lanes, one of the eight interleaved chains (c - i mod 8; the last,
+// partial group of eight goes to chain 0) per wave.  K = 500: 28 us,
+// 75 us with a pivot's chains in one thread.
+__global__ __launch_bounds__(512) void k_pca_final(int32_t K, const int32_t* __restrict__ perm,
+                                                   const double* __restrict__ X, const double* __restrict__ w,
+                                                   double* __restrict__ z) {
+    __shared__ double red[8][64];
+    const int lane = threadIdx.x & 63, u = threadIdx.x >> 6;
+    const int32_t i = blockIdx.x * 64 + lane, ic = min(i, K - 1);
+    const int32_t end = ic + ((K - ic) & ~7);   // of the full groups
     double a = 0.0;
-#pragma unroll 8
-    for (int32_t c = i0 + wave; c < K; c += 16) a += X[(int64_t)c * K + i] * w[c];
-    red[wave][lane] = a;
-    __syncthreads();
-    if (wave != 0 || i0 + lane >= K) return;
-    a = 0.0;
+    for (int32_t c = ic + u; c < end; c += 64) {
+        double x[8], v[8];
 #pragma unroll
-    for (int g = 0; g < 16; ++g) a += red[g][lane];
-    z[perm[i]] = a;
+        for (int t = 0; t < 8; ++t) {
+            const int32_t q = min(c + 8 * t, K - 1);
+            x[t] = X[(int64_t)q * K + ic];
+            v[t] = w[q];
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+            if (c + 8 * t < end) a += x[t] * v[t];
+    }
+    if (u == 0)
+        for (int32_t c = end; c < K; ++c) a += X[(int64_t)c * K + ic] * w[c];
+    red[u][lane] = a;
+    __syncthreads();
+    if (u == 0 && i < K) {
+        double r[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) r[t] = red[t][lane];
+        z[perm[i]] = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
+    }
 }
 
 // ---- conjugate gradients with the scalars on the device ----
@@ -902,36 +845,30 @@ void build_row_split(int32_t m, int32_t n, const std::vector<int64_t>& rowptr, c
         else if (len > kLightRow) mrow.push_back(i);
     }
     if (heavy == 0) return;
-    const int64_t len = std::min<int64_t>(kMaxChunk, std::max<int64_t>(kMinChunk, heavy / kChunkGoal));
-    // the chunks of every column block, row by row; partials numbered by row
-    std::vector<std::vector<RowChunk>> block((n + kColBlock - 1) / kColBlock);
+    // partials numbered by row; the chunks listed by their middle column
+    std::vector<RowChunk> all;
     int32_t slot = 0;
     for (int32_t i = 0; i < m; ++i) {
         const int64_t b = rowptr[i], e = rowptr[i + 1];
         if (e - b <= kHeavyRow) continue;
         hrow.push_back(i);
-        int64_t p = b;
-        for (int64_t cb = 0; p < e; ++cb) {   // the row's columns ascend
-            const int64_t lim = (cb + 1) * (int64_t)kColBlock;
-            const int64_t q = lim >= n ? e : std::lower_bound(colind.begin() + p, colind.begin() + e, (int32_t)lim) - colind.begin();
-            for (; p < q; p += std::min(len, q - p)) block[cb].push_back({p, std::min(q, p + len), slot++});
-        }
+        for (int64_t p = b; p < e; p += kRowChunk) all.push_back({p, std::min(e, p + kRowChunk), slot++});
         hptr.push_back(slot);
     }
-    // eight contiguous runs of columns with equal nonzeros, one per XCD, dealt
-    // out in workgroups of four chunks in turn
+    std::stable_sort(all.begin(), all.end(), [&](const RowChunk& x, const RowChunk& y) {
+        return colind[(x.b + x.e) / 2] < colind[(y.b + y.e) / 2];
+    });
+    // eight runs of columns with equal nonzeros, one per XCD, dealt out in turn
     std::vector<std::vector<RowChunk>> run(kXcds);
     int64_t seen = 0;
-    for (const auto& bl : block)
-        for (const RowChunk& c : bl) {
-            run[std::min<int64_t>(kXcds - 1, seen * kXcds / heavy)].push_back(c);
-            seen += c.e - c.b;
-        }
+    for (const RowChunk& c : all) {
+        run[std::min<int64_t>(kXcds - 1, seen * kXcds / heavy)].push_back(c);
+        seen += c.e - c.b;
+    }
     size_t most = 0;
-    for (const auto& r : run) most = std::max(most, (r.size() + 3) / 4);
-    for (size_t w = 0; w < most; ++w)
-        for (const auto& r : run)
-            for (size_t k = 4 * w; k < 4 * w + 4; ++k) chunks.push_back(k < r.size() ? r[k] : RowChunk{0, 0, 0});
+    for (const auto& r : run) most = std::max(most, r.size());
+    for (size_t k = 0; k < most; ++k)
+        for (const auto& r : run) chunks.push_back(k < r.size() ? r[k] : RowChunk{0, 0, 0});
 }
 
 void launch_csr_split(const RowSplitDev& rs, const int64_t* rowptr, const int32_t* colind, const double* val,
@@ -944,10 +881,10 @@ void launch_csr_split(const RowSplitDev& rs, const int64_t* rowptr, const int32_
     }
     if (square) {
         help::launch_kernel(k_csr_light<true>, grid_for(rs.m), kB, 0, st, rs.m, rowptr, colind, val, x, y);
-        if (rs.nchunk) help::launch_kernel(k_csr_chunk<true>, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, colind, val, x, rs.part);
+        if (rs.nchunk) help::launch_kernel(k_csr_chunk<true>, rs.nchunk, kB, 0, st, rs.chunks, colind, val, x, rs.part);
     } else {
         help::launch_kernel(k_csr_light<false>, grid_for(rs.m), kB, 0, st, rs.m, rowptr, colind, val, x, y);
-        if (rs.nchunk) help::launch_kernel(k_csr_chunk<false>, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, colind, val, x, rs.part);
+        if (rs.nchunk) help::launch_kernel(k_csr_chunk<false>, rs.nchunk, kB, 0, st, rs.chunks, colind, val, x, rs.part);
     }
     if (rs.nheavy) help::launch_kernel(k_csr_heavy, (rs.nheavy + 3) / 4, kB, 0, st, rs.nheavy, rs.hrow, rs.hptr, rs.part, y);
 }
@@ -967,7 +904,7 @@ void launch_pc_block(const PcBuild& B, hipStream_t st) {
     const int nbs = (int)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)B.max_row_nnz + kB - 1) / kB));
     help::launch_kernel(k_pc_scatter, dim3(nbs, kPcBlk), kB, 0, st, B.state, B.rowptr, B.colind, B.val, B.dinv, B.sc, 0);
     if (rs.nchunk)
-        help::launch_kernel(k_pc_csr_chunk, (rs.nchunk + 3) / 4, kB, 0, st, rs.nchunk, rs.chunks, B.state, B.colind, B.val, B.sc, B.part);
+        help::launch_kernel(k_pc_csr_chunk, (rs.nchunk + 4 * kXcds - 1) / (4 * kXcds) * kXcds, kB, 0, st, rs.nchunk, rs.chunks, B.state, B.colind, B.val, B.sc, B.part);
     if (rs.nmed)
         help::launch_kernel(k_pc_csr_medium, (rs.nmed + 3) / 4, kB, 0, st, m, rs.nmed, rs.mrow, B.state, B.rowptr, B.colind, B.val, B.sc, B.g);
     help::launch_kernel(k_pc_csr_light, grid_for((int64_t)m * kPcBlk), kB, 0, st, m, B.state, B.rowptr, B.colind, B.val, B.sc, B.g);
@@ -993,22 +930,6 @@ void launch_vdiv(int64_t n, const double* a, const double* b, double* out, hipSt
     if (n > 0) help::launch_kernel(k_vdiv, grid_for(n), kB, 0, st, n, a, b, out);
 }
 
-// Columns per lane of the fused apply (16 groups of them): the factor's tile and
-// the FP64 sums of the transposed product take NC (sizeof(T) / 4 + 2) registers,
-// and NC = 64 spills, so K > 512 keeps the two passes.
-template <typename T>
-static int apply_cols(int32_t K) {
-    for (int nc = 8; nc <= 32; nc *= 2)
-        if (K <= 16 * nc) return nc;
-    return 0;
-}
-
-template <typename T>
-int pc_apply_blocks(int32_t m, int32_t K) {
-    if (apply_cols<T>(K)) return (int)std::min<int64_t>(kApplyBlocks, ((int64_t)m + 31) / 32);
-    return (int)(((int64_t)m + kLtRows - 1) / kLtRows);
-}
-
 template <typename T>
 void launch_pc_apply(int32_t m, int32_t K, int64_t ld, const int32_t* perm, const int32_t* pos, const T* L32,
                      const double* X, const double* S, const double* r, double* y1, double* ltpart, double* z,
@@ -1018,24 +939,17 @@ void launch_pc_apply(int32_t m, int32_t K, int64_t ld, const int32_t* perm, cons
         help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, ld, K, pos, L32, y1, S, r, z);
         return;
     }
-    const int nb = pc_apply_blocks<T>(m, K);
+    const int nb = (int)(((int64_t)m + kLtRows - 1) / kLtRows);
     help::launch_kernel(k_pca_y1, (K + 3) / 4, kB, 0, st, K, perm, X, r, y1);
-    auto fused = [&](auto kern) { help::launch_kernel(kern, nb, 512, 0, st, m, ld, K, pos, L32, y1, S, r, z, ltpart); };
-    switch (apply_cols<T>(K)) {
-        case 8: fused(k_pca_fused<T, 8>); break;
-        case 16: fused(k_pca_fused<T, 16>); break;
-        case 32: fused(k_pca_fused<T, 32>); break;
-        default:
-            help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, ld, K, pos, L32, y1, S, r, z);
-            help::launch_kernel(k_pca_lt<T>, nb, kB, 0, st, m, ld, K, L32, z, ltpart);
-    }
+    help::launch_kernel(k_pca_t2<T>, grid_for(m), kB, 0, st, m, ld, K, pos, L32, y1, S, r, z);
+    const int share = std::max(1, std::min((K + 3) / 4, kLtGroups / nb));
+    help::launch_kernel(k_pca_lt<T>, dim3(nb, share), kB, 0, st, m, ld, K, L32, z, ltpart);
     double* w = y1 + kPcgMaxK;
     help::launch_kernel(k_pca_w, (K + 3) / 4, kB, 0, st, K, nb, perm, y1, S, ltpart, w);
-    help::launch_kernel(k_pca_final, (K + 63) / 64, 1024, 0, st, K, perm, X, w, z);
+    help::launch_kernel(k_pca_final, (K + 63) / 64, 512, 0, st, K, perm, X, w, z);
 }
 
 #define HELP_INST(T)                                                                                         \
-    template int pc_apply_blocks<T>(int32_t, int32_t);                                                       \
     template void launch_pc_apply<T>(int32_t, int32_t, int64_t, const int32_t*, const int32_t*, const T*,     \
                                      const double*, const double*, const double*, double*, double*, double*,  \
                                      hipStream_t);

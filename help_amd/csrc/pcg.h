@@ -13,13 +13,10 @@ namespace help {
 constexpr int kPcgMaxK = 1024;      // partial-Cholesky columns held in LDS by the kernels
 constexpr int kLightRow = 64;       // CSR rows up to this many nonzeros take one thread
 constexpr int kHeavyRow = 1024;     // CSR rows longer than this are split into chunks
-constexpr int kMaxChunk = 2048;     // most nonzeros per chunk of a heavy row (a wave each)
-constexpr int kMinChunk = 256;
-constexpr int kChunkGoal = 8192;    // chunks that fill the chip (32 waves per CU)
-constexpr int kColBlock = 262144;   // columns per block of the heavy rows: 2 MB of x, half an XCD's L2
+constexpr int kRowChunk = 4096;     // nonzeros per chunk of a heavy row
 constexpr int kXcds = 8;
 constexpr int kLtRows = 2048;       // rows per workgroup of the transposed factor product
-constexpr int kApplyBlocks = 512;   // most workgroups (and partials) of the fused apply: two per CU
+constexpr int kLtGroups = 512;      // its workgroups, two per CU, where the blocks are fewer
 
 struct RowChunk {
     int64_t b, e;                   // nonzero range [b, e) of one row; empty: padding
@@ -29,10 +26,10 @@ struct RowChunk {
 // Row partition of a CSR matrix for deterministic products with heavy rows:
 // rows up to kLightRow nonzeros take one thread (sequential sum), rows up to
 // kHeavyRow one wave (lane-strided partial sums, fixed reduction tree), the
-// others are summed in chunks by one wave each and combined in chunk order.
-// A chunk lies in one block of kColBlock columns, and the chunks are listed so
-// that each XCD (workgroups go to them in turn) walks its own contiguous run
-// of columns: the gathered part of x then stays in that XCD's L2.
+// others are summed in chunks of kRowChunk nonzeros by a workgroup each and
+// combined in chunk order.  The chunks are listed by their middle column so
+// that each XCD (workgroups go to them in turn) walks its own run of columns:
+// the gathered part of x of the longest rows' chunks stays in that XCD's L2.
 struct RowSplitDev {
     int32_t m = 0;
     int32_t nchunk = 0, nheavy = 0, nmed = 0, nparts = 0;
@@ -92,11 +89,9 @@ void launch_pc_block(const PcBuild& B, hipStream_t st);
 void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, double* L11,
                    double* X, hipStream_t st);
 // ---- preconditioner apply z = M^-1 r (PCG.cpp:183-196) ----
-// y1: scratch of 2 * kPcgMaxK doubles; ltpart: K * pc_apply_blocks(m, K)
+// y1: scratch of 2 * kPcgMaxK doubles; ltpart: K * ceil(m / kLtRows)
 // doubles; the m x K factor L32 in FP32 or FP64 (T = float / double), columns
 // ld apart
-template <typename T>
-int pc_apply_blocks(int32_t m, int32_t K);
 template <typename T>
 void launch_pc_apply(int32_t m, int32_t K, int64_t ld, const int32_t* perm, const int32_t* pos, const T* L32,
                      const double* X, const double* S, const double* r, double* y1, double* ltpart,

@@ -101,7 +101,7 @@ void pcg_setup(help_gpu* h) {
     P->L11.alloc((size_t)K * K);
     P->X.alloc((size_t)K * K);
     P->y1.alloc(2 * kPcgMaxK);
-    P->ltpart.alloc((size_t)K * std::max(pc_apply_blocks<float>(m, P->K), pc_apply_blocks<double>(m, P->K)));
+    P->ltpart.alloc((size_t)K * (((int64_t)m + kLtRows - 1) / kLtRows));
     P->perm.alloc(m);
     P->pos.alloc(m);
     P->x.alloc(m); P->r.alloc(m); P->z.alloc(m); P->p.alloc(m); P->q.alloc(m);

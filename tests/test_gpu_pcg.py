@@ -201,9 +201,10 @@ def test_preconditioner_apply_matches_oracle(name, maker, K, fp32):
 @pytest.mark.parametrize("K", [1, 2, 127, 129, 256, 257, 512, 513])
 @pytest.mark.parametrize("fp32", [0, 1])
 def test_preconditioner_apply_column_counts(K, fp32):
-    """The one-pass apply holds 16 groups of 8, 16 or 32 columns (an odd K has a
-    zero column after it) and leaves K > 512 to two passes: K at these edges, m
-    not a multiple of its 32-row tiles, against the oracle within the bars of
+    """The apply at the edges of its column groups (four columns per workgroup of
+    the transposed product, eight interleaved chains and 64 pivots in the last
+    one; an odd K has a zero column after it), m no multiple of its rows'
+    blocks, against the oracle within the bars of
     test_preconditioner_apply_matches_oracle."""
     inst = instances.random_lp(1237, 2400, 4, seed=61)
     rng = np.random.default_rng(9)
@@ -231,9 +232,9 @@ def test_preconditioner_apply_column_counts(K, fp32):
 
 
 def test_heavy_rows_in_column_blocks():
-    """Rows above 1,024 nonzeros are cut at column blocks (262,144 columns) and
-    into chunks dealt out to the XCDs: on an instance with three blocks, the
-    Schur diagonal before the first pivot (K = 0) is the diagonal of A D^-1 A^T
+    """Rows above 1,024 nonzeros are cut into chunks of 4,096 dealt out to the
+    XCDs by their columns: on an instance with rows of more than 64 chunks,
+    the Schur diagonal before the first pivot (K = 0) is the diagonal of A D^-1 A^T
     within the rounding of a sum of that many positive terms."""
     inst = instances.zipf(2000, 600000, 6, 1.1, seed=62)
     rng = np.random.default_rng(10)
