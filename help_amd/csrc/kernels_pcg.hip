@@ -444,9 +444,11 @@ __global__ __launch_bounds__(256) void k_pc_block(int32_t m, const PcState* __re
     for (int c = 0; c < kPcBlk; ++c)
 #pragma unroll
         for (int q = 0; q < 4; ++q) a[c][q] = 0.0;
-    double l[2][4];   // this group of four columns and the next one
+    double l[2][4] = {};   // this group of four columns and the next one
+    if (kb > 0) {          // (there may be fewer than four columns in all)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) l[0][q] = L[(int64_t)q * m + j];
+        for (int q = 0; q < 4; ++q) l[0][q] = L[(int64_t)q * m + j];
+    }
     for (int32_t r = 0; r < kb; r += 8) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
