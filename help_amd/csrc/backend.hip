@@ -1443,8 +1443,9 @@ int help_gpu_renew(help_gpu* h, const double* d, help_renew_stats* rs) {
         if (h->use_pcg) {
             HIPCHK(hipEventRecord(h->ev[1], st));
             {
-                ProfScope ps(h, HELP_K_PCG_BUILD, help::pcg_build_bytes(h));
+                ProfScope ps(h, HELP_K_PCG_BUILD, 0.0);
                 help::pcg_renew(h);
+                ps.set_work(help::pcg_build_bytes(h));
             }
             HIPCHK(hipEventRecord(h->ev[2], st));
             HIPCHK(hipStreamSynchronize(st));

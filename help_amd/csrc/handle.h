@@ -238,7 +238,7 @@ namespace help {
 void pcg_setup(help_gpu* h);
 void pcg_renew(help_gpu* h);
 int pcg_solve(help_gpu* h, const double* rhs, const double* x0, double* x2, double& rel);
-// algorithmic HBM bytes: one partial-Cholesky build, one CG iteration
+// algorithmic HBM bytes: the last partial-Cholesky build, one CG iteration
 double pcg_build_bytes(const help_gpu* h);
 double pcg_iteration_bytes(const help_gpu* h);
 void pcg_download(help_gpu* h, int32_t* K, int32_t* perm, double* D, double* S, double* L);

@@ -206,42 +206,54 @@ __device__ inline bool better(double v, int32_t i, double bv, int32_t bi) {
     return v > bv || (v == bv && i < bi);
 }
 
-// The pivots are taken kPcBlk at a time.  A block starts with kPcBlk
-// candidates, the largest Schur diagonals (ties to the lowest position); their
-// columns of A D^-1 A^T and their left-looking sums over all finished factor
-// columns are formed together, so the m x k factor and A are read once per
-// block instead of once per pivot.  Each step then takes the pivot as before,
-// the largest Schur diagonal of all, and adds the block's own columns; when
-// that pivot is none of the candidates the block ends there and the next one
-// starts with it.  The order of the pivots is the greedy one whatever the
-// candidates, and a column's sum over the earlier ones keeps its four
-// interleaved chains (PCG.cpp:85-102 in that order), so light rows round as
-// with one column at a time.  The state (PcState) stays on the device: every
-// kernel returns at once when its block has ended.
-// m = 10^6, K = 500 (zipf): 64.3 ms per build, 291 ms pivot by pivot (of which
-// the factor reads 178 ms and the products with A 100 ms).
+// A group of pivots starts with kPcBlk candidates, the largest Schur diagonals
+// (ties to the lowest position), and is formed in one of two ways:
+// * as a block: the candidates' columns of A D^-1 A^T and their left-looking
+//   sums over all finished factor columns together, so the m x k factor and A
+//   are read once per block instead of once per pivot.  Each step then takes the
+//   largest Schur diagonal of all and adds the block's own columns; when that
+//   pivot is none of the candidates the block ends there.
+// * pivot by pivot: each step takes the largest Schur diagonal, whatever row it
+//   is, then forms its product with A and its sums.
+// Either way the state counts the leading pivots that were candidates
+// (PcState::taken), from which the host chooses the next group's form
+// (pcg_renew).  Rows in groups of more than kPcBlk near-parallel ones with
+// similar diagonals lose all other candidates to the first pivot, and a block of
+// one pivot costs more than a single one (kPcFew).
+// The order of the pivots is the greedy one whatever the groups, and a column's
+// sum over the earlier ones keeps its four interleaved chains (PCG.cpp:85-102
+// in that order), so every column rounds the same in both forms.  The state
+// stays on the device: every kernel of a block returns at once when it has
+// ended.
+// m = 10^6, K = 500 (zipf): 63.4 ms per build, 328 ms with a search, a product
+// and the sums per pivot (of which the factor reads take 178 ms and the
+// products with A 136 ms).  Rows in groups of 20 near-parallel ones: 386 ms;
+// 390 ms per pivot, 637 ms in blocks alone.  m = 30,000, K = 77: 2.1 ms; 2.2
+// per pivot, 12.7 in blocks alone.
 typedef PcBest Best;
 __device__ inline bool ahead(const Best& a, const Best& b) { return better(a.v, a.pos, b.v, b.pos); }
 
-__device__ inline Best block_best(Best x, Best* red) {
-    const int t = threadIdx.x;
-    red[t] = x;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w && ahead(red[t + w], red[t])) red[t] = red[t + w];
-        __syncthreads();
+__device__ inline Best block_best(Best x, Best (&red)[kB / 64]) {
+    for (int off = 32; off > 0; off >>= 1) {
+        const Best o = {__shfl_xor(x.v, off), __shfl_xor(x.pos, off), __shfl_xor(x.row, off)};
+        if (ahead(o, x)) x = o;
     }
-    const Best b = red[0];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    Best b = red[0];
+#pragma unroll
+    for (int w = 1; w < kB / 64; ++w)
+        if (ahead(red[w], b)) b = red[w];
     __syncthreads();
     return b;
 }
 
-// the block's kPcBlk best rows not yet pivoted, in order; the first one is also
+// the workgroup's kPcBlk best rows not yet pivoted, in order; the first one is also
 // its argmax partial
 __global__ __launch_bounds__(256) void k_pc_top_part(int32_t m, const int32_t* __restrict__ pos,
                                                      const double* __restrict__ S, const PcState* __restrict__ st,
                                                      PcBest* __restrict__ top, PcBest* __restrict__ arg) {
-    __shared__ Best red[kB];
+    __shared__ Best red[kB / 64];
     const int32_t k = st->k;
     const Best none = {-HUGE_VAL, INT_MAX, -1};
     // this thread's best row strictly behind `last`
@@ -264,11 +276,11 @@ __global__ __launch_bounds__(256) void k_pc_top_part(int32_t m, const int32_t* _
     }
 }
 
-// the candidates of the next block out of nb blocks' best
+// the candidates of the next group out of nb workgroups' best
 __global__ __launch_bounds__(256) void k_pc_top_pick(int32_t nb, int32_t K, const PcBest* __restrict__ top,
                                                      PcState* __restrict__ st) {
     constexpr int kPer = kTopBlocks / kB;   // lists per thread, each in order
-    __shared__ Best red[kB];
+    __shared__ Best red[kB / 64];
     const Best none = {-HUGE_VAL, INT_MAX, -1};
     int at[kPer];
     Best head[kPer];
@@ -278,9 +290,7 @@ __global__ __launch_bounds__(256) void k_pc_top_pick(int32_t nb, int32_t K, cons
         at[u] = 0;
         head[u] = b < nb ? top[b * kPcBlk] : none;
     }
-    const int32_t force = st->force;
-    if (threadIdx.x == 0 && force >= 0) st->cand[0] = force;
-    for (int r = force >= 0 ? 1 : 0; r < kPcBlk; ++r) {
+    for (int r = 0; r < kPcBlk; ++r) {
         Best mine = none;
 #pragma unroll
         for (int u = 0; u < kPer; ++u)
@@ -294,22 +304,24 @@ __global__ __launch_bounds__(256) void k_pc_top_pick(int32_t nb, int32_t K, cons
     }
     if (threadIdx.x == 0) {
         st->k0 = st->k;
+        st->taken = 0;
         st->stop = st->k >= K;
-        st->force = -1;
     }
 }
 
-// sc[j][c] = A(cand_c, j) dinv_j on the candidates' rows (blockIdx.y = c), or 0
-__global__ void k_pc_scatter(const PcState* __restrict__ st, const int64_t* __restrict__ rowptr,
+// sc[j][c] = A(cand_c, j) dinv_j on the candidates' rows (blockIdx.y = c), or 0;
+// one: sc[j] on the pivot's row (k_pc_column clears it)
+__global__ void k_pc_scatter(const PcState* __restrict__ st, int one, const int64_t* __restrict__ rowptr,
                              const int32_t* __restrict__ colind, const double* __restrict__ val,
                              const double* __restrict__ dinv, double* __restrict__ sc, int clear) {
     const int c = blockIdx.y;
-    const int32_t col = st->cand[c];
+    const int32_t col = one ? st->col : st->cand[c];
     if (st->stop || col < 0) return;
+    const int stride = one ? 1 : kPcBlk;
     const int64_t b = rowptr[col], e = rowptr[col + 1];
     for (int64_t p = b + (int64_t)blockIdx.x * kB + threadIdx.x; p < e; p += (int64_t)gridDim.x * kB) {
         const int32_t j = colind[p];
-        sc[(int64_t)j * kPcBlk + c] = clear ? 0.0 : val[p] * dinv[j];
+        sc[(int64_t)j * stride + c] = clear ? 0.0 : val[p] * dinv[j];
     }
 }
 
@@ -469,18 +481,18 @@ __global__ __launch_bounds__(256) void k_pc_block(int32_t m, const PcState* __re
         for (int q = 0; q < 4; ++q) acc[(int64_t)(4 * c + q) * m + j] = a[c][q];
 }
 
-// The next pivot: the best of np partials.  Out of candidates or done: the block
-// stops.  Else it is swapped to position k, w_r = D_r L(col, r) for r < k and
-// D_k = g(col) - sum_r w_r L(col, r).
-__global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t K, int32_t np, const PcBest* __restrict__ arg,
-                                                  PcState* __restrict__ st, int32_t* __restrict__ perm,
-                                                  int32_t* __restrict__ pos, const double* __restrict__ g,
-                                                  const double* __restrict__ L, double* __restrict__ D,
+// The next pivot: the best of np partials.  In a block (one = 0), done or none of
+// the candidates: the block stops.  Else it is swapped to position k and
+// w_r = D_r L(col, r) for r < k; s = sum_r w_r L(col, r).
+__global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t K, int one, int32_t np,
+                                                  const PcBest* __restrict__ arg, PcState* __restrict__ st,
+                                                  int32_t* __restrict__ perm, int32_t* __restrict__ pos,
+                                                  const double* __restrict__ L, const double* __restrict__ D,
                                                   double* __restrict__ w) {
-    __shared__ Best redb[kB];
+    __shared__ Best redb[kB / 64];
     __shared__ double red[kB];
     if (st->stop) return;
-    const int32_t k = st->k;
+    const int32_t k = st->k, before = k - st->k0, taken = st->taken;
     Best mine = {-HUGE_VAL, INT_MAX, -1};
     for (int i = threadIdx.x; i < np; i += kB) {
         const Best c = arg[i];
@@ -488,31 +500,17 @@ __global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t K, int32_t 
     }
     Best b = block_best(mine, redb);
     // no row is ahead of none (every value left is NaN): the row at position k
-    const bool lost = b.row < 0 && k < K;
-    if (lost) b = {0.0, k, perm[k]};
+    if (b.row < 0 && k < K) b = {0.0, k, perm[k]};
     int ci = -1;
 #pragma unroll
     for (int c = 0; c < kPcBlk; ++c)
         if (k < K && st->cand[c] == b.row) ci = c;
     __syncthreads();   // every thread has read the state
-    if (ci < 0) {
-        if (threadIdx.x == 0) {
-            st->stop = 1;
-            if (lost) st->force = b.row;
-        }
+    if (k >= K || (ci < 0 && !one)) {
+        if (threadIdx.x == 0) st->stop = 1;
         return;
     }
     const int32_t col = b.row;
-    if (threadIdx.x == 0) {
-        const int32_t a = perm[k];
-        perm[k] = col;
-        perm[b.pos] = a;
-        pos[a] = b.pos;
-        pos[col] = k;
-        st->col = col;
-        st->ci = ci;
-        st->k = k + 1;
-    }
     double acc = 0.0;
     for (int32_t r = threadIdx.x; r < k; r += kB) {
         const double l = L[(int64_t)r * m + col];
@@ -521,22 +519,41 @@ __global__ __launch_bounds__(256) void k_pc_pivot(int32_t m, int32_t K, int32_t 
         acc += wr * l;
     }
     const double s = block_sum(acc, red);
-    if (threadIdx.x == 0) D[k] = g[(int64_t)ci * m + col] - s;
+    if (threadIdx.x == 0) {
+        const int32_t a = perm[k];
+        perm[k] = col;
+        perm[b.pos] = a;
+        pos[a] = b.pos;
+        pos[col] = k;
+        st->col = col;
+        st->ci = one ? 0 : ci;
+        st->s = s;
+        st->k = k + 1;
+        if (ci >= 0 && taken == before) st->taken = taken + 1;
+    }
 }
 
-// column k of L over all rows: 1 at the pivot, 0 at earlier pivots, else
-// (g_j - sum_r L(j,r) w_r) / D_k; the Schur diagonal loses D_k L(j,k)^2; the
-// best row left of every block
+// D_k = g(col) - s, and column k of L over all rows: 1 at the pivot, 0 at
+// earlier pivots, else (g_j - sum_r L(j,r) w_r) / D_k; the Schur diagonal loses
+// D_k L(j,k)^2; the best row left of every workgroup.  kBlock: the sums over the
+// columns before the block are there (accs).  Else the pivot's vector is cleared.
+template <bool kBlock>
 __global__ __launch_bounds__(256) void k_pc_column(int32_t m, const PcState* __restrict__ st,
                                                    const int32_t* __restrict__ pos, const double* __restrict__ g,
                                                    const double* __restrict__ accs, const double* __restrict__ wg,
-                                                   const double* __restrict__ D, double* __restrict__ L,
+                                                   double* __restrict__ D, double* __restrict__ L,
                                                    float* __restrict__ L32, int64_t ld32, double* __restrict__ S,
-                                                   PcBest* __restrict__ arg) {
-    __shared__ Best red[kB];
+                                                   PcBest* __restrict__ arg, const int64_t* __restrict__ rowptr,
+                                                   const int32_t* __restrict__ colind, double* __restrict__ sc) {
+    __shared__ Best red[kB / 64];
     if (st->stop) return;
-    const int32_t k = st->k - 1, kb = st->k0 & ~3, col = st->col, ci = st->ci;
-    const double dk = D[k];
+    const int32_t k = st->k - 1, kb = kBlock ? st->k0 & ~3 : 0, col = st->col, ci = st->ci;
+    const double dk = g[(int64_t)ci * m + col] - st->s;
+    if (blockIdx.x == 0 && threadIdx.x == 0) D[k] = dk;
+    if constexpr (!kBlock) {
+        for (int64_t p = rowptr[col] + (int64_t)blockIdx.x * kB + threadIdx.x; p < rowptr[col + 1]; p += (int64_t)gridDim.x * kB)
+            sc[colind[p]] = 0.0;
+    }
     Best best = {-HUGE_VAL, INT_MAX, -1};
     for (int64_t j = (int64_t)blockIdx.x * kB + threadIdx.x; j < m; j += (int64_t)gridDim.x * kB) {
         double l = 0.0;
@@ -544,9 +561,11 @@ __global__ __launch_bounds__(256) void k_pc_column(int32_t m, const PcState* __r
         if (j == col) {
             l = 1.0;
         } else if (pj >= k) {
-            double a[4];
+            double a[4] = {};
+            if constexpr (kBlock) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) a[q] = accs[(int64_t)(4 * ci + q) * m + j];
+                for (int q = 0; q < 4; ++q) a[q] = accs[(int64_t)(4 * ci + q) * m + j];
+            }
             int32_t r = kb;
             for (; r + 3 < k; r += 4)
 #pragma unroll
@@ -896,15 +915,33 @@ void launch_csc_t_scaled(int32_t n, const int64_t* colptr, const int32_t* rowind
     if (n > 0) help::launch_kernel(k_csc_ts, grid_for(n), kB, 0, st, n, colptr, rowind, val, dinv, x, t);
 }
 
+namespace {
+int pc_blocks(const PcBuild& B, int most) { return (int)std::min<int64_t>(most, ((int64_t)B.rows.m + kB - 1) / kB); }
+void pc_candidates(const PcBuild& B, hipStream_t st) {
+    const int nbt = pc_blocks(B, kTopBlocks);
+    help::launch_kernel(k_pc_top_part, nbt, kB, 0, st, B.rows.m, B.pos, B.S, B.state, B.top, B.arg);
+    help::launch_kernel(k_pc_top_pick, 1, kB, 0, st, nbt, B.K, B.top, B.state);
+}
+void pc_scatter(const PcBuild& B, int one, int clear, hipStream_t st) {
+    const int nb = (int)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)B.max_row_nnz + kB - 1) / kB));
+    help::launch_kernel(k_pc_scatter, dim3(nb, one ? 1 : kPcBlk), kB, 0, st, B.state, one, B.rowptr, B.colind, B.val, B.dinv, B.sc, clear);
+}
+// top: the partials of the search are the candidates', else the last column's
+void pc_pivot(const PcBuild& B, int one, bool top, hipStream_t st) {
+    const int np = pc_blocks(B, top ? kTopBlocks : kColumnBlocks);
+    help::launch_kernel(k_pc_pivot, 1, kB, 0, st, B.rows.m, B.K, one, np, B.arg, B.state, B.perm, B.pos, B.L, B.D, B.w);
+}
+template <bool kBlock>
+void pc_column(const PcBuild& B, hipStream_t st) {
+    help::launch_kernel(k_pc_column<kBlock>, pc_blocks(B, kColumnBlocks), kB, 0, st, B.rows.m, B.state, B.pos, B.g, B.acc, B.w, B.D, B.L, B.L32, B.ld32, B.S, B.arg, B.rowptr, B.colind, B.sc);
+}
+}  // namespace
+
 void launch_pc_block(const PcBuild& B, hipStream_t st) {
-    const int32_t m = B.rows.m, K = B.K;
-    const int nbt = (int)std::min<int64_t>(kTopBlocks, ((int64_t)m + kB - 1) / kB);
-    const int nbc = (int)std::min<int64_t>(kColumnBlocks, ((int64_t)m + kB - 1) / kB);
+    const int32_t m = B.rows.m;
     const RowSplitDev& rs = B.rows;
-    help::launch_kernel(k_pc_top_part, nbt, kB, 0, st, m, B.pos, B.S, B.state, B.top, B.arg);
-    help::launch_kernel(k_pc_top_pick, 1, kB, 0, st, nbt, K, B.top, B.state);
-    const int nbs = (int)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)B.max_row_nnz + kB - 1) / kB));
-    help::launch_kernel(k_pc_scatter, dim3(nbs, kPcBlk), kB, 0, st, B.state, B.rowptr, B.colind, B.val, B.dinv, B.sc, 0);
+    pc_candidates(B, st);
+    pc_scatter(B, 0, 0, st);
     if (rs.nchunk)
         help::launch_kernel(k_pc_csr_chunk, (rs.nchunk + 4 * kXcds - 1) / (4 * kXcds) * kXcds, kB, 0, st, rs.nchunk, rs.chunks, B.state, B.colind, B.val, B.sc, B.part);
     if (rs.nmed)
@@ -912,12 +949,22 @@ void launch_pc_block(const PcBuild& B, hipStream_t st) {
     help::launch_kernel(k_pc_csr_light, grid_for((int64_t)m * kPcBlk), kB, 0, st, m, B.state, B.rowptr, B.colind, B.val, B.sc, B.g);
     if (rs.nheavy)
         help::launch_kernel(k_pc_csr_heavy, rs.nheavy, kB, 0, st, m, rs.hrow, rs.hptr, B.state, B.part, B.g);
-    help::launch_kernel(k_pc_scatter, dim3(nbs, kPcBlk), kB, 0, st, B.state, B.rowptr, B.colind, B.val, B.dinv, B.sc, 1);
-    help::launch_kernel(k_pc_weights, grid_for((int64_t)K * kPcBlk), kB, 0, st, m, B.state, B.D, B.L, B.wb);
+    pc_scatter(B, 0, 1, st);
+    help::launch_kernel(k_pc_weights, grid_for((int64_t)B.K * kPcBlk), kB, 0, st, m, B.state, B.D, B.L, B.wb);
     help::launch_kernel(k_pc_block, grid_for(m), kB, 0, st, m, B.state, B.pos, B.wb, B.L, B.acc);
     for (int s = 0; s < kPcBlk; ++s) {
-        help::launch_kernel(k_pc_pivot, 1, kB, 0, st, m, K, s == 0 ? nbt : nbc, B.arg, B.state, B.perm, B.pos, B.g, B.L, B.D, B.w);
-        help::launch_kernel(k_pc_column, nbc, kB, 0, st, m, B.state, B.pos, B.g, B.acc, B.w, B.D, B.L, B.L32, B.ld32, B.S, B.arg);
+        pc_pivot(B, 0, s == 0, st);
+        pc_column<true>(B, st);
+    }
+}
+
+void launch_pc_pivots(const PcBuild& B, int32_t steps, bool candidates, hipStream_t st) {
+    if (candidates) pc_candidates(B, st);
+    for (int s = 0; s < steps; ++s) {
+        pc_pivot(B, 1, s == 0 && candidates, st);
+        pc_scatter(B, 1, 0, st);
+        launch_csr_split(B.rows, B.rowptr, B.colind, B.val, B.sc, B.g, false, st);
+        pc_column<false>(B, st);
     }
 }
 

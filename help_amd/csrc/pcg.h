@@ -53,16 +53,19 @@ void launch_vdiv(int64_t n, const double* a, const double* b, double* out, hipSt
 void launch_csc_t_scaled(int32_t n, const int64_t* colptr, const int32_t* rowind, const double* val,
                          const double* dinv, const double* x, double* t, hipStream_t st);
 
-// ---- partial Cholesky build, kPcBlk pivots per call sequence ----
-constexpr int kPcBlk = 16;          // candidates (and most pivots) of a block
+// ---- partial Cholesky build, a group of pivots per call sequence ----
+constexpr int kPcBlk = 16;          // candidates (and most pivots) of a group
+constexpr int kPcFew = 4;           // candidates from which a block pays: with one it takes as long as 1.6
+                                    // single pivots at m = 10^6, 3.2 at 200,000, 6 at 30,000
 constexpr int kTopBlocks = 512;
 constexpr int kColumnBlocks = 2048;
 struct PcState {
     int32_t k;                      // pivots taken
-    int32_t k0;                     // ... when the block started
-    int32_t stop;                   // the block has ended
-    int32_t col, ci;                // the step's pivot row and its place among the candidates
-    int32_t force;                  // row to lead the next block's candidates, or -1
+    int32_t k0;                     // ... when the group started
+    int32_t taken;                  // the group's leading pivots that were candidates
+    int32_t stop;                   // the group has ended
+    int32_t col, ci;                // the step's pivot row and its place among the columns in g
+    double s;                       // sum_r D_r L(col, r)^2 over the columns before the step's
     int32_t cand[kPcBlk];
 };
 struct PcBest {
@@ -85,7 +88,11 @@ struct PcBuild {
     double *part;                   // partials of the heavy rows * kPcBlk
     double *g, *acc, *wb;           // m * kPcBlk; 4 m kPcBlk; K * kPcBlk
 };
+// a block: up to kPcBlk pivots, as long as they are candidates
 void launch_pc_block(const PcBuild& B, hipStream_t st);
+// steps pivots one by one (at most K - k); without candidates (after another
+// group of single pivots only) PcState::k0 and taken stay as they are
+void launch_pc_pivots(const PcBuild& B, int32_t steps, bool candidates, hipStream_t st);
 void launch_pc_l11(int32_t m, int32_t K, const int32_t* perm, const double* L, double* L11,
                    double* X, hipStream_t st);
 // ---- preconditioner apply z = M^-1 r (PCG.cpp:183-196) ----

@@ -6,7 +6,6 @@
 // with the preconditioner applied from the FP32 copy of the factor.
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 #include <mutex>
 #include <string>
 
@@ -60,7 +59,8 @@ struct PcgState {
     DBuf<int32_t> perm, pos;
     DBuf<PcState> state;
     DBuf<PcBest> top, arg;
-    PcState* hstate = nullptr;       // pinned
+    PcState* hstate = nullptr;       // pinned: the state after the last two groups of the build
+    double build_bytes = 0;          // algorithmic bytes of the last build
     DBuf<double> x, r, z, p, q, t;
     std::vector<int32_t> iota;
 };
@@ -97,7 +97,7 @@ void pcg_setup(help_gpu* h) {
     P->state.alloc(1);
     P->top.alloc(kTopBlocks * kPcBlk);
     P->arg.alloc(std::max(kTopBlocks, kColumnBlocks));
-    HIPCHK(hipHostMalloc((void**)&P->hstate, sizeof(PcState), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&P->hstate, 2 * sizeof(PcState), hipHostMallocDefault));
     P->L11.alloc((size_t)K * K);
     P->X.alloc((size_t)K * K);
     P->y1.alloc(2 * kPcgMaxK);
@@ -136,34 +136,60 @@ void pcg_renew(help_gpu* h) {
     B.perm = P->perm.p; B.pos = P->pos.p;
     B.S = P->S.p; B.D = P->D.p; B.L = P->L.p; B.w = P->w.p; B.L32 = h->opts.pcg_fp32_precond ? P->L32.p : nullptr;
     B.sc = P->sc.p; B.part = P->bpart.p; B.g = P->g.p; B.acc = P->acc.p; B.wb = P->wb.p;
-    std::memset(P->hstate, 0, sizeof(PcState));
-    P->hstate->force = -1;
-    HIPCHK(hipMemcpyAsync(P->state.p, P->hstate, sizeof(PcState), hipMemcpyHostToDevice, st));
-    // as many blocks as the pivots need if every candidate is taken; then, as
-    // long as pivots are missing, as many again as the rest needs.  A block
-    // takes at least one pivot, or names the row that leads the next one.
-    int32_t k = 0;
-    for (int64_t blocks = 0; k < K;) {
-        if (blocks > 2 * (int64_t)K + kPcBlk) throw HipError("partial Cholesky: no pivot taken", HELP_ERR_HIP);
-        for (int32_t b = 0; b < (K - k + kPcBlk - 1) / kPcBlk; ++b, ++blocks) launch_pc_block(B, st);
-        HIPCHK(hipMemcpyAsync(P->hstate, P->state.p, sizeof(PcState), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        k = P->hstate->k;
+    HIPCHK(hipMemsetAsync(P->state.p, 0, sizeof(PcState), st));
+    // Groups of pivots: a block as long as the last group's leading candidates
+    // were enough for one to pay, else pivot by pivot in groups of 4, 16 and then
+    // 64 until they are again (a block that pays starts over at 4; the last group
+    // needs no candidates).  A block that fails costs as much as a few pivots, so
+    // small K starts without one.  The state comes back after every group; after
+    // a block that paid, the next one is queued before its state is read.
+    // m = 30,000, K = 16: 0.37 ms, 0.40 where no block pays; 0.30 and 2.65 in
+    // blocks alone, 0.41 pivot by pivot.
+    const double nnz = (double)h->nnz, N = h->n, M = m;
+    int32_t k = 0, steps = kPcFew;
+    bool block = K > 2 * kPcBlk, paid = false, single = false;   // single: the last group went pivot by pivot
+    int64_t launched = 0, read = 0;
+    bool form[2] = {false, false};   // of the groups in flight: block?
+    P->build_bytes = 12.0 * nnz + 8.0 * (N + M);   // the Schur diagonal
+    while (k < K) {
+        const bool blk = block && K - k >= kPcFew;
+        if (launched == read || (launched == read + 1 && paid && form[read & 1] && K - k >= kPcBlk + kPcFew)) {
+            if (blk) {
+                launch_pc_block(B, st);
+            } else {
+                launch_pc_pivots(B, std::min(steps, K - k), steps < K - k || !single, st);
+                steps = std::min(4 * steps, 4 * kPcBlk);
+            }
+            form[launched & 1] = blk;
+            HIPCHK(hipMemcpyAsync(P->hstate + (launched & 1), P->state.p, sizeof(PcState), hipMemcpyDeviceToHost, st));
+            HIPCHK(hipEventRecord(P->ev[launched & 1], st));
+            ++launched;
+            continue;
+        }
+        HIPCHK(hipEventSynchronize(P->ev[read & 1]));
+        const PcState& s = P->hstate[read & 1];
+        const bool was = form[read & 1];
+        // A block reads A once, with kPcBlk vectors (8 (n + m) each), the
+        // finished columns once and the candidates' sums (32 m each), and per
+        // pivot its sums and the block's own columns; pivot by pivot, each reads
+        // A with one vector and the columns before it.  Either way a pivot takes
+        // the Schur diagonal and a column in FP64 and FP32.
+        const double k0 = was ? s.k0 : k, got = s.k - k0, own = 4.0 * got * (got - 1);   // own columns: 8 m got (got - 1) / 2
+        P->build_bytes += was ? 12.0 * nnz + kPcBlk * (8.0 * (N + M) + 32.0 * M) + 8.0 * M * k0 + got * 32.0 * M
+                              : got * (12.0 * nnz + 8.0 * (N + M) + 8.0 * M * k0);
+        P->build_bytes += M * (own + 36.0 * got);
+        k = s.k;
+        block = s.taken >= kPcFew;
+        paid = was && block;
+        single = !was;
+        if (paid) steps = kPcFew;
+        ++read;
     }
     launch_pc_l11(m, K, P->perm.p, P->L.p, P->L11.p, P->X.p, st);
     HIPCHK(hipGetLastError());
 }
 
-// per block of kPcBlk pivots: A once (12 nnz) with kPcBlk vectors (8 (n + m)
-// each), the k finished columns once (8 m k) and the candidates' sums (32 m
-// each); per pivot its sums, the block's own columns (half of them on
-// average), the Schur diagonal and the new column in FP64 and FP32
-double pcg_build_bytes(const help_gpu* h) {
-    const double nnz = (double)h->nnz, m = h->m, n = h->n, K = h->pcg ? h->pcg->K : 0;
-    const double blocks = K / kPcBlk;
-    return blocks * (12.0 * nnz + kPcBlk * (8.0 * (n + m) + 32.0 * m)) + 8.0 * m * K * blocks / 2 +
-           K * m * (32.0 + 8.0 + 4.0 * kPcBlk + 16.0 + 12.0);
-}
+double pcg_build_bytes(const help_gpu* h) { return h->pcg ? h->pcg->build_bytes : 0.0; }
 
 // per iteration: A^T p scaled (12 nnz + 8 m + 16 n), A t (12 nnz + 8 n + 8 m),
 // the preconditioner (two passes over the m x K factor: 8 m K in FP32,

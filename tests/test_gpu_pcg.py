@@ -99,6 +99,91 @@ def test_partial_cholesky_blocks_match_oracle(name, maker, K, dfun):
     assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
 
 
+def _parallel_rows(sizes, tail, seed):
+    """Rows in groups of the given sizes, a group's rows nearly parallel (three
+    columns of entries 1 +- 0.001), each group's diagonals 0.97 times those of the
+    one before, `tail` small rows behind, every row with a small column of its
+    own and weakly coupled to others; and a d under which the groups' columns
+    hardly count and all rows differ."""
+    rng = np.random.default_rng(seed)
+    G, m = len(sizes), sum(sizes) + tail
+    first = np.concatenate(([0], np.cumsum(sizes)))
+    grp = [np.arange(first[g], first[g + 1]) for g in range(G)] * 3
+    far = np.sort(rng.integers(0, m, (2 * m, 4)), axis=1)
+    far = far[(far[:, 1:] != far[:, :-1]).all(axis=1)]
+    counts = np.concatenate(([len(r) for r in grp], np.full(len(far), 4), np.ones(m, int)))
+    rowind = np.concatenate(grp + [far.ravel(), np.arange(m)]).astype(np.int32)
+    val = np.concatenate((1 + 1e-3 * rng.standard_normal(3 * sum(sizes)), 0.01 * rng.standard_normal(far.size), np.ones(m)))
+    n = len(counts)
+    inst = Instance(m, n, np.concatenate(([0], np.cumsum(counts))).astype(np.int64), rowind, val, np.ones(m), np.ones(n))
+    close, apart = np.ones(n), np.ones(n)
+    close[:3 * G] = np.tile(1e-4 / 0.97 ** np.arange(G), 3)
+    close[-m:] = 1e3
+    apart[:3 * G] = 1e6
+    apart[-m:] = np.exp(rng.uniform(-1, 1, m) * np.log(10.0))
+    return inst, close, apart
+
+
+@pytest.mark.parametrize("name,sizes,K", [
+    ("groups of 20", [20] * 60, 50),
+    ("few pivots", [20] * 30, 3),
+    ("at most two blocks of pivots", [20] * 30, 27),
+    ("groups, then single rows, then groups", [20] * 9 + [1] * 90 + [20] * 40, 120),
+    ("single rows, then groups of 5", [1] * 55 + [5] * 60, 99),
+    ("single rows", [1] * 150, 130)])
+def test_partial_cholesky_parallel_rows_match_oracle(name, sizes, K):
+    """Where few of a group's candidates are taken the build goes on pivot by
+    pivot, and back to blocks where many are: the oracle's pivots and factor
+    within the bars of test_partial_cholesky_matches_oracle.  (The groups' leaders
+    stay ahead of what a first pivot leaves of the others, some 1e-6 of it.)"""
+    inst, d, _ = _parallel_rows(sizes, 300, seed=81)
+    _flush(f"pcg factor, {name}: m={inst.m} n={inst.n} K={K}")
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=K)
+    be.construct(inst)
+    be.renew(d)
+    perm, D, S, Lg = be.pcg_factor()
+    be.destruct()
+    operm, oD, oS, oL = _oracle_pchol(inst, d, K)
+    assert np.array_equal(perm, operm)
+    assert np.allclose(D, oD, rtol=1e-11, atol=0)
+    assert np.allclose(S, oS, rtol=1e-9, atol=1e-12 * np.abs(oS).max())
+    assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
+
+
+def test_partial_cholesky_cost_on_parallel_rows():
+    """A block of 16 candidates that takes one of them costs several single
+    pivots.  Rows in groups of 20 near-parallel ones (one candidate per block)
+    against the same instance with all rows apart (every candidate taken), 200
+    pivots of 200,000 rows: 3.2 times as long pivot by pivot, 10 times in
+    blocks; the bar is between the two."""
+    inst, close, apart = _parallel_rows([20] * 10000, 0, seed=82)
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=200)
+    be.construct(inst)
+    ms = {}
+    for name, d in (("apart", apart), ("close", close)):
+        for _ in range(5):
+            be.renew(d)
+            ms[name] = min(ms.get(name, np.inf), be.renew_stats.ms_precond)
+    be.destruct()
+    _flush(f"build of 200 pivots, m={inst.m}: rows apart {ms['apart']:.2f} ms, in groups {ms['close']:.2f} ms")
+    assert ms["close"] <= 5.5 * ms["apart"]
+
+
+def test_partial_cholesky_ends_without_numbers():
+    """Where every Schur diagonal left is NaN the pivots are the rows at the next
+    positions: the build ends with a permutation."""
+    inst = instances.random_lp(300, 600, 4, seed=83)
+    for bad in (1, inst.n):
+        d = np.ones(inst.n)
+        d[:bad] = np.nan
+        be = LinearEquation(mode=L.MODE_PCG, pcg_k=60)
+        be.construct(inst)
+        be.renew(d)
+        perm = be.pcg_factor()[0]
+        be.destruct()
+        assert np.array_equal(np.sort(perm), np.arange(inst.m))
+
+
 def test_pcg_solve_matches_dense():
     inst = instances.random_lp(400, 800, 4, seed=23)
     rng = np.random.default_rng(2)
