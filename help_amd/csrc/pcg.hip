@@ -61,6 +61,7 @@ struct PcgState {
     DBuf<PcBest> top, arg;
     PcState* hstate = nullptr;       // pinned: the state after the last two groups of the build
     double build_bytes = 0;          // algorithmic bytes of the last build
+    bool blocks = false;             // the build may take its pivots in blocks
     DBuf<double> x, r, z, p, q, t;
     std::vector<int32_t> iota;
 };
@@ -87,17 +88,6 @@ void pcg_setup(help_gpu* h) {
     P->D.alloc(K);
     P->w.alloc(K);
     P->S.alloc(m);
-    // the build's block of pivots: the candidates' vectors over the columns, the
-    // columns of A D^-1 A^T and their left-looking sums
-    P->sc.alloc((size_t)n * kPcBlk);
-    P->g.alloc((size_t)m * kPcBlk);
-    P->acc.alloc((size_t)m * kPcBlk * 4);
-    P->wb.alloc((size_t)K * kPcBlk);
-    P->bpart.alloc(std::max<size_t>(1, (size_t)h->rows.nparts * kPcBlk));
-    P->state.alloc(1);
-    P->top.alloc(kTopBlocks * kPcBlk);
-    P->arg.alloc(std::max(kTopBlocks, kColumnBlocks));
-    HIPCHK(hipHostMalloc((void**)&P->hstate, 2 * sizeof(PcState), hipHostMallocDefault));
     P->L11.alloc((size_t)K * K);
     P->X.alloc((size_t)K * K);
     P->y1.alloc(2 * kPcgMaxK);
@@ -112,7 +102,36 @@ void pcg_setup(help_gpu* h) {
     for (auto& e : P->ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     P->iota.resize(m);
     for (int32_t i = 0; i < m; ++i) P->iota[i] = i;
-    HIPCHK(hipMemsetAsync(P->sc.p, 0, sizeof(double) * n * kPcBlk, st));
+    if (P->K > 0) {
+        P->state.alloc(1);
+        P->top.alloc(kTopBlocks * kPcBlk);
+        P->arg.alloc(std::max(kTopBlocks, kColumnBlocks));
+        HIPCHK(hipHostMalloc((void**)&P->hstate, 2 * sizeof(PcState), hipHostMallocDefault));
+        // the build's blocks: the candidates' vectors over the columns, the
+        // columns of A D^-1 A^T and their left-looking sums (8 (16 n + 80 m)
+        // bytes).  Where they do not fit, or no block could pay (the first group
+        // of K < 2 kPcFew leaves fewer than kPcFew pivots), the build goes pivot
+        // by pivot.
+        P->blocks = P->K >= 2 * kPcFew;
+        if (P->blocks) {
+            try {
+                P->sc.alloc((size_t)n * kPcBlk);
+                P->g.alloc((size_t)m * kPcBlk);
+                P->acc.alloc((size_t)m * kPcBlk * 4);
+                P->wb.alloc((size_t)K * kPcBlk);
+                P->bpart.alloc(std::max<size_t>(1, (size_t)h->rows.nparts * kPcBlk));
+            } catch (const HipError&) {
+                (void)hipGetLastError();
+                for (auto* b : {&P->sc, &P->g, &P->acc, &P->wb, &P->bpart}) b->free();
+                P->blocks = false;
+            }
+        }
+        if (!P->blocks) {
+            P->sc.alloc(n);
+            P->g.alloc(m);
+        }
+        HIPCHK(hipMemsetAsync(P->sc.p, 0, sizeof(double) * P->sc.n, st));
+    }
     HIPCHK(hipStreamSynchronize(st));
 }
 
@@ -136,7 +155,7 @@ void pcg_renew(help_gpu* h) {
     B.perm = P->perm.p; B.pos = P->pos.p;
     B.S = P->S.p; B.D = P->D.p; B.L = P->L.p; B.w = P->w.p; B.L32 = h->opts.pcg_fp32_precond ? P->L32.p : nullptr;
     B.sc = P->sc.p; B.part = P->bpart.p; B.g = P->g.p; B.acc = P->acc.p; B.wb = P->wb.p;
-    HIPCHK(hipMemsetAsync(P->state.p, 0, sizeof(PcState), st));
+    if (K > 0) HIPCHK(hipMemsetAsync(P->state.p, 0, sizeof(PcState), st));
     // Groups of pivots: a block as long as the last group's leading candidates
     // were enough for one to pay, else pivot by pivot in groups of 4, 16 and then
     // 64 until they are again (a block that pays starts over at 4; the last group
@@ -146,13 +165,13 @@ void pcg_renew(help_gpu* h) {
     // m = 30,000, K = 16: 0.37 ms, 0.40 where no block pays; 0.30 and 2.65 in
     // blocks alone, 0.41 pivot by pivot.
     const double nnz = (double)h->nnz, N = h->n, M = m;
-    int32_t k = 0, steps = kPcFew;
-    bool block = K > 2 * kPcBlk, paid = false, single = false;   // single: the last group went pivot by pivot
+    int32_t k = 0, steps = P->blocks ? kPcFew : K;
+    bool block = P->blocks && K > 2 * kPcBlk, paid = false, single = false;   // single: the last group went pivot by pivot
     int64_t launched = 0, read = 0;
     bool form[2] = {false, false};   // of the groups in flight: block?
     P->build_bytes = 12.0 * nnz + 8.0 * (N + M);   // the Schur diagonal
     while (k < K) {
-        const bool blk = block && K - k >= kPcFew;
+        const bool blk = block && P->blocks && K - k >= kPcFew;
         if (launched == read || (launched == read + 1 && paid && form[read & 1] && K - k >= kPcBlk + kPcFew)) {
             if (blk) {
                 launch_pc_block(B, st);

@@ -1,6 +1,7 @@
 """GPU parity of the matrix-free PCG mode (HELP PCG.cpp / UsePCG_CPU.cpp):
 the partial-Cholesky preconditioner against the CPU oracle, the solve against
 dense and sparse direct solves, and the HSD driver end to end."""
+import ctypes as C
 import json
 import os
 
@@ -148,6 +149,53 @@ def test_partial_cholesky_parallel_rows_match_oracle(name, sizes, K):
     assert np.allclose(D, oD, rtol=1e-11, atol=0)
     assert np.allclose(S, oS, rtol=1e-9, atol=1e-12 * np.abs(oS).max())
     assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
+
+
+@pytest.mark.parametrize("sizes", [[20] * 30, [1] * 60])
+@pytest.mark.parametrize("K", [7, 8, 9])
+def test_partial_cholesky_first_blocks_match_oracle(K, sizes):
+    """The fewest pivots that a block can follow the first four ones with, and
+    one fewer (no memory for blocks then), within the bars of
+    test_partial_cholesky_matches_oracle."""
+    inst, d, _ = _parallel_rows(sizes, 300, seed=84)
+    be = LinearEquation(mode=L.MODE_PCG, pcg_k=K)
+    be.construct(inst)
+    be.renew(d)
+    perm, D, S, Lg = be.pcg_factor()
+    be.destruct()
+    operm, oD, oS, oL = _oracle_pchol(inst, d, K)
+    assert np.array_equal(perm, operm)
+    assert np.allclose(D, oD, rtol=1e-11, atol=0)
+    assert np.allclose(S, oS, rtol=1e-9, atol=1e-12 * np.abs(oS).max())
+    assert np.allclose(Lg, oL, rtol=1e-9, atol=1e-11)
+
+
+def test_no_block_memory_without_pivots():
+    """A handle with pcg_k = 0 (a diagonal preconditioner, or the network's graph
+    alone) holds nothing of the build: what one with K = 64 holds beside it is
+    at least the build's blocks, 16 n + 80 m doubles, and 63 more factor columns
+    in FP64 and FP32 (64 MiB for the allocator's rounding)."""
+    from test_zz_no_alloc import _hip
+    hip = _hip()
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t)] * 2
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+    inst = instances.random_lp(400000, 800000, 3, seed=85)
+    held = {}
+    for K in (0, 64):
+        be = LinearEquation(mode=L.MODE_PCG, pcg_k=0)
+        be.construct(instances.random_lp(100, 200, 3, seed=86))   # (the runtime's own allocations)
+        be.destruct()
+        before = free()
+        be = LinearEquation(mode=L.MODE_PCG, pcg_k=K)
+        be.construct(inst)
+        held[K] = before - free()
+        be.destruct()
+    _flush(f"m={inst.m} n={inst.n}: {held[0] / 2**20:.0f} MiB with K = 0, {held[64] / 2**20:.0f} MiB with K = 64")
+    assert held[64] - held[0] >= 8 * (16 * inst.n + 80 * inst.m) + 63 * 12 * inst.m - 2**26
 
 
 def test_partial_cholesky_cost_on_parallel_rows():
