@@ -760,7 +760,7 @@ void setup_device_common(help_gpu* h) {
     h->d_err.alloc(1);
     std::vector<help::RowChunk> chunks;
     std::vector<int32_t> hrow, hptr, mrow;
-    help::build_row_split(m, n, h->R.rowptr, h->csrcol, chunks, hrow, hptr, mrow);
+    help::build_row_split(m, h->R.rowptr, h->csrcol, chunks, hrow, hptr, mrow);
     for (int32_t i = 0; i < m; ++i)
         h->max_row_nnz = std::max<int32_t>(h->max_row_nnz, (int32_t)(h->R.rowptr[i + 1] - h->R.rowptr[i]));
     h->d_chunks.upload(chunks, st);

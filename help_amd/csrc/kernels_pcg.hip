@@ -852,7 +852,7 @@ __global__ void k_cg_init(double* __restrict__ s, double rr, double rz) {
 
 }  // namespace
 
-void build_row_split(int32_t m, int32_t n, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
+void build_row_split(int32_t m, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
                      std::vector<RowChunk>& chunks, std::vector<int32_t>& hrow, std::vector<int32_t>& hptr,
                      std::vector<int32_t>& mrow) {
     chunks.clear();

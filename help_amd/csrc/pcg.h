@@ -40,7 +40,7 @@ struct RowSplitDev {
     double* part = nullptr;          // one partial per chunk
 };
 
-void build_row_split(int32_t m, int32_t n, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
+void build_row_split(int32_t m, const std::vector<int64_t>& rowptr, const std::vector<int32_t>& colind,
                      std::vector<RowChunk>& chunks, std::vector<int32_t>& hrow, std::vector<int32_t>& hptr,
                      std::vector<int32_t>& mrow);
 

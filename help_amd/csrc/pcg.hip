@@ -75,16 +75,9 @@ void pcg_setup(help_gpu* h) {
     const int32_t m = h->m, n = h->n;
     P->K = std::max(0, std::min<int32_t>(std::min(h->opts.pcg_k, kPcgMaxK), m));
     const int64_t K = std::max<int32_t>(P->K, 1);
-    // an even number of columns: the apply reads them in pairs, and a zero
-    // column follows an odd K
-    const int64_t K2 = (K + 1) / 2 * 2;
-    P->L.alloc((size_t)m * K2);
-    HIPCHK(hipMemsetAsync(P->L.p + (size_t)m * K, 0, sizeof(double) * (size_t)m * (K2 - K), st));
+    P->L.alloc((size_t)m * K);
     P->ld32 = ((int64_t)m + 31) / 32 * 32;
-    if (h->opts.pcg_fp32_precond) {
-        P->L32.alloc((size_t)P->ld32 * K2);
-        HIPCHK(hipMemsetAsync(P->L32.p + (size_t)P->ld32 * K, 0, sizeof(float) * (size_t)P->ld32 * (K2 - K), st));
-    }
+    if (h->opts.pcg_fp32_precond) P->L32.alloc((size_t)P->ld32 * K);
     P->D.alloc(K);
     P->w.alloc(K);
     P->S.alloc(m);
