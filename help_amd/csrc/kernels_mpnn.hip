@@ -57,8 +57,6 @@ __global__ void k_feat_col(int32_t n, const double* __restrict__ dinv, double nu
     xc[(int64_t)j * kNnFC + 1] = 1.0f;
 }
 
-// mode 0: part[b] = sum of log(x) over x > 0, part[nblk + b] = their count;
-// mode 1: part[b] = sum of x^2
 // Partial sums of the input statistics, blockIdx.y = 0: log g_i and the
 // count of g_i > 0, 1: the same for 1/d, 2: r_i^2 (rows of gridDim.x partials
 // in that order).  Bound by the launches and the copy to the host: one of
@@ -136,8 +134,8 @@ __device__ inline f32x4_t load4(const Bf16* __restrict__ p) {
 __device__ inline f32x4_t load4(const float* __restrict__ p) { return *reinterpret_cast<const f32x4_t*>(p); }
 
 // ------------------------------------------------------------ dense layers
-template <typename AT, typename IT>
-__global__ __launch_bounds__(256) void k_dense(int64_t N, const IT* __restrict__ in1, int k1,
+template <typename AT>
+__global__ __launch_bounds__(256) void k_dense(int64_t N, const AT* __restrict__ in1, int k1,
                                                const AT* __restrict__ in2, int k2, const float* __restrict__ W,
                                                const float* __restrict__ b, AT* __restrict__ out) {
     __shared__ float Ws[2 * kNnH * kNnH];
@@ -691,25 +689,22 @@ void nn_stats_partials(int64_t m, int64_t n, const double* g, const double* dinv
     help::launch_kernel(k_stats, dim3(nblk, 3), kB, 0, st, m, n, g, dinv, r, part);
 }
 
-template <typename AT, typename IT>
-void nn_dense(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const float* W, const float* b, AT* out,
+template <typename AT>
+void nn_dense(int64_t N, const AT* in1, int k1, const AT* in2, int k2, const float* W, const float* b, AT* out,
               hipStream_t st) {
     if (N <= 0) return;
-    if constexpr (std::is_same<AT, Bf16>::value && std::is_same<IT, Bf16>::value) {
+    if constexpr (std::is_same<AT, Bf16>::value) {
         if ((k1 + k2) % 32 == 0 && k1 % 8 == 0 && k1 + k2 <= 2 * kNnH) {
             help::launch_kernel(k_dense_mfma, grid_cap((N + 63) / 64, 2048), kB, 0, st, N, in1, k1, in2, k2, W, b, out);
             return;
         }
     }
-    if constexpr (std::is_same<IT, float>::value) {
-        if (k2 == 0 && (k1 == kNnFR || k1 == kNnFC)) {   // the input layers
-            if (k1 == kNnFR) help::launch_kernel(k_dense_in<AT, kNnFR>, grid_for(8 * N), kB, 0, st, N, in1, W, b, out);
-            else help::launch_kernel(k_dense_in<AT, kNnFC>, grid_for(8 * N), kB, 0, st, N, in1, W, b, out);
-            return;
-        }
-    }
-    if constexpr (std::is_same<AT, IT>::value)
-        help::launch_kernel(k_dense<AT, IT>, grid_cap((N + 3) / 4, 2048), kB, 0, st, N, in1, k1, in2, k2, W, b, out);
+    help::launch_kernel(k_dense<AT>, grid_cap((N + 3) / 4, 2048), kB, 0, st, N, in1, k1, in2, k2, W, b, out);
+}
+
+template <typename AT, int K>
+void nn_dense_in(int64_t N, const float* in, const float* W, const float* b, AT* out, hipStream_t st) {
+    if (N > 0) help::launch_kernel(k_dense_in<AT, K>, grid_for(8 * N), kB, 0, st, N, in, W, b, out);
 }
 
 void nn_mfma_bf16_probe(const float* a, const float* b, float* out, hipStream_t st) {
@@ -768,12 +763,9 @@ void nn_dense_bwd_w(int64_t N, const AT* in1, const AT* in2, const float* dh, co
     else help::launch_kernel(k_dense_bwd_w<AT, 4>, nn_wgrad_blocks(N), kB, 0, st, N, in1, in2, dh, h, partial);
 }
 
-template <typename AT>
-void nn_dense_bwd_w_in(int64_t N, const float* in, int k, const float* dh, const AT* h, float* partial,
-                       hipStream_t st) {
-    if (N <= 0) return;
-    if (k == kNnFR) help::launch_kernel(k_dense_bwd_w_in<AT, kNnFR>, nn_wgrad_blocks(N), kB, 0, st, N, in, dh, h, partial);
-    else help::launch_kernel(k_dense_bwd_w_in<AT, kNnFC>, nn_wgrad_blocks(N), kB, 0, st, N, in, dh, h, partial);
+template <typename AT, int K>
+void nn_dense_bwd_w_in(int64_t N, const float* in, const float* dh, const AT* h, float* partial, hipStream_t st) {
+    if (N > 0) help::launch_kernel(k_dense_bwd_w_in<AT, K>, nn_wgrad_blocks(N), kB, 0, st, N, in, dh, h, partial);
 }
 
 void nn_reduce_blocks(int npar, int nblk, const float* partial, float* out, hipStream_t st) {
@@ -799,7 +791,7 @@ void nn_check_finite(int32_t m, const double* x, int32_t* flag, hipStream_t st) 
 }
 
 #define NN_INST(AT)                                                                                              \
-    template void nn_dense<AT, AT>(int64_t, const AT*, int, const AT*, int, const float*, const float*, AT*,       \
+    template void nn_dense<AT>(int64_t, const AT*, int, const AT*, int, const float*, const float*, AT*,       \
                                    hipStream_t);                                                                 \
     template void nn_mean<AT>(int32_t, const int64_t*, const int32_t*, const double*, const AT*, AT*, hipStream_t); \
     template void nn_output<AT>(int32_t, const AT*, const float*, const float*, const double*, double, float*,     \
@@ -809,11 +801,12 @@ void nn_check_finite(int32_t m, const double* x, int32_t* flag, hipStream_t st) 
     template void nn_dense_bwd_in<AT>(int64_t, const float*, const AT*, const float*, float*, float*, bool,       \
                                       hipStream_t);                                                              \
     template void nn_dense_bwd_w<AT>(int64_t, const AT*, const AT*, const float*, const AT*, float*, hipStream_t); \
-    template void nn_dense_bwd_w_in<AT>(int64_t, const float*, int, const float*, const AT*, float*, hipStream_t);
+    template void nn_dense_in<AT, kNnFR>(int64_t, const float*, const float*, const float*, AT*, hipStream_t);    \
+    template void nn_dense_in<AT, kNnFC>(int64_t, const float*, const float*, const float*, AT*, hipStream_t);    \
+    template void nn_dense_bwd_w_in<AT, kNnFR>(int64_t, const float*, const float*, const AT*, float*, hipStream_t); \
+    template void nn_dense_bwd_w_in<AT, kNnFC>(int64_t, const float*, const float*, const AT*, float*, hipStream_t);
 NN_INST(float)
 NN_INST(Bf16)
-template void nn_dense<Bf16, float>(int64_t, const float*, int, const Bf16*, int, const float*, const float*, Bf16*,
-                                    hipStream_t);
 #undef NN_INST
 
 }  // namespace help

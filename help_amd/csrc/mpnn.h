@@ -52,9 +52,12 @@ void nn_features(int32_t m, int32_t n, const double* g, const double* r, const d
 // 5 nblk partial sums: log g and its count, log 1/d and its count, r^2
 void nn_stats_partials(int64_t m, int64_t n, const double* g, const double* dinv, const double* r, double* part,
                        int nblk, hipStream_t st);
-template <typename AT, typename IT>
-void nn_dense(int64_t N, const IT* in1, int k1, const AT* in2, int k2, const float* W, const float* b, AT* out,
+template <typename AT>
+void nn_dense(int64_t N, const AT* in1, int k1, const AT* in2, int k2, const float* W, const float* b, AT* out,
               hipStream_t st);
+// an input layer of K = kNnFR or kNnFC features
+template <typename AT, int K>
+void nn_dense_in(int64_t N, const float* in, const float* W, const float* b, AT* out, hipStream_t st);
 // one V_MFMA_F32_16X16X32_BF16 from zero: lane l feeds a[8l..8l+7], b[8l..8l+7]; out[4l+r]
 void nn_mfma_bf16_probe(const float* a, const float* b, float* out, hipStream_t st);
 template <typename AT>
@@ -83,10 +86,9 @@ void nn_dense_bwd_in(int64_t N, const float* dh, const AT* h, const float* W, fl
 template <typename AT>
 void nn_dense_bwd_w(int64_t N, const AT* in1, const AT* in2, const float* dh, const AT* h, float* partial,
                     hipStream_t st);
-// the same for an input layer of k = kNnFR or kNnFC features
-template <typename AT>
-void nn_dense_bwd_w_in(int64_t N, const float* in, int k, const float* dh, const AT* h, float* partial,
-                       hipStream_t st);
+// the same for an input layer of K = kNnFR or kNnFC features
+template <typename AT, int K>
+void nn_dense_bwd_w_in(int64_t N, const float* in, const float* dh, const AT* h, float* partial, hipStream_t st);
 void nn_reduce_blocks(int npar, int nblk, const float* partial, float* out, hipStream_t st);
 // din[src] (+)= sum over the transposed adjacency of val * dout[dst] / deg(dst)
 void nn_mean_bwd(int32_t Nsrc, const int64_t* ptrT, const int32_t* idxT, const double* valT,

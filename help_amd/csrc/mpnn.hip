@@ -112,17 +112,17 @@ void forward(help_mpnn* net, help_gpu* h, const double* d, const double* r, doub
     const int64_t *rp = h->d_rowptr.p, *cp = h->d_colptr.p;
     const int32_t *ci = h->d_colind.p, *ri = h->d_rowind.p;
     const double *rv = h->d_csrval.p, *cv = h->d_val.p;
-    help::nn_dense<AT, float>(m, net->xr.p, help::kNnFR, nullptr, 0, W + NnLayout::Wr0, W + NnLayout::br0, a.hr0, st);
-    help::nn_dense<AT, float>(n, net->xc.p, help::kNnFC, nullptr, 0, W + NnLayout::Wc0, W + NnLayout::bc0, a.hc0, st);
+    help::nn_dense_in<AT, help::kNnFR>(m, net->xr.p, W + NnLayout::Wr0, W + NnLayout::br0, a.hr0, st);
+    help::nn_dense_in<AT, help::kNnFC>(n, net->xc.p, W + NnLayout::Wc0, W + NnLayout::bc0, a.hc0, st);
     help::nn_mean<AT>(n, cp, ri, cv, a.hr0, a.ac1, st);                                     // L1
-    help::nn_dense<AT, AT>(n, a.hc0, kNnH, a.ac1, kNnH, W + NnLayout::W(1), W + NnLayout::b(1), a.hc1, st);
+    help::nn_dense<AT>(n, a.hc0, kNnH, a.ac1, kNnH, W + NnLayout::W(1), W + NnLayout::b(1), a.hc1, st);
     help::nn_mean<AT>(m, rp, ci, rv, a.hc1, a.ar2, st);                                     // L2
-    help::nn_dense<AT, AT>(m, a.hr0, kNnH, a.ar2, kNnH, W + NnLayout::W(2), W + NnLayout::b(2), a.hr1, st);
+    help::nn_dense<AT>(m, a.hr0, kNnH, a.ar2, kNnH, W + NnLayout::W(2), W + NnLayout::b(2), a.hr1, st);
     help::nn_mean<AT>(n, cp, ri, cv, a.hr1, a.ac3, st);                                     // L3
-    help::nn_dense<AT, AT>(n, a.hc1, kNnH, a.ac3, kNnH, W + NnLayout::W(3), W + NnLayout::b(3), a.hc2, st);
+    help::nn_dense<AT>(n, a.hc1, kNnH, a.ac3, kNnH, W + NnLayout::W(3), W + NnLayout::b(3), a.hc2, st);
     help::nn_mean<AT>(m, rp, ci, rv, a.hc2, a.ar4, st);                                     // L4
-    help::nn_dense<AT, AT>(m, a.hr1, kNnH, a.ar4, kNnH, W + NnLayout::W(4), W + NnLayout::b(4), a.hr2, st);
-    help::nn_dense<AT, AT>(m, a.hr2, kNnH, nullptr, 0, W + NnLayout::Wh, W + NnLayout::bh, a.z, st);
+    help::nn_dense<AT>(m, a.hr1, kNnH, a.ar4, kNnH, W + NnLayout::W(4), W + NnLayout::b(4), a.hr2, st);
+    help::nn_dense<AT>(m, a.hr2, kNnH, nullptr, 0, W + NnLayout::Wh, W + NnLayout::bh, a.z, st);
     help::nn_output<AT>(m, a.z, W + NnLayout::wo, W + NnLayout::bo, net->g.p, net->rs, net->y.p, x0, st);
     HIPCHK(hipGetLastError());
 }
@@ -136,12 +136,11 @@ void dense_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const AT* in1, const
     help::nn_reduce_blocks(((in2 ? 2 : 1) * kNnH + 1) * kNnH, help::nn_wgrad_blocks(N), net->partial.p,
                            net->grad.p + off, st);
 }
-// the same for an input layer of k features
-template <typename AT>
-void input_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const float* in, int k, const float* dh, const AT* h,
-                 int off) {
-    help::nn_dense_bwd_w_in<AT>(N, in, k, dh, h, net->partial.p, st);
-    help::nn_reduce_blocks((k + 1) * kNnH, help::nn_wgrad_blocks(N), net->partial.p, net->grad.p + off, st);
+// the same for an input layer of K features
+template <typename AT, int K>
+void input_wgrad(help_mpnn* net, hipStream_t st, int64_t N, const float* in, const float* dh, const AT* h, int off) {
+    help::nn_dense_bwd_w_in<AT, K>(N, in, dh, h, net->partial.p, st);
+    help::nn_reduce_blocks((K + 1) * kNnH, help::nn_wgrad_blocks(N), net->partial.p, net->grad.p + off, st);
 }
 
 template <typename AT>
@@ -188,8 +187,8 @@ void backward(help_mpnn* net, help_gpu* h, const double* dy) {
     help::nn_dense_bwd_in<AT>(n, C2, a.hc1, W + NnLayout::W(1), C1, Q, false, st);               // d hc0, d ac1
     help::nn_mean_bwd(m, rp, ci, rv, cp, Q, R1, true, st);                                      // d hr0 +=
     // input layers
-    input_wgrad<AT>(net, st, m, net->xr.p, help::kNnFR, R1, a.hr0, NnLayout::Wr0);
-    input_wgrad<AT>(net, st, n, net->xc.p, help::kNnFC, C1, a.hc0, NnLayout::Wc0);
+    input_wgrad<AT, help::kNnFR>(net, st, m, net->xr.p, R1, a.hr0, NnLayout::Wr0);
+    input_wgrad<AT, help::kNnFC>(net, st, n, net->xc.p, C1, a.hc0, NnLayout::Wc0);
     HIPCHK(hipGetLastError());
     net->have_grad = true;
 }
