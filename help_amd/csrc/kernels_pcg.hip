@@ -157,6 +157,11 @@ __global__ __launch_bounds__(256) void k_csr_heavy(int32_t nheavy, const int32_t
 // Bound by the gathers of x.  19 million nonzeros in columns of 6 and 1, x of
 // 8 MB: 96 us, 119 us when each thread read its own column.
 constexpr int kCscChunk = 1024;
+// place of nonzero p in the chunk that starts at c0, or its nearer end
+__device__ inline int chunk_place(int64_t p, int64_t c0) {
+    const int64_t q = p - c0;
+    return (int)(q < 0 ? 0 : q < kCscChunk ? q : kCscChunk);
+}
 __global__ __launch_bounds__(256) void k_csc_ts(int32_t n, const int64_t* __restrict__ colptr,
                                                 const int32_t* __restrict__ rowind, const double* __restrict__ val,
                                                 const double* __restrict__ dinv, const double* __restrict__ x,
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(256) void k_csc_ts(int32_t n, const int64_t* __rest
                 bx[pos(u * kB + tid)] = g[u];
             }
         __syncthreads();
-        const int lo = (int)((b > c0 ? b : c0) - c0), hi = (int)((e < c0 + kCscChunk ? e : c0 + kCscChunk) - c0);
+        const int lo = chunk_place(b, c0), hi = chunk_place(e, c0);
         for (int q = lo; q < hi; q += 4) {
             double w[4];
 #pragma unroll

@@ -82,3 +82,25 @@ int main() {{
     return 0;
 }}
 """)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_column_chunk_places_far_columns(tmp_path):
+    """k_csc_ts takes a column's part of a chunk of nonzeros between two places in
+    it: both inside the chunk, also for a column that begins or ends more than
+    2^31 nonzeros from it."""
+    text = open(os.path.join(CSRC, "kernels_pcg.hip")).read()
+    assert re.search(r"lo = chunk_place\(b, c0\), hi = chunk_place\(e, c0\);", text)
+    _run(tmp_path, "constexpr int kCscChunk = 1024;\n" + _cut("kernels_pcg.hip", r"^__device__ inline int chunk_place\(") + """
+int main() {
+    const int64_t far[] = {0, 1, 1023, 1024, 1025, 2147483647ll, 2147483648ll, 2147484672ll, 4294967296ll, 4294967297ll,
+                           1ll << 40};
+    for (int64_t c0 : {0ll, 1024ll, 5000000000ll})
+        for (int64_t d : far)
+            for (int64_t p : {c0 + d, c0 - d}) {
+                const int64_t want = p < c0 ? 0 : p > c0 + kCscChunk ? kCscChunk : p - c0;
+                if (chunk_place(p, c0) != want) return 1;
+            }
+    return 0;
+}
+""")
