@@ -395,7 +395,8 @@ __global__ __launch_bounds__(256) void k_out_w(int32_t m, const AT* __restrict__
     for (int64_t i0 = ((int64_t)blockIdx.x * 4 + wave) * 4; i0 < m; i0 += (int64_t)gridDim.x * 16) {
         const int64_t i = i0 + lk < m ? i0 + lk : m - 1;
         const float d = i0 + lk < m ? dyv[i] : 0.0f;
-        const f32x4_t v = load4(z + i * kNnH + 4 * lc);
+        f32x4_t v = load4(z + i * kNnH + 4 * lc);
+        if (i0 + lk >= m) v = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};   // (0 times an infinite z is no zero)
         acc += d * v;
         bs[0] += d;
     }

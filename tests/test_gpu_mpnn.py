@@ -93,6 +93,33 @@ def test_gradients_fp32_node_counts(name, maker):
     be.destruct()
 
 
+def test_output_weight_gradient_of_an_infinite_row():
+    """m no multiple of four, and only the last row's first activation of the
+    head overflows (r is positive there alone, one chain of weights from it to the
+    output): dL/dwo_0 = sum_i dy_i z_i0 has one infinite term, the others are
+    zero, so it is infinite and not NaN; so is the bias's."""
+    inst = instances.random_lp(37, 60, 3, seed=90)
+    rng = np.random.default_rng(8)
+    r = -np.ones(inst.m)
+    r[-1] = 1.0
+    net = Mpnn(bf16=False, seed=3)
+    H, layer = 64, 2 * 64 * 64 + 64
+    p = np.zeros_like(net.params())
+    W1 = 4 * H + H + 2 * H + H
+    p[0] = 1e20                                   # input layer: r / rms(r) to feature 0
+    p[W1 + layer] = p[W1 + 3 * layer] = 1.0       # row layers 2 and 4: feature 0 to itself
+    p[W1 + 4 * layer] = 1e30                      # head
+    wo = W1 + 4 * layer + H * H + H
+    p[wo] = 1.0
+    assert wo + H + 1 == p.size
+    net.set_params(p)
+    be = graph_handle(inst)
+    _, g = net.loss_grad(be, np.exp(rng.uniform(-1, 1, inst.n)), r, rng.standard_normal(inst.m) * 1e-2, want_grad=True)
+    net.close()
+    be.destruct()
+    assert np.isposinf(g[wo]) and np.isposinf(g[wo + H])
+
+
 def test_gradients_bf16_close_to_autograd():
     import mpnn_oracle as MO
     inst, d, r, dy = _case(seed=1)
