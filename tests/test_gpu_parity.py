@@ -214,6 +214,37 @@ def test_solve_tall_fronts(mode, hub):
     assert min(np.linalg.norm(x2 - o2), np.linalg.norm(x2 + o2)) <= 1e-10 * np.linalg.norm(o2)
 
 
+@pytest.mark.parametrize("mode,hub", [(L.MODE_DIRECT_FP32, 4300), (L.MODE_DIRECT_FP64, 6200)])
+def test_solve_tall_fronts_signed(mode, hub):
+    """The fronts of test_solve_tall_fronts, with a b1 and with the signs:
+    x2 = M^-1 (A D^-1 b1 - b2) of a dense solve in FP64 and x1 = D^-1 (b1 - A^T x2),
+    both within 1e-10 as in test_solve_matches_oracle."""
+    rng = np.random.default_rng(hub + 1)
+    leaves = 3
+    m = hub + leaves
+    cols = [np.concatenate(([i], np.arange(leaves, m))) for i in range(leaves)] + [np.array([i]) for i in range(m)]
+    vals = [rng.standard_normal(len(c)) for c in cols[:leaves]] + [np.ones(1)] * m
+    inst = _from_columns(m, cols, vals)
+    d = log_uniform(rng, inst.n, -1, 1)
+    b1, b2 = rng.standard_normal(inst.n), rng.standard_normal(m)
+    be = LinearEquation(mode=mode)
+    be.construct(inst)
+    assert be.supernodes()[1][0] > hub
+    be.renew(d)
+    x1, x2 = be.solve(d, b1, b2)
+    be.destruct()
+    V = np.zeros((m, leaves))
+    for j in range(leaves):
+        V[cols[j], j] = vals[j]
+    M = (V / d[:leaves]) @ V.T
+    M[np.arange(m), np.arange(m)] += 1.0 / d[leaves:] + 1e-5
+    o2 = np.linalg.solve(M, V @ (b1[:leaves] / d[:leaves]) + b1[leaves:] / d[leaves:] - b2)
+    o1 = (b1 - np.concatenate((V.T @ o2, o2))) / d
+    e1, e2 = np.linalg.norm(x1 - o1) / np.linalg.norm(o1), np.linalg.norm(x2 - o2) / np.linalg.norm(o2)
+    _flush(f"tall fronts mode={mode}: x1 {e1:.1e}, x2 {e2:.1e}")
+    assert e2 <= 1e-10 and e1 <= 1e-10
+
+
 @pytest.mark.parametrize("ordering", [L.ORDER_AMD, L.ORDER_ND])
 def test_factor_gathered_fronts(ordering):
     """Fronts whose update-matrix tiles add up their children's entries
