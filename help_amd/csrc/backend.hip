@@ -533,7 +533,7 @@ void build_schedules(help_gpu* h) {
             }
         }
         // one fused launch for the phase's panels when its workgroups (one per
-        // row block, 110 KB of LDS each in FP64) fit the chip at once
+        // row block, 144 KB of LDS each in FP64) fit the chip at once
         const int32_t npa = (int32_t)h->panel.size() - pa;
         const bool fuse = npa <= kFusedPanelMax;
         Op op{OP_POTRF, po, (int32_t)h->potrf.size() - po, wp};

@@ -115,7 +115,7 @@ struct EaRef {
 };
 
 constexpr int kTile = 64;      // GEMM tile and panel width
-// most workgroups of a fused panel launch (FP64: one per CU, 110 KB of LDS)
+// most workgroups of a fused panel launch (FP64: one per CU, 144 KB of its 160 KiB of LDS)
 constexpr int kFusedPanelMax = 240;
 constexpr int kSmallRows = 256;
 constexpr int kSmallElems = 4032;  // panel elements of a small front; with the 64x65

@@ -522,6 +522,9 @@ void k_potrf_mfma(const PanelTask* __restrict__ tasks, T* __restrict__ L,
     __shared__ T XR[2][4 * kTile];         // panel kb's rows of X in XR[kb % 2]
     __shared__ T rps[kTile], pivs[kTile], sdv[kTile], isdv[kTile];
     __shared__ T As[kTrsm ? kTile * kTile : 1];   // the row block, As[k*64 + i]
+    static_assert(sizeof(S) + sizeof(Uf) + sizeof(XF) + sizeof(Mn) + sizeof(XR) + 4 * sizeof(rps) + sizeof(As) <=
+                      160 * 1024,
+                  "a workgroup's LDS");
     const PanelTask tk = tasks[blockIdx.x];
     const int32_t b = tk.b, n = tk.n, c = tk.c;
     const int nb = min(kTile, n - b);
