@@ -119,7 +119,8 @@ typedef struct help_renew_stats {
     double  ms_assemble;     /* ADA^T numeric assembly                          */
     double  ms_factor;       /* numeric factorization                           */
     double  ms_precond;      /* partial-Cholesky build (PCG modes)              */
-    int32_t n_tiny_pivots;   /* pivots replaced in the FP32 factor              */
+    int32_t n_tiny_pivots;   /* non-positive pivots replaced in this renew's factor
+                                (either precision, every column)              */
     int32_t factor_bits;     /* 32 or 64: precision of this renew's factor      */
 } help_renew_stats;
 

@@ -560,6 +560,19 @@ def _first_bad_supernode(be, inst, d):
     return None
 
 
+@pytest.mark.parametrize("path", [0, 1, 2])
+def test_replaced_pivots_are_counted_in_every_column(cfg0, path):
+    """A shift below minus every eigenvalue makes all pivots negative: a replaced
+    pivot leaves the others as they are, so the count is the number of rows, in
+    small fronts and in tiled ones of many columns alike."""
+    be = LinearEquation(front_path=path, beta=-1e6)
+    be.construct(cfg0)
+    be.renew(np.ones(cfg0.n))
+    _flush(f"replaced pivots front_path={path}: {be.renew_stats.n_tiny_pivots} of {cfg0.m}")
+    assert be.renew_stats.n_tiny_pivots == cfg0.m
+    be.destruct()
+
+
 @pytest.mark.parametrize("path,depth", [(0, 0), (1, 0), (2, 0), (1, 4), (1, 8)])
 def test_factor_paths_diagnostic(cfg0, path, depth):
     """Every supernode's columns against the oracle with the automatic front
