@@ -8,10 +8,10 @@
 // * Greedy partial Cholesky (PCG.cpp:38-103): per pivot an argmax over the
 //   Schur diagonal; the candidates' rows of A scattered into n-vectors, their
 //   columns of ADA^T and their left-looking updates against the previous
-//   columns in blocks of kPcBlk (column-major m x K factor, so the
-//   thread-per-row update reads coalesced).
+//   columns, in blocks of kPcBlk or pivot by pivot (column-major m x K factor,
+//   so the thread-per-row update reads coalesced).
 // * Preconditioner apply (PCG.cpp:183-196) with the factor in FP32: the
-//   product and the transposed product in one pass over the m x K factor.
+//   product and the transposed product, a pass over the m x K factor each.
 #include <algorithm>
 #include <climits>
 #include <cmath>
